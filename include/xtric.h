@@ -52,16 +52,18 @@ typedef struct xt_graph xt_graph;
 /* Per-phase device times of the last count on a context, from HIP events on
  * the stream the kernels ran on (milliseconds). */
 typedef struct xt_timing {
-  double orient_ms;   /* degree keys + out-degree count + scans + oriented fill */
-  double count_ms;    /* intersection + reduction kernels (the three phases below) */
+  double orient_ms;   /* degree keys + out-degree count + scans + oriented fill;
+                         in rank space: ranks, rows as ranks, lists */
+  double count_ms;    /* intersection + reduction kernels (the three phases below;
+                         in rank space all of it is group_ms) */
   double total_ms;    /* first to last event of the count */
   double light_ms;    /* one pass over the input rows: light edges intersected,
                          heavy edges listed under their owners */
   double items_ms;    /* tiles of the owners' item lists (counts, scan, descriptors) */
   double group_ms;    /* persistent group kernel: staged list x streamed lists */
   int64_t ne_plus;    /* oriented edges |E+| */
-  int64_t n_heavy;    /* oriented edges intersected by the group kernel */
-  int64_t n_tiles;    /* group tiles drawn from the device work queue */
+  int64_t n_heavy;    /* oriented edges intersected by the group kernel (rank space: all) */
+  int64_t n_tiles;    /* group tiles drawn from the device work queue (rank space: 0) */
   int64_t n_wave_tiles; /* wave tiles (owners with short out-lists, k_count_waves) */
 } xt_timing;
 
@@ -72,7 +74,12 @@ int xt_ctx_create(int device, xt_ctx** out);
 int xt_ctx_destroy(xt_ctx* ctx);
 const char* xt_last_error(const xt_ctx* ctx);
 int xt_last_timing(const xt_ctx* ctx, xt_timing* out);
-/* Tuning knobs (set by xxtric_amd.autotune from measurements; 0 keeps the
+/* Plain totals of one graph in degree orientation are counted in rank space
+ * (vertices ranked by degree, lists of smaller ranks in 16 bits, bit maps in
+ * LDS); the knobs below belong to the edge tiles that all other counts use, and
+ * a context on which one of them is away from its default uses edge tiles for
+ * plain totals too.
+ * Tuning knobs (set by xxtric_amd.autotune from measurements; 0 keeps the
  * current value): light_cut -- edges whose two out-lists are both at most this
  * long are intersected one per thread, the rest by the group kernel or wave
  * tiles (default 32 for one graph; for batches and the server 8 from 2^22

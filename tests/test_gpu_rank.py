@@ -1,0 +1,130 @@
+"""The count in rank space (plain totals in degree orientation, library default
+knobs) at the sizes where it can go wrong: lists around one chunk, one line and
+one wave, ranks on both sides of the 16-bit limit, more cold ids than one hash
+holds, rows across chunks, rows of many empty neighbours, labels in any order.
+Expected values: the oracle, closed forms, and the edge tiles (asked for by
+setting one of their knobs)."""
+import numpy as np
+import pytest
+
+import oracle_py as O
+from helpers import complete, csr_from_edges, random_graph
+
+pytestmark = pytest.mark.gpu
+
+HOT = 65535  # ranks below are kept in 16 bits
+
+
+def _say(*a):
+    print("[case]", *a, flush=True)
+
+
+def _tiles(ctx, g):
+    ctx.tune(small_cut=32)
+    try:
+        return g.count()
+    finally:
+        ctx.tune(small_cut=-1)
+
+
+def _circulant(n, k):
+    """Vertex i joined to i +- 1 .. k: n k (k - 1) / 2 triangles for n > 3 k."""
+    step = np.concatenate([np.arange(-k, 0), np.arange(1, k + 1)])
+    t = np.sort((np.arange(n, dtype=np.int64)[:, None] + step[None, :]) % n, axis=1)
+    return np.arange(n + 1, dtype=np.int64) * (2 * k), t.reshape(-1)
+
+
+def _beside(a, b):
+    return np.concatenate([a[0], a[0][-1] + b[0][1:]]), np.concatenate([a[1], b[1] + len(a[0]) - 1])
+
+
+@pytest.mark.parametrize("n", [3, 9, 10, 17, 33, 34, 65, 66, 130, 1025])
+def test_list_lengths(ctx, n):
+    """K_n: lists of every length up to n - 1, around chunk, line, lane and wave sizes."""
+    _say("complete", n)
+    off = np.arange(n + 1, dtype=np.int64) * (n - 1)
+    cols = np.tile(np.arange(n, dtype=np.int64), n).reshape(n, n)
+    assert ctx.count_csr(off, cols[~np.eye(n, dtype=bool)].reshape(-1)) == n * (n - 1) * (n - 2) // 6
+
+
+@pytest.mark.parametrize("n", [HOT - 1, HOT, HOT + 1, HOT + 2, HOT + 70])
+def test_ranks_around_the_hot_limit(ctx, n):
+    """All degrees equal, so any vertex may take the ranks on either side."""
+    k = 5
+    _say("circulant", n, k)
+    assert ctx.count_csr(*_circulant(n, k)) == n * k * (k - 1) // 2
+
+
+@pytest.mark.parametrize("k,clique", [(34, 64), (110, 200), (600, 1150)])
+def test_cold_lists(ctx, k, clique):
+    """65,600 vertices of degree 2k outrank a clique of smaller degree: its lists are all
+    cold ids -- within the small hash, past it, and more than one filling of the large one."""
+    n = 65600
+    _say("circulant and clique", k, clique)
+    i = np.arange(clique, dtype=np.int64)
+    cols = np.tile(i, clique).reshape(clique, clique)[~np.eye(clique, dtype=bool)].reshape(-1)
+    off, tails = _beside(_circulant(n, k), (np.arange(clique + 1, dtype=np.int64) * (clique - 1), cols))
+    g = ctx.graph(off, tails.astype(np.int32))
+    exp = n * k * (k - 1) // 2 + clique * (clique - 1) * (clique - 2) // 6
+    assert g.count() == exp
+    assert ctx.timing()["ne_plus"] == len(tails) // 2
+    g.close()
+
+
+@pytest.mark.parametrize("make", ["empty_between", "self_loops", "star", "two_hubs", "isolated_tail"])
+def test_row_shapes(ctx, make):
+    _say(make)
+    rng = np.random.default_rng(4)
+    if make == "empty_between":    # every 700th vertex has edges: chunks span thousands of empty rows
+        a = rng.integers(0, 300, (4000, 2)) * 700
+        off, tails = csr_from_edges(300 * 700, [(int(x), int(y)) for x, y in a if x != y])
+    elif make == "self_loops":
+        a = rng.integers(0, 900, (9000, 2))
+        off, tails = csr_from_edges(900, [(int(x), int(y)) for x, y in a] + [(i, i) for i in range(0, 900, 7)])
+    elif make == "star":           # one row across dozens of chunks, closed by a path
+        n = 50001
+        off, tails = csr_from_edges(n, [(0, i) for i in range(1, n)] + [(i, i + 1) for i in range(1, n - 1)])
+    elif make == "two_hubs":       # a row ends and the next begins inside a chunk, both longer than it
+        n = 9000
+        off, tails = csr_from_edges(n, [(0, 1)] + [(h, i) for h in (0, 1) for i in range(2, n)])
+    else:                          # one edge, then rows without any
+        off, tails = csr_from_edges(5000, [(0, 1), (1, 2), (0, 2)])
+    exp = O.count_degree_ordered(off, tails.astype(np.int32))
+    assert ctx.count_csr(off, tails) == exp
+    g = ctx.graph(off, tails)
+    assert g.count() == exp and _tiles(ctx, g) == exp
+    g.close()
+
+
+@pytest.mark.parametrize("scale,permute", [(9, True), (13, False), (17, True), (17, False), (20, True)])
+def test_rmat_equals_the_edge_tiles(ctx, scale, permute):
+    _say("rmat", scale, permute)
+    g = ctx.rmat(scale, 16, 5, permute)
+    a = g.count()
+    assert a == _tiles(ctx, g) == g.count(orient="id")
+    if scale <= 17:
+        assert a == O.count_degree_ordered(*g.download())
+    g.close()
+
+
+def test_device_csr_and_graph_sizes_in_a_row(ctx):
+    """The reference launcher's int64 CSR, and scratch that is kept from larger graphs."""
+    for off, tails in (O.rmat_csr(15, 16, 3, True), complete(40), random_graph(200, 0.2, 9), O.rmat_csr(12, 16, 3, False)):
+        _say("device csr", len(off) - 1)
+        d = [ctx.to_device(np.asarray(x, np.int64)) for x in (off, tails, [11])]
+        ctx.single_gpu_count(len(off) - 1, d[0].ptr, d[1].ptr, d[2].ptr)
+        assert int(d[2].download(np.int64, 1)[0]) == 11 + O.count_degree_ordered(off, np.asarray(tails, np.int32))
+        for b in d:
+            b.close()
+
+
+def test_ids_out_of_range_are_reported(ctx):
+    from xxtric_amd import XtError, capi
+    off, tails = complete(30)
+    tails = tails.astype(np.int32)
+    tails[17] = 30
+    g = ctx.graph(off, tails)
+    with pytest.raises(XtError) as e:
+        g.count()
+    assert e.value.code == capi.XT_ERR_INPUT
+    g.close()

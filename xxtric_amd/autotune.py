@@ -50,7 +50,9 @@ SPACE = {
     "tile_run": (4, 8, 16, 32, 64),
     "group_hash": (1, 2),
 }
-DEFAULTS = {"light_cut": 32, "wave_owner": 256, "group_round": 2, "group_blocks": 4, "items_per_tile": 256,
+# The library's own choice (-1): a plain count in rank space, which takes none of
+# these knobs; any knob away from its default asks for the edge tiles.
+DEFAULTS = {"light_cut": -1, "wave_owner": -1, "group_round": 2, "group_blocks": 4, "items_per_tile": 256,
             "tile_run": 16, "group_hash": 1}
 BATCH_DEFAULTS = dict(DEFAULTS, light_cut=8, wave_owner=64)
 

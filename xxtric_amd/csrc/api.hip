@@ -119,9 +119,11 @@ int ensure(xt_ctx* ctx, DevBuf& b, size_t bytes) {
 // One statically sized device array, resident on every GPU the library runs
 // on until the process ends.  Its host-side name is not a device address:
 // host code uses only the per-device address from hipGetSymbolAddress.
-constexpr size_t kNoAllocScratchBytes = (size_t)64 << 20;  // 64 MiB
+constexpr size_t kNoAllocScratchBytes = (size_t)64 << 20;  // 64 MiB for the graph
+constexpr size_t kNoAllocSumBytes = 16384;                  // and the sharded sums beside it
 constexpr int kMaxDevices = 64;
-static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
+static_assert((kNumCounters - kNumSlots) * sizeof(uint64_t) + 256 <= kNoAllocSumBytes, "room for the sums");
+static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes + kNoAllocSumBytes];
 
 struct NoAllocDevice {
   std::mutex init_mu;   // guards ptr / ready
@@ -154,16 +156,37 @@ static int check_host_offsets(xt_ctx* ctx, int64_t nv, int64_t ne, const int64_t
   return XT_OK;
 }
 
+// Whether a plain total in degree orientation is counted in rank space: at
+// every size (ms per count, rank space against edge tiles: RGG n = 64 0.03 and
+// 0.09, n = 100,000 0.07 and 0.14; G(n, p) of degree 64 on 200,000 0.46 and
+// 1.45; R-MAT s18 0.30 and 0.85, s22 6.4 and 12.3, s26 189 and 357).  The knobs
+// of the edge tiles, when set, ask for those.
+static bool ranks(const xt_ctx* ctx, int64_t nv, int64_t ne) {
+  const bool knobs = ctx->small_cut != 0 || ctx->wave_owner != -1 || ctx->group_blocks != 4 || ctx->group_round != 2 ||
+                     ctx->group_hash != kHashMix || ctx->items_per_tile != 256 || ctx->tile_run != 16 ||
+                     ctx->force_wide;
+  return !knobs && ne > 0 && rank_fits(ctx, nv, ne);
+}
+
 template <typename T>
 int count_device_csr(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* off,
-                     const T* tails, uint32_t flags, hipStream_t st, bool timed, const OwnedRange* range) {
+                     const T* tails, uint32_t flags, hipStream_t st, bool timed, bool may_rank,
+                     const OwnedRange* range) {
   const int mode = (flags & XT_ORIENT_ID) ? kOrientId : kOrientDegree;
-  XT_TRY(ensure(ctx, s.counters, kNumSlots * sizeof(uint64_t)));
-  XT_TRY(fill_u64(ctx, s.counters.as<uint64_t>(), kNumSlots, 0, st));
+  ctx->last_ranked = false;
+  XT_TRY(ensure(ctx, s.counters, kNumCounters * sizeof(uint64_t)));
+  XT_TRY(fill_u64(ctx, s.counters.as<uint64_t>(), kNumCounters, 0, st));
   uint64_t* pv = nullptr;
   if (flags & XT_PER_VERTEX) {
     XT_TRY(ensure(ctx, s.pv, (size_t)(nv > 0 ? nv : 1) * sizeof(uint64_t)));
     pv = s.pv.as<uint64_t>();
+  }
+  if (may_rank && !pv && !range && mode == kOrientDegree && ranks(ctx, nv, ne)) {
+    if (timed) XT_HIP(ctx, hipEventRecord(ctx->ev[kEvStart], st));
+    XT_TRY(rank_count<T>(ctx, s, nv, ne, off, tails, st, timed ? ctx->ev[kEvOriented] : nullptr));
+    if (timed) XT_HIP(ctx, hipEventRecord(ctx->ev[kEvCounted], st));
+    ctx->last_ranked = true;
+    return XT_OK;
   }
   // Grow every scratch buffer before the first event so no allocation (and
   // its implicit synchronisation) falls inside the timed window.
@@ -180,26 +203,29 @@ int count_device_csr(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int6
 }
 
 template int count_device_csr<int32_t>(xt_ctx*, Scratch&, int64_t, int64_t, const int64_t*, const int32_t*,
-                                       uint32_t, hipStream_t, bool, const OwnedRange*);
+                                       uint32_t, hipStream_t, bool, bool, const OwnedRange*);
 template int count_device_csr<int64_t>(xt_ctx*, Scratch&, int64_t, int64_t, const int64_t*, const int64_t*,
-                                       uint32_t, hipStream_t, bool, const OwnedRange*);
+                                       uint32_t, hipStream_t, bool, bool, const OwnedRange*);
 
 // Reads the count, the input-error slots and the timing after a count.
 static int finish_count(xt_ctx* ctx, int64_t nv, uint32_t flags, hipStream_t st, bool timed,
                         uint64_t* total, uint64_t* per_vertex) {
-  uint64_t h[kNumSlots];
+  uint64_t h[kNumCounters];
   XT_HIP(ctx, hipMemcpyAsync(h, ctx->s.counters.p, sizeof(h), hipMemcpyDeviceToHost, st));
   if (per_vertex && (flags & XT_PER_VERTEX) && nv > 0)
     XT_HIP(ctx, hipMemcpyAsync(per_vertex, ctx->s.pv.p, (size_t)nv * sizeof(uint64_t),
                                hipMemcpyDeviceToHost, st));
   XT_HIP(ctx, hipStreamSynchronize(st));
   if (h[kBadIds]) return set_err(ctx, XT_ERR_INPUT, "neighbour id out of range [0, nv)");
-  if (total) *total = h[kTotal];
+  if (total) *total = h[kTotal] + sum_of(h, kSumTotal);
   int64_t nep = 0, nheavy = 0, ntiles = 0, nwave = 0;
+  const bool ranked = ctx->last_ranked;
   const bool worked = nv > 0 && ctx->s.itcnt.p != nullptr && ctx->s.ooff.p != nullptr;
-  if (nv > 0)
+  if (ranked)
+    nep = nheavy = (int64_t)sum_of(h, kSumEdges);
+  else if (nv > 0)
     XT_HIP(ctx, hipMemcpy(&nep, ctx->s.ooff.as<int64_t>() + nv, sizeof(int64_t), hipMemcpyDeviceToHost));
-  const bool split = worked && nep > 0;  // the light/items/group phases ran
+  const bool split = worked && nep > 0 && !ranked;  // the light/items/group phases ran
   if (split) {
     nheavy = (int64_t)h[kHeavyItems];
     XT_HIP(ctx, hipMemcpy(&ntiles, ctx->s.tileoff.as<int64_t>() + nv, sizeof(int64_t), hipMemcpyDeviceToHost));
@@ -222,6 +248,7 @@ static int finish_count(xt_ctx* ctx, int64_t nv, uint32_t flags, hipStream_t st,
     ctx->timing.orient_ms = a;
     ctx->timing.count_ms = b;
     ctx->timing.total_ms = c;
+    if (ranked) ctx->timing.group_ms = b;
     if (split) {
       float l = 0, i = 0, g = 0;
       XT_HIP(ctx, hipEventElapsedTime(&l, ctx->ev[kEvOriented], ctx->ev[kEvLight]));
@@ -289,7 +316,7 @@ int xt_ctx_create(int device, xt_ctx** out) {
         delete ctx;
         return XT_ERR_HIP;
       }
-    if (ensure(ctx, ctx->s.counters, kNumSlots * sizeof(uint64_t)) != XT_OK) {
+    if (ensure(ctx, ctx->s.counters, kNumCounters * sizeof(uint64_t)) != XT_OK) {
       release(ctx->s);
       delete ctx;
       return XT_ERR_NOMEM;
@@ -520,7 +547,7 @@ int xt_count_csr(xt_ctx* ctx, int64_t nv, int64_t ne, const int64_t* offsets, co
     int32_t* d_tails = ctx->s.in_tails.as<int32_t>();
     XT_TRY(upload_csr(ctx, nv, ne, offsets, tails, 8, d_off, d_tails, st));
     if (flags & XT_VALIDATE) XT_TRY(validate<int32_t>(ctx, nv, ne, d_off, d_tails, (flags & XT_CHECK_SYMMETRY) != 0, st));
-    XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, nv, ne, d_off, d_tails, flags, st, true));
+    XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, nv, ne, d_off, d_tails, flags, st, true, true));
     return finish_count(ctx, nv, flags, st, true, total, per_vertex);
   });
 }
@@ -544,7 +571,7 @@ int xt_single_gpu_count(xt_ctx* ctx, int64_t nv, const int64_t* d_indices, const
     // Offsets must be a valid index (and rows sorted) before the chunked
     // kernels search them; the reference launcher assumes the same.
     XT_TRY(validate<int64_t>(ctx, nv, ne, d_indices, d_edge_list, false, st));
-    XT_TRY(count_device_csr<int64_t>(ctx, ctx->s, nv, ne, d_indices, d_edge_list, XT_ORIENT_DEGREE, st, false));
+    XT_TRY(count_device_csr<int64_t>(ctx, ctx->s, nv, ne, d_indices, d_edge_list, XT_ORIENT_DEGREE, st, false, true));
     uint64_t bad = 0;
     XT_HIP(ctx, hipMemcpyAsync(&bad, ctx->s.counters.as<uint64_t>() + kBadIds, sizeof(bad),
                                hipMemcpyDeviceToHost, st));
@@ -589,7 +616,7 @@ int xt_single_gpu_count_noalloc(xt_ctx* ctx, int64_t nv, const int64_t* d_indice
     uint64_t* counters = s.counters.as<uint64_t>();
     auto run = [&]() -> int {
       XT_TRY(validate<int64_t>(ctx, nv, ne, d_indices, d_edge_list, false, st, counters));
-      XT_TRY(count_device_csr<int64_t>(ctx, s, nv, ne, d_indices, d_edge_list, XT_ORIENT_DEGREE, st, false));
+      XT_TRY(count_device_csr<int64_t>(ctx, s, nv, ne, d_indices, d_edge_list, XT_ORIENT_DEGREE, st, false, false));
       uint64_t bad = 0;
       XT_HIP(ctx, hipMemcpyAsync(&bad, counters + kBadIds, sizeof(bad), hipMemcpyDeviceToHost, st));
       XT_HIP(ctx, hipStreamSynchronize(st));
@@ -903,7 +930,7 @@ int xt_graph_count(xt_ctx* ctx, xt_graph* g, uint32_t flags, uint64_t* total, ui
     XT_HIP(ctx, hipSetDevice(ctx->device));
     if (per_vertex && !(flags & XT_PER_VERTEX)) return set_err(ctx, XT_ERR_ARG, "per_vertex needs XT_PER_VERTEX");
     hipStream_t st = ctx->stream;
-    XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, g->nv, g->ne, g->off, g->tails, flags, st, true));
+    XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, g->nv, g->ne, g->off, g->tails, flags, st, true, true));
     return finish_count(ctx, g->nv, flags, st, true, total, per_vertex);
   });
 }
@@ -920,11 +947,11 @@ int xt_graph_count_owned(xt_ctx* ctx, xt_graph* g, int64_t lo, int64_t hi, uint3
     // The owned-range count skips what cannot be owned, so the graph's total
     // takes a count of its own (run first: the timing kept is the owned count's).
     if (total) {
-      XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, g->nv, g->ne, g->off, g->tails, flags, st, true));
+      XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, g->nv, g->ne, g->off, g->tails, flags, st, true, true));
       XT_TRY(finish_count(ctx, g->nv, flags, st, true, total, nullptr));
     }
     const OwnedRange range{lo, hi};
-    XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, g->nv, g->ne, g->off, g->tails, flags, st, true, &range));
+    XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, g->nv, g->ne, g->off, g->tails, flags, st, true, false, &range));
     XT_TRY(finish_count(ctx, g->nv, flags, st, true, nullptr, nullptr));
     uint64_t h[2] = {0, 0};
     XT_HIP(ctx, hipMemcpy(h, ctx->s.counters.as<uint64_t>() + kOwned, sizeof(h), hipMemcpyDeviceToHost));
@@ -962,7 +989,7 @@ int xt_graph_alg_bytes(xt_ctx* ctx, xt_graph* g, uint32_t flags, uint64_t* bytes
     XT_HIP(ctx, hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
     const int mode = (flags & XT_ORIENT_ID) ? kOrientId : kOrientDegree;
-    XT_TRY(ensure(ctx, ctx->s.counters, kNumSlots * sizeof(uint64_t)));
+    XT_TRY(ensure(ctx, ctx->s.counters, kNumCounters * sizeof(uint64_t)));
     XT_TRY(fill_u64(ctx, ctx->s.counters.as<uint64_t>(), kNumSlots, 0, st));
     XT_TRY(orient<int32_t>(ctx, ctx->s, g->nv, g->ne, g->off, g->tails, mode, st));
     XT_TRY(alg_stats(ctx, ctx->s, g->nv, g->ne, st));

@@ -34,6 +34,7 @@
 #include <type_traits>
 
 #include "xt_device.hpp"
+#include "xt_hash.hpp"
 #include "xt_internal.hpp"
 
 namespace xt {
@@ -172,13 +173,6 @@ __device__ __forceinline__ uint32_t light_intersect8(const int32_t* __restrict__
 #pragma unroll
     for (int k = 0; k < 8; k++) h += a[i] == b[k] ? 1u : 0u;
   return h;
-}
-
-// Lane l's value of v, in every lane (l uniform).
-__device__ __forceinline__ int64_t readlane64(int64_t v, int l) {
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, l);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)v >> 32), l);
-  return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
 // Rows of the oriented edges [eb, ee) staged in LDS when they fit.
@@ -669,15 +663,7 @@ __global__ __launch_bounds__(256) void k_tile_desc(int64_t nv, const int64_t* __
   }
 }
 
-// LDS hash of N+(x): buckets of four ids; empty slots hold kEmpty = 2^31 - 1.
-// A bucket that was full when a later key hashed to it has the top bit of its
-// last slot set ("spilled"); that key went to the next bucket (linear probing
-// by bucket).  A lookup reads its home bucket with one 16-byte LDS read and
-// stops at the first bucket that holds the id or has not spilled.  Ids are
-// below 2^31 - 1, so neither an empty nor a marked slot equals an id, and the
-// padding id -1 matches nothing.
-constexpr int32_t kEmpty = 0x7fffffff;
-
+// LDS hash of N+(x) (buckets as in xt_hash.hpp).
 // Byte offset of w's home bucket, times 16.  MIX: the top 11 bits of
 // w * 0x9E3779B1 (mod 2^32), a multiplicative hash -- ids that share their low
 // bits (strided or bit-structured labels, such as an R-MAT graph's without a
@@ -697,15 +683,6 @@ __device__ __forceinline__ uint32_t bucket_addr(int32_t w) {
 __device__ __forceinline__ const int4& bucket_at(const int4* tab, uint32_t addr) {
   return *reinterpret_cast<const int4*>(reinterpret_cast<const char*>(tab) + addr);
 }
-
-// 0 when the bucket holds w (slot values xor w, minimum over the four slots).
-__device__ __forceinline__ uint32_t bucket_miss(const int4 t, int32_t w) {
-  const uint32_t x = (uint32_t)(t.x ^ w), y = (uint32_t)(t.y ^ w), z = (uint32_t)(t.z ^ w);
-  const uint32_t q = (uint32_t)((t.w & 0x7fffffff) ^ w);
-  return min(min(x, y), min(z, q));
-}
-
-__device__ __forceinline__ bool bucket_spilled(const int4 t) { return t.w < 0; }
 
 // Inserts key; sets *spilled when a full bucket had to be passed.
 template <bool MIX>
@@ -1204,44 +1181,7 @@ constexpr int kWaveLogMax = 8;  // per-wave LDS hash: up to 256 buckets of four 
 constexpr int kWaveOwnerMax = 2 << kWaveLogMax;  // owner lists fill at most half the slots
 constexpr int kWaveThreads = 256;  // four independent waves per workgroup
 
-// Home bucket of w among 2^LOGB: a multiplicative hash, so ids sharing their
-// low bits (strided or clustered labels) still spread.
-template <int LOGB>
-__device__ __forceinline__ uint32_t wave_bucket(int32_t w) {
-  return ((uint32_t)w * 0x9E3779B1u) >> (32 - LOGB);
-}
-
-// Inserts key; returns whether a full bucket had to be passed (and was
-// marked spilled, as in tab_insert).
-template <int LOGB>
-__device__ __forceinline__ bool wave_tab_insert(int4* tab, int32_t key) {
-  uint32_t b = wave_bucket<LOGB>(key);
-  bool passed = false;
-  for (;;) {
-    int* s = reinterpret_cast<int*>(tab + b);
-    if (atomicCAS(s, kEmpty, key) == kEmpty) return passed;
-    if (atomicCAS(s + 1, kEmpty, key) == kEmpty) return passed;
-    if (atomicCAS(s + 2, kEmpty, key) == kEmpty) return passed;
-    if (atomicCAS(s + 3, kEmpty, key) == kEmpty) return passed;
-    atomicOr(s + 3, (int)0x80000000);
-    passed = true;
-    b = (b + 1) & ((1u << LOGB) - 1);
-  }
-}
-
-// Continues a lookup past the spilled home bucket b; ends because at most half
-// the slots are used, so some bucket is not full and therefore not spilled.
-template <int LOGB>
-__device__ __forceinline__ bool wave_tab_continue(const int4* tab, uint32_t b, int32_t w) {
-  for (;;) {
-    b = (b + 1) & ((1u << LOGB) - 1);
-    const int4 t = tab[b];
-    if (bucket_miss(t, w) == 0) return true;
-    if (!bucket_spilled(t)) return false;
-  }
-}
-
-// The same, returning the slot index 4*bucket + s of w, or -1.
+// wave_tab_continue returning the slot index 4*bucket + s of w, or -1.
 template <int LOGB>
 __device__ __forceinline__ int wave_tab_continue_slot(const int4* tab, uint32_t b, int32_t w) {
   for (;;) {
@@ -1251,14 +1191,6 @@ __device__ __forceinline__ int wave_tab_continue_slot(const int4* tab, uint32_t 
     if (sl >= 0) return sl;
     if (!bucket_spilled(t)) return -1;
   }
-}
-
-// Orders this wave's LDS accesses before and after it (one wave owns the
-// table; LDS instructions of a wave execute in order).
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Wave tiles are tdesc[*t_begin .. *t_end).  Each wave draws runs of
@@ -1891,7 +1823,7 @@ static void for_each_need(Scratch& s, int64_t nv, int64_t ne, bool per_vertex, F
   f(s.qscan, (size_t)(nchunks + 1) * sizeof(int64_t));
   f(s.ooff, (size_t)(nvv + 1) * sizeof(int64_t));
   f(s.otails, (size_t)(nee + kOtailsPad) * sizeof(int32_t));
-  f(s.counters, kNumSlots * sizeof(uint64_t));
+  f(s.counters, kNumCounters * sizeof(uint64_t));
   f(s.oflags, (size_t)(nchunks * kBlock));
   f(s.crows, (size_t)(2 * nchunks) * sizeof(int64_t));
   f(s.itcnt, (size_t)nvv * sizeof(uint32_t));
@@ -1913,10 +1845,13 @@ int reserve(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, bool per_vertex) {
 
 static size_t round256(size_t n) { return (n + 255) & ~(size_t)255; }
 
+// Of the counters only the slots' 192 bytes: the region holds the sums besides.
 size_t carve_bytes(int64_t nv, int64_t ne) {
   Scratch tmp;
   size_t tot = 0;
-  for_each_need(tmp, nv, ne, false, [&](DevBuf&, size_t bytes) { tot += round256(bytes); });
+  for_each_need(tmp, nv, ne, false, [&](DevBuf& b, size_t bytes) {
+    tot += round256(&b == &tmp.counters ? size_t{192} : bytes);
+  });
   return tot;
 }
 
@@ -1932,7 +1867,8 @@ void carve(Scratch& s, unsigned char* base, int64_t nv, int64_t ne) {
 
 void release(Scratch& s) {
   DevBuf* bufs[] = {&s.deg, &s.dplus, &s.tailcnt, &s.qscan, &s.ooff, &s.otails, &s.counters,
-                    &s.oflags, &s.crows, &s.itcnt, &s.items, &s.tileoff, &s.tiledesc, &s.vrec, &s.pv, &s.scan_tmp, &s.in_off,
+                    &s.oflags, &s.crows, &s.itcnt, &s.items, &s.tileoff, &s.tiledesc, &s.vrec, &s.pv, &s.rhist, &s.rank,
+                    &s.ocount, &s.rpart, &s.rlists, &s.rrec, &s.scan_tmp, &s.in_off,
                     &s.in_tails};
   for (DevBuf* b : bufs) {
     if (b->fixed) continue;
@@ -1988,7 +1924,11 @@ __global__ __launch_bounds__(256) void k_inner(int64_t start, int64_t end, int64
 }
 
 __global__ void k_add_total(const uint64_t* __restrict__ counters, unsigned long long* __restrict__ out) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) atomicAdd(out, (unsigned long long)counters[kTotal]);
+  // one wave: a shard of the sum per lane
+  uint64_t t = counters[kNumSlots + (threadIdx.x & (kShards - 1)) * kNumSums + kSumTotal];
+  if (threadIdx.x == 0) t += counters[kTotal];
+  t = wave_sum_u64(t);
+  if (threadIdx.x == 0 && blockIdx.x == 0) atomicAdd(out, (unsigned long long)t);
 }
 
 int launch_masked(xt_ctx* ctx, int64_t nedges, const int64_t* mask, const int64_t* ind,

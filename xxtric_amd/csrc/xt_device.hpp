@@ -89,6 +89,13 @@ __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
   return v;
 }
 
+// Lane l's value of v, in every lane (l uniform).
+__device__ __forceinline__ int64_t readlane64(int64_t v, int l) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, l);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)v >> 32), l);
+  return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
 // Block-wide sum (blockDim.x threads, multiple of 64); result valid in thread 0.
 template <int kThreads>
 __device__ __forceinline__ uint64_t block_sum_u64(uint64_t v, uint64_t* s_tmp /* kThreads/64 */) {
@@ -114,6 +121,24 @@ __device__ __forceinline__ int64_t wave_incl_scan_i64(int64_t v) {
     if (lane >= off) v += y;
   }
   return v;
+}
+
+// The same of 32-bit values by data-parallel-primitive moves: shifts inside
+// rows of 16 lanes, then the last lane of a row to the next row and of the
+// lower half to the upper (no LDS traffic, unlike the shuffles).
+__device__ __forceinline__ uint32_t wave_incl_scan_u32(uint32_t v) {
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);  // row_shr:1
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);  // row_shr:2
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);  // row_shr:4
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);  // row_shr:8
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  return v;
+}
+
+// Bits of m (uniform) at lanes below this one.
+__device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
 }
 
 // Exclusive block scan of one value per thread; *total receives the block sum.
@@ -153,6 +178,13 @@ __device__ __forceinline__ void load_run(const T* __restrict__ tails, int64_t e0
   }
 #pragma unroll
   for (int j = 0; j < kRun; j++) vals[j] = (e0 + j < ee) ? (int64_t)tails[e0 + j] : 0;
+}
+
+// Adds v to sum k of the shard that this workgroup adds to (shards after
+// `slots` slots, `sums` words apart).
+__device__ __forceinline__ void add_to_shard(uint64_t* counters, int slots, int shards, int sums, int k, uint64_t v) {
+  if (v)
+    atomicAdd((unsigned long long*)&counters[slots + (int)(blockIdx.x & (shards - 1)) * sums + k], (unsigned long long)v);
 }
 
 // SplitMix64 output function (Steele, Lea, Flood, OOPSLA 2014).

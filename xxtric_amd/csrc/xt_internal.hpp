@@ -51,8 +51,27 @@ enum Slot : int {
   kOwned = 12,         // owned-range count: triangles whose minimum vertex is owned
   kLocal = 13,         // ... and whose middle vertex is owned too
   kWaveQueue = 14,     // next wave tile of k_count_waves, one queue per XCD (14..21)
-  kNumSlots = 24
+  kNumSlots = 32
 };
+
+// Sums that many workgroups add to, after the slots: kShards copies, each on a
+// 128-byte line of its own, added up by whoever reads them.  Additions to one
+// address are made one after another, about 18 ns apart whatever the XCD: a
+// million workgroups on one address take 18 ms.
+enum Sum : int {
+  kSumTotal = 0,  // triangles (rank space)
+  kSumEdges,      // oriented edges (rank space)
+  kSumLists,      // 128-byte lines handed out of the shard's region (rank space)
+  kNumSums = 16
+};
+constexpr int kShards = 64;
+constexpr int kNumCounters = kNumSlots + kShards * kNumSums;
+
+inline uint64_t sum_of(const uint64_t* counters, Sum k) {
+  uint64_t t = 0;
+  for (int i = 0; i < kShards; i++) t += counters[kNumSlots + i * kNumSums + k];
+  return t;
+}
 
 // Orientation rules.
 enum Orient : int { kOrientDegree = 0, kOrientId = 1 };
@@ -77,7 +96,7 @@ struct Scratch {
   DevBuf ooff;      // int64[nv+1]         oriented offsets
   DevBuf vrec;      // uint64[nv]          ooff[x] | d+(x) << 32 when |E+| < 2^32 (gathered per entry)
   DevBuf otails;    // int32[ne+4]         oriented out-lists, ascending ids (|E+| <= ne), padded
-  DevBuf counters;  // uint64[16]          total, tile queue, input-error flags, statistics
+  DevBuf counters;  // uint64[kNumCounters] slots (total, tile queue, input-error flags, statistics), then sharded sums
   DevBuf oflags;    // uint8[ne/8]         kept-entry mask per 8 CSR entries (orientation)
   DevBuf crows;     // int64[2*nchunks]    first and last row of each kChunk-entry input chunk
   DevBuf itcnt;     // uint32[nv]          heavy edges owned by each vertex
@@ -85,6 +104,13 @@ struct Scratch {
   DevBuf tileoff;   // int64[2nv+1]        exclusive scan of tiles per owner (group tiles, then wave tiles)
   DevBuf tiledesc;  // 32 B[nv+ne/256+1]  {first item, ooff[x], x, items, d+(x)} of each tile
   DevBuf pv;        // uint64[nv]          per-vertex counts
+  // The count in rank space (rank.hip; it also uses crows, int32 pairs, and itcnt).
+  DevBuf rhist;     // uint32[2*classes]   vertices per degree class, ranks handed out per class
+  DevBuf rank;      // uint32[nv]          rank by descending degree
+  DevBuf ocount;    // uint64[nv]          neighbours of smaller rank | those below 65535 << 32
+  DevBuf rpart;     // uint32[ne]          rows as ranks, smaller ones first
+  DevBuf rlists;    // 16 B chunks         lists of smaller ranks (hot 16-bit, cold 32-bit)
+  DevBuf rrec;      // 16 B[nv]            list record of every rank
   DevBuf scan_tmp;  // int64[..]           block sums of the scans
   DevBuf in_off;    // int64[nv+1]         staged input offsets (xt_count_csr)
   DevBuf in_tails;  // int32[ne]           staged input ids (xt_count_csr)
@@ -111,6 +137,7 @@ struct xt_ctx {
   int tile_run = 16;         // consecutive tiles a group-kernel workgroup draws at once (1..64)
   int wave_owner = -1;       // wave tiles for owner lists up to this long; -1 default, 0 off
   int last_wave_owner = 0;  // wave-owner cut of the last count (tiles [tileoff[nv], tileoff[2nv]) when > 0)
+  bool last_ranked = false;  // the last count ran in rank space
   bool force_wide = false;  // use the 64-bit offset layout of graphs with >= 2^32 entries everywhere
   int fail_allocs = 0;      // failure injection: scratch allocations left to fail
 };
@@ -184,10 +211,21 @@ template <typename T>
 int validate(xt_ctx* ctx, int64_t nv, int64_t ne, const int64_t* off, const T* tails,
              bool symmetry, hipStream_t st, uint64_t* counters = nullptr);
 
+// The plain total of one graph counted in rank space: adds to the sums
+// kSumTotal and kSumEdges.  split_done (nullable) is recorded
+// once the lists stand.  Only for sizes that rank_fits() accepts.
+bool rank_fits(const xt_ctx* ctx, int64_t nv, int64_t ne);
+template <typename T>
+int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* off, const T* tails, hipStream_t st,
+               hipEvent_t split_done);
+
 // Whole single-graph count on the device (orientation + intersection).
+// may_rank: a plain total may be counted in rank space.  The total is the slot
+// kTotal plus the sum kSumTotal.
 template <typename T>
 int count_device_csr(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* off, const T* tails,
-                     uint32_t flags, hipStream_t st, bool timed, const OwnedRange* range = nullptr);
+                     uint32_t flags, hipStream_t st, bool timed, bool may_rank,
+                     const OwnedRange* range = nullptr);
 
 // Device generators.
 int gen_rmat(xt_ctx* ctx, int scale, int edgefactor, const uint32_t thr[3], uint64_t seed,
