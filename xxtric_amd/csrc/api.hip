@@ -207,9 +207,10 @@ template int count_device_csr<int32_t>(xt_ctx*, Scratch&, int64_t, int64_t, cons
 template int count_device_csr<int64_t>(xt_ctx*, Scratch&, int64_t, int64_t, const int64_t*, const int64_t*,
                                        uint32_t, hipStream_t, bool, bool, const OwnedRange*);
 
-// Reads the count, the input-error slots and the timing after a count.
+// Reads the count, the input-error slots and the timing after a count; sums
+// (nullable, kNumCounters words) gets all counters.
 static int finish_count(xt_ctx* ctx, int64_t nv, uint32_t flags, hipStream_t st, bool timed,
-                        uint64_t* total, uint64_t* per_vertex) {
+                        uint64_t* total, uint64_t* per_vertex, uint64_t* sums = nullptr) {
   uint64_t h[kNumCounters];
   XT_HIP(ctx, hipMemcpyAsync(h, ctx->s.counters.p, sizeof(h), hipMemcpyDeviceToHost, st));
   if (per_vertex && (flags & XT_PER_VERTEX) && nv > 0)
@@ -217,7 +218,8 @@ static int finish_count(xt_ctx* ctx, int64_t nv, uint32_t flags, hipStream_t st,
                                hipMemcpyDeviceToHost, st));
   XT_HIP(ctx, hipStreamSynchronize(st));
   if (h[kBadIds]) return set_err(ctx, XT_ERR_INPUT, "neighbour id out of range [0, nv)");
-  if (total) *total = h[kTotal] + sum_of(h, kSumTotal);
+  if (total) *total = sum_of(h, kSumTotal);
+  if (sums) std::memcpy(sums, h, sizeof(h));
   int64_t nep = 0, nheavy = 0, ntiles = 0, nwave = 0;
   const bool ranked = ctx->last_ranked;
   const bool worked = nv > 0 && ctx->s.itcnt.p != nullptr && ctx->s.ooff.p != nullptr;
@@ -227,7 +229,7 @@ static int finish_count(xt_ctx* ctx, int64_t nv, uint32_t flags, hipStream_t st,
     XT_HIP(ctx, hipMemcpy(&nep, ctx->s.ooff.as<int64_t>() + nv, sizeof(int64_t), hipMemcpyDeviceToHost));
   const bool split = worked && nep > 0 && !ranked;  // the light/items/group phases ran
   if (split) {
-    nheavy = (int64_t)h[kHeavyItems];
+    nheavy = (int64_t)sum_of(h, kSumHeavy);
     XT_HIP(ctx, hipMemcpy(&ntiles, ctx->s.tileoff.as<int64_t>() + nv, sizeof(int64_t), hipMemcpyDeviceToHost));
     if (ctx->last_wave_owner > 0) {
       int64_t wend = 0;
@@ -952,11 +954,10 @@ int xt_graph_count_owned(xt_ctx* ctx, xt_graph* g, int64_t lo, int64_t hi, uint3
     }
     const OwnedRange range{lo, hi};
     XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, g->nv, g->ne, g->off, g->tails, flags, st, true, false, &range));
-    XT_TRY(finish_count(ctx, g->nv, flags, st, true, nullptr, nullptr));
-    uint64_t h[2] = {0, 0};
-    XT_HIP(ctx, hipMemcpy(h, ctx->s.counters.as<uint64_t>() + kOwned, sizeof(h), hipMemcpyDeviceToHost));
-    *owned = h[0];
-    if (local) *local = h[1];
+    uint64_t h[kNumCounters];
+    XT_TRY(finish_count(ctx, g->nv, flags, st, true, nullptr, nullptr, h));
+    *owned = sum_of(h, kSumOwned);
+    if (local) *local = sum_of(h, kSumLocal);
     return XT_OK;
   });
 }

@@ -82,7 +82,8 @@ __global__ __launch_bounds__(256) void k_rebase_many(int64_t ng, int64_t total, 
 }
 
 __global__ void k_copy_total(const uint64_t* __restrict__ counters, uint64_t* __restrict__ dst) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *dst = counters[kTotal];
+  const uint64_t t = wave_sum_u64(counters[kNumSlots + (threadIdx.x & (kShards - 1)) * kNumSums + kSumTotal]);
+  if (threadIdx.x == 0 && blockIdx.x == 0) *dst = t;
 }
 
 }  // namespace xt

@@ -26,7 +26,7 @@
 // the scalar unit.  Each oriented edge reads only its shorter list; the longer
 // one is read once per tile.
 // Reductions: per-thread (and per-wave scalar) counters -> wave64 shuffle tree
-// -> LDS -> one 64-bit atomic per workgroup (per tile for the group kernel).
+// -> LDS -> one 64-bit atomic per workgroup, to one of kShards sums (per graph in a batch).
 //
 // Per-vertex credit (XT_PER_VERTEX): the triangle {a, b, w} belongs to
 // min(a, b, w) (xxtric.hpp:165); hits credited to the edge's endpoints are
@@ -564,17 +564,17 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(BATCH &&
       atomicAdd(&gtotal[g0 + threadIdx.x], s_g[threadIdx.x]);
   } else {
     const uint64_t bsum = block_sum_u64<kBlock>(hits_all, s_red);
-    if (threadIdx.x == 0 && bsum) atomicAdd((unsigned long long*)&counters[kTotal], (unsigned long long)bsum);
+    if (threadIdx.x == 0) add_sum(counters, kSumTotal, bsum);
   }
   if constexpr (CM == kCreditRange) {
     __syncthreads();
     const uint64_t bo = block_sum_u64<kBlock>((uint64_t)r_owned, s_red);
-    if (threadIdx.x == 0 && bo) atomicAdd((unsigned long long*)&counters[kOwned], (unsigned long long)bo);
+    if (threadIdx.x == 0) add_sum(counters, kSumOwned, bo);
     __syncthreads();
     const uint64_t bl = block_sum_u64<kBlock>((uint64_t)r_local, s_red);
-    if (threadIdx.x == 0 && bl) atomicAdd((unsigned long long*)&counters[kLocal], (unsigned long long)bl);
+    if (threadIdx.x == 0) add_sum(counters, kSumLocal, bl);
   }
-  if (threadIdx.x == 0 && nown) atomicAdd((unsigned long long*)&counters[kHeavyItems], (unsigned long long)nown);
+  if (!BATCH && threadIdx.x == 0) add_sum(counters, kSumHeavy, (uint64_t)nown);  // a batch reports no items
 }
 
 // Out-degrees saturated at 65535, from the oriented offsets.
@@ -783,6 +783,7 @@ __global__ __launch_bounds__(kGroupThreads) __attribute__((amdgpu_waves_per_eu(W
     }
     return run_next++;
   };
+  uint64_t all_hits = 0, all_owned = 0, all_local = 0;  // thread 0: sums over the tiles
   int64_t table_a0 = -1;  // owner list staged in s_tab (its oriented offset), -1 none
   // Descriptors are copied global -> LDS by wave 0's lanes 0-1 with one 16-byte
   // LDS-DMA load each (no registers held across the tile).
@@ -1142,16 +1143,15 @@ __global__ __launch_bounds__(kGroupThreads) __attribute__((amdgpu_waves_per_eu(W
     if constexpr (CM == kCreditRange) {
       __syncthreads();
       const uint64_t bo = block_sum_u64<kT>((uint64_t)r_owned + (lane == 0 ? (uint64_t)r_owned_w : 0ull), s_red);
-      if (tid == 0 && bo) atomicAdd((unsigned long long*)&counters[kOwned], (unsigned long long)bo);
+      all_owned += bo;  // thread 0 has the sums
       __syncthreads();
       const uint64_t bl = block_sum_u64<kT>((uint64_t)r_local + (lane == 0 ? (uint64_t)r_local_w : 0ull), s_red);
-      if (tid == 0 && bl) atomicAdd((unsigned long long*)&counters[kLocal], (unsigned long long)bl);
+      all_local += bl;
     }
-    if (tid == 0 && bh) {
-      if constexpr (BATCH)
-        atomicAdd(&gtotal[gid[x]], (unsigned long long)bh);
-      else
-        atomicAdd((unsigned long long*)&counters[kTotal], (unsigned long long)bh);
+    if constexpr (BATCH) {
+      if (tid == 0 && bh) atomicAdd(&gtotal[gid[x]], (unsigned long long)bh);
+    } else {
+      all_hits += bh;
     }
     if (wave == 0) {
       __builtin_amdgcn_s_waitcnt(0);  // the next descriptor's LDS-DMA copy has landed
@@ -1162,6 +1162,11 @@ __global__ __launch_bounds__(kGroupThreads) __attribute__((amdgpu_waves_per_eu(W
     __syncthreads();  // next tile published; LDS free for reuse
   }
   flush_slots();  // the last table's counters (the loop ends on a barrier)
+  if (tid == 0) {
+    add_sum(counters, kSumTotal, all_hits);
+    add_sum(counters, kSumOwned, all_owned);
+    add_sum(counters, kSumLocal, all_local);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1559,11 +1564,13 @@ __global__ __launch_bounds__(kWaveThreads) __attribute__((amdgpu_waves_per_eu(WP
     if constexpr (BATCH)
       atomicAdd(&gtotal[g_cur], (unsigned long long)hits);
     else
-      atomicAdd((unsigned long long*)&counters[kTotal], (unsigned long long)hits);
+      add_sum(counters, kSumTotal, hits);
   }
   if constexpr (RANGE) {
-    if (lane == 0 && owned) atomicAdd((unsigned long long*)&counters[kOwned], (unsigned long long)owned);
-    if (lane == 0 && local) atomicAdd((unsigned long long*)&counters[kLocal], (unsigned long long)local);
+    if (lane == 0) {
+      add_sum(counters, kSumOwned, owned);
+      add_sum(counters, kSumLocal, local);
+    }
   }
 }
 
@@ -1923,11 +1930,9 @@ __global__ __launch_bounds__(256) void k_inner(int64_t start, int64_t end, int64
   if (threadIdx.x == 0 && b) atomicAdd(out, (unsigned long long)b);
 }
 
+// One wave: a shard of the sum per lane.
 __global__ void k_add_total(const uint64_t* __restrict__ counters, unsigned long long* __restrict__ out) {
-  // one wave: a shard of the sum per lane
-  uint64_t t = counters[kNumSlots + (threadIdx.x & (kShards - 1)) * kNumSums + kSumTotal];
-  if (threadIdx.x == 0) t += counters[kTotal];
-  t = wave_sum_u64(t);
+  const uint64_t t = wave_sum_u64(counters[kNumSlots + (threadIdx.x & (kShards - 1)) * kNumSums + kSumTotal]);
   if (threadIdx.x == 0 && blockIdx.x == 0) atomicAdd(out, (unsigned long long)t);
 }
 

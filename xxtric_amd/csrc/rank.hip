@@ -1,0 +1,991 @@
+// rank.hip -- the count in rank space (gfx950): plain totals of one graph.
+//
+// Vertices are ranked by descending degree (rank 0 = the largest hub) and
+// every triangle w < v < u (ranks) is counted once, at its edge (u, v), as an
+// id common to N(v) and to the part of N(u) below v, N(x) holding x's
+// neighbours of smaller rank.  Three things follow from ranks that labels do
+// not give:
+//  * only the ids of N(u) below v can close the edge (u, v), a prefix when
+//    N(u) is in rank order: sum of prefixes against the sum of
+//    min(d+(u), d+(v)) that the edge tiles of count.hip stream: 0.62 of it
+//    (R-MAT s20, 1.97e9 -> 1.23e9 ids);
+//  * the ids that occur in lists are small: those below 65535 ("hot") are
+//    stored in 16 bits, and are nearly all that is streamed (s20: 0.9998), so
+//    an id costs two bytes instead of four;
+//  * N(v)'s hot ids are a 65536-bit map, 8 KB of LDS: one 4-byte LDS read and
+//    a bit test per streamed id instead of a 16-byte hash bucket and four
+//    compares, and a table per wave instead of one per workgroup.
+// Ids from 65535 on ("cold") only matter when v is cold too: then u's cold
+// list is streamed through a hash of N(v)'s cold ids.
+//
+// Both passes that gather or stream are bound by the lines that miss L2 (about
+// 52-55 G lines of 128 bytes a second on this GPU, from HBM or from the 256 MB
+// cache).  R-MAT s26: 353 ms with edge tiles, 186-189 here: k_rank_split 42,
+// k_rank_lists 11, k_rank_count 132-135.
+//
+// Five kernels, no scan over the vertices and no item list:
+//  k_rank_prep    degree classes counted, first and last row of every chunk
+//  k_rank_assign  ranks: counting sort of the vertices by degree class
+//  k_rank_split   per row, in place of the labels: ranks, smaller ones first
+//  k_rank_lists   per vertex: the smaller ranks as a list (hot ascending
+//                 16-bit, then cold 32-bit) and a 32-byte record
+//  k_rank_count   per chunk of entries, one wave: v's map, the lists of its
+//                 larger neighbours u streamed through it
+#include <cmath>
+#include <type_traits>
+
+#include "xt_device.hpp"
+#include "xt_hash.hpp"
+#include "xt_internal.hpp"
+
+namespace xt {
+
+constexpr uint32_t kHot = 65535;       // ranks below are hot; 65535 itself pads 16-bit lists
+constexpr uint32_t kNoRank = ~0u;      // a self-loop or an id out of range; pads cold lists
+constexpr int kRankClasses = 896;      // degree classes: exact below 64, then 32 per octave
+constexpr int kRankMarks = 12;         // ids kept per list for finding prefixes
+constexpr int kAssignRun = 8;          // vertices per thread of k_rank_assign
+constexpr int kLaneList = 32;          // lists of up to this many ids are written by one lane, unsorted
+constexpr int kTinyRow = 8;            // rows of up to this many ids and 64 items: a lane per item
+
+__device__ __forceinline__ int degree_class(int64_t d) {
+  if (d < 64) return d < 0 ? 0 : (int)d;
+  const uint32_t x = d > 0x7fffffff ? 0x7fffffffu : (uint32_t)d;
+  const int e = 31 - __clz((int)x);
+  return 64 + (e - 6) * 32 + (int)((x >> (e - 5)) & 31u);
+}
+
+// Record of the vertex of one rank: where its list starts (16-byte units), the
+// 16-byte chunks of its hot part (ascending ids) and of its cold part, and the
+// first id of every segment of ceil(hot / 12) hot chunks: the segments that
+// start below v hold every id below v.  (Eight cuts at the same ranks for every
+// list, in 16 bytes, streamed 1.26 times the ids below v at R-MAT s22.)
+struct alignas(16) RankRec {
+  uint32_t start;
+  uint32_t len;  // hot chunks | cold chunks << 16
+  uint32_t mark[kRankMarks / 2];
+};
+static_assert(sizeof(RankRec) == 32, "two 16-byte loads");
+
+__device__ __forceinline__ uint32_t mark_step(uint32_t hot) { return (hot + kRankMarks - 1) / kRankMarks; }
+
+// 16-byte chunks a list of t chunks is given: it starts on a multiple of its size up
+// to eight chunks (a 128-byte line), so no list crosses more lines than it
+// fills.
+__device__ __forceinline__ uint32_t list_room(uint32_t t) {
+  return t <= 2 ? t : t <= 4 ? 4 : (t + 7) & ~7u;
+}
+
+// ---------------------------------------------------------------------------
+// Degree classes counted (one histogram per workgroup in LDS), per-row
+// counters cleared, and the first and last row of every S-entry chunk
+// (crows[2c], crows[2c + 1]), each written by the row that holds the boundary.
+__global__ __launch_bounds__(256) void k_rank_prep(int64_t nv, int64_t ne, const int64_t* __restrict__ off, int64_t S,
+                                                   int32_t* __restrict__ crows, uint64_t* __restrict__ oc,
+                                                   uint32_t* __restrict__ ic, uint32_t* __restrict__ hist) {
+  __shared__ uint32_t s_h[kRankClasses];
+  for (int k = threadIdx.x; k < kRankClasses; k += 256) s_h[k] = 0;
+  __syncthreads();
+  const int64_t nchunks = (ne + S - 1) / S;
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; u < nv; u += stride) {
+    const int64_t a = off[u], b = off[u + 1];
+    oc[u] = 0;
+    ic[u] = 0;
+    atomicAdd(&s_h[degree_class(b - a)], 1u);
+    if (a < 0 || b > ne || a >= b) continue;
+    for (int64_t c = (a + S - 1) / S; c * S < b; c++) crows[2 * c] = (int32_t)u;
+    for (int64_t c1 = a / S + 1; c1 * S <= b; c1++) crows[2 * c1 - 1] = (int32_t)u;
+    if (b == ne) crows[2 * nchunks - 1] = (int32_t)u;
+  }
+  __syncthreads();
+  for (int k = threadIdx.x; k < kRankClasses; k += 256)
+    if (s_h[k]) atomicAdd(&hist[k], s_h[k]);
+}
+
+// rank[u]: the number of vertices of larger classes, plus u's place among its
+// class (workgroups take places by one atomic per class they hold; any order
+// inside a class is a valid total order).
+__global__ __launch_bounds__(256) void k_rank_assign(int64_t nv, const int64_t* __restrict__ off,
+                                                     const uint32_t* __restrict__ hist, uint32_t* __restrict__ taken,
+                                                     uint32_t* __restrict__ rank) {
+  __shared__ uint32_t s_base[kRankClasses], s_n[kRankClasses];
+  __shared__ int64_t s_scan[256 / kWave];
+  constexpr int kPer = (kRankClasses + 255) / 256;
+  uint32_t h[kPer];
+  int64_t sum = 0;
+#pragma unroll
+  for (int j = 0; j < kPer; j++) {  // descending classes
+    const int k = kRankClasses - 1 - ((int)threadIdx.x * kPer + j);
+    h[j] = k >= 0 ? hist[k] : 0u;
+    sum += h[j];
+  }
+  int64_t total;
+  int64_t at = block_excl_scan_i64<256>(sum, s_scan, &total);
+#pragma unroll
+  for (int j = 0; j < kPer; j++) {
+    const int k = kRankClasses - 1 - ((int)threadIdx.x * kPer + j);
+    if (k >= 0) {
+      s_base[k] = (uint32_t)at;
+      s_n[k] = 0;
+    }
+    at += h[j];
+  }
+  __syncthreads();
+  const int64_t u0 = (int64_t)blockIdx.x * (256 * kAssignRun) + threadIdx.x;
+  int cls[kAssignRun];
+  uint32_t loc[kAssignRun];
+#pragma unroll
+  for (int j = 0; j < kAssignRun; j++) {
+    const int64_t u = u0 + 256 * j;
+    cls[j] = -1;
+    if (u < nv) {
+      cls[j] = degree_class(off[u + 1] - off[u]);
+      loc[j] = atomicAdd(&s_n[cls[j]], 1u);
+    }
+  }
+  __syncthreads();
+  for (int k = threadIdx.x; k < kRankClasses; k += 256)
+    if (s_n[k]) s_base[k] += atomicAdd(&taken[k], s_n[k]);
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kAssignRun; j++)
+    if (cls[j] >= 0) rank[u0 + 256 * j] = s_base[cls[j]] + loc[j];
+}
+
+// ---------------------------------------------------------------------------
+// Row u's entries as ranks, the smaller ones (N(u)) at the front of the row's
+// own range of `part` and the larger ones at its back; oc[u] = |N(u)| | hot
+// ones << 32.  One workgroup per 2048 entries, eight per thread.  Every row
+// that starts in the chunk marks its first entry with its end and its rank, so
+// a thread meets its rows in LDS whatever empty rows lie between them.  A row
+// inside the chunk is placed by a block scan, through LDS; the chunk's first
+// and last row, which may continue in another chunk, take their places by
+// atomics.  Entries that are no edge (self-loops, ids out of range) go to the
+// back as kNoRank.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_rank_split(int64_t nv, int64_t ne, const int64_t* __restrict__ off,
+                                                       const T* __restrict__ tails, const uint32_t* __restrict__ rank,
+                                                       const int32_t* __restrict__ crows, int per,
+                                                       uint32_t* __restrict__ part, uint64_t* __restrict__ oc,
+                                                       uint32_t* __restrict__ ic, uint64_t* __restrict__ counters) {
+  __shared__ alignas(16) int16_t s_end[kChunk];       // first entry of a row: where the row ends (clamped); 0 elsewhere
+  __shared__ uint32_t s_rk[kChunk];       // and its rank; later the chunk's entries in their new order
+  __shared__ uint32_t s_pre[kChunk + 1];  // smaller ranks before each entry | hot ones << 16
+  __shared__ int64_t s_scan[kBlock / kWave];
+  __shared__ int s_last[kBlock / kWave];
+  __shared__ uint32_t s_ob[2], s_ib[2];   // places taken by the first and the last row
+  __shared__ int s_rng[3];                // the inner rows' range; whether the first row starts before the chunk
+  uint32_t* s_part = s_rk;
+  const int64_t nchunks = (ne + kChunk - 1) / kChunk;
+  const int64_t c = xcd_block(nchunks);
+  if (c >= nchunks) return;  // whole workgroup
+  const int64_t eb = c * kChunk;
+  const int n = (int)min((int64_t)kChunk, ne - eb);
+  const int64_t nsub = 2 * ((ne + (int64_t)kChunk / per - 1) / ((int64_t)kChunk / per));
+  int64_t ulo = crows[2 * c * per], uhi = crows[min(2 * (c * per + per) - 1, nsub - 1)];
+  ulo = ulo < 0 ? 0 : (ulo > nv - 1 ? nv - 1 : ulo);
+  uhi = uhi < ulo ? ulo : (uhi > nv - 1 ? nv - 1 : uhi);
+  const int64_t span = uhi - ulo + 1;
+  auto rel = [&](int64_t o) -> int {  // an offset relative to the chunk, clamped to [-1, kChunk + 1]
+    const int64_t d = o - eb;
+    return (int)(d < -1 ? -1 : (d > kChunk + 1 ? kChunk + 1 : d));
+  };
+  const int tid = (int)threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
+  const int i0 = tid * kPerThread;
+  const bool live = i0 < n;
+  *reinterpret_cast<int4*>(&s_end[i0]) = make_int4(0, 0, 0, 0);
+  uint32_t rv[kPerThread];
+  uint32_t bad = 0;
+  if (live) {
+    int64_t vals[kPerThread];
+    load_run<T>(tails, eb + i0, eb + n, vals);
+#pragma unroll
+    for (int j = 0; j < kPerThread; j++) {  // eight gathers in flight
+      const bool in = i0 + j < n, ok = in && vals[j] >= 0 && vals[j] < nv;
+      if (in && !ok) bad++;
+      const uint32_t r = rank[ok ? vals[j] : 0];
+      rv[j] = ok ? r : kNoRank;
+    }
+  }
+  if (bad) atomicAdd((unsigned long long*)&counters[kBadIds], (unsigned long long)bad);
+  __syncthreads();
+  for (int64_t k = tid; k < span; k += kBlock) {
+    const int64_t o0 = off[ulo + k], o1 = off[ulo + k + 1];
+    const int ro = rel(o0), re = rel(o1);
+    if (re > 0 && ro < n && o1 > o0) {
+      s_end[max(ro, 0)] = (int16_t)re;
+      s_rk[max(ro, 0)] = rank[ulo + k];
+    }
+    if (k == 0) {
+      s_rng[0] = ro < 0 || re > n ? min(re, n) : 0;
+      s_rng[2] = ro < 0;
+    }
+    if (k == span - 1) s_rng[1] = re > n || ro < 0 ? max(ro, 0) : n;
+  }
+  __syncthreads();
+  // The row of this thread's first entry: the last mark up to it.
+  int ends[kPerThread];
+  int last = -1;
+  {
+    const int4 q = *reinterpret_cast<const int4*>(&s_end[i0]);
+    const int w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      ends[2 * j] = (int16_t)(w[j] & 0xffff);
+      ends[2 * j + 1] = w[j] >> 16;
+    }
+#pragma unroll
+    for (int j = 0; j < kPerThread; j++)
+      if (ends[j]) last = i0 + j;
+  }
+  int upto = last;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const int y = __shfl_up(upto, o, kWave);
+    if (lane >= o) upto = max(upto, y);
+  }
+  if (lane == kWave - 1) s_last[wv] = upto;
+  int at = __shfl_up(upto, 1, kWave);
+  if (lane == 0) at = -1;
+  __syncthreads();
+  for (int w = 0; w < wv; w++) at = max(at, s_last[w]);
+  if (ends[0]) at = i0;
+  at = max(at, 0);  // entry 0 is marked whenever the offsets are an index
+  uint32_t small = 0, hot = 0;
+  if (live) {
+    uint32_t ru = s_rk[at];
+#pragma unroll
+    for (int j = 0; j < kPerThread; j++) {
+      if (i0 + j < n) {
+        if (ends[j]) ru = s_rk[i0 + j];
+        if (rv[j] < ru) {
+          small |= 1u << j;
+          if (rv[j] < kHot) hot |= 1u << j;
+        } else if (rv[j] == ru) {
+          rv[j] = kNoRank;  // self-loop
+        }
+      }
+    }
+  }
+  int64_t total;
+  const int64_t pre =
+      block_excl_scan_i64<kBlock>((int64_t)(__popc(small) | (__popc(hot) << 16)), s_scan, &total);  // < 2^28: fields do not meet
+  if (live) {
+#pragma unroll
+    for (int j = 0; j < kPerThread; j++)
+      if (i0 + j < n) {
+        const uint32_t m = (1u << j) - 1u;
+        s_pre[i0 + j] = (uint32_t)pre + (uint32_t)(__popc(small & m) | (__popc(hot & m) << 16));
+      }
+  }
+  if (tid == 0) s_pre[n] = (uint32_t)total;
+  __syncthreads();  // s_rk is read: its place takes the new order
+  for (int64_t k = tid; k < span; k += kBlock) {
+    const int64_t o0 = off[ulo + k], o1 = off[ulo + k + 1];
+    const int ro = rel(o0), re = rel(o1);
+    if (re <= 0 || ro >= n || o1 <= o0) continue;
+    const int a = max(ro, 0), b = min(re, n);
+    const uint32_t q = s_pre[b] - s_pre[a];
+    const uint32_t outs = q & 0xffffu;
+    if (ro >= 0 && re <= n) {
+      oc[ulo + k] = (uint64_t)outs | ((uint64_t)(q >> 16) << 32);
+    } else {
+      const int s = k == 0 ? 0 : 1;
+      const uint32_t ins = (uint32_t)(b - a) - outs;
+      s_ob[s] = outs ? (uint32_t)atomicAdd((unsigned long long*)&oc[ulo + k],
+                                           (unsigned long long)outs | ((unsigned long long)(q >> 16) << 32))
+                     : 0u;
+      s_ib[s] = ins ? atomicAdd(&ic[ulo + k], ins) : 0u;
+    }
+  }
+  __syncthreads();
+  if (live) {
+    int cur = at, nxt = s_end[at];
+#pragma unroll
+    for (int j = 0; j < kPerThread; j++) {
+      const int i = i0 + j;
+      if (i < n) {
+        if (ends[j]) {
+          cur = i;
+          nxt = ends[j];
+        }
+        const bool first = cur == 0 && s_rng[2];  // continues from an earlier chunk
+        const uint32_t before = (s_pre[i] - s_pre[cur]) & 0xffffu;
+        const bool out = (small >> j) & 1u;
+        if (!first && nxt <= n) {
+          s_part[out ? cur + (int)before : nxt - 1 - (i - cur - (int)before)] = rv[j];
+        } else {
+          const int s = first || uhi == ulo ? 0 : 1;
+          const int64_t u = s == 0 ? ulo : uhi;
+          part[out ? off[u] + (int64_t)s_ob[s] + before
+                   : off[u + 1] - 1 - (int64_t)s_ib[s] - (int64_t)(i - cur - (int)before)] = rv[j];
+        }
+      }
+    }
+  }
+  __syncthreads();
+  for (int i = s_rng[0] + tid; i < s_rng[1]; i += kBlock) part[eb + i] = s_part[i];  // the inner rows
+}
+
+// ---------------------------------------------------------------------------
+// Lists and records, by independent waves.  A wave takes `rows` vertices at a
+// time, one per lane, few neighbouring ones from all over the graph (labels that
+// bring vertices of large degree together do not load one wave).  Their lists lie
+// together, those of whole lines first, then of four, two and one chunk,
+// placed by one scan over the four counts, in room that the wave draws
+// `grant` lines at a time from one of kListShards regions (one atomic per 128
+// vertices on one address made 9 of 19 ms at R-MAT s26).  Lists of up to
+// kLaneList ids are written by their lane, unsorted: they fill a line at most.
+// Longer ones are written by the whole wave, one after another: up to 64 ids
+// are ranked by counting the smaller ones, more are sorted by a bit map of
+// their hot ids in LDS with running counts (an id's place is the count before
+// its word plus the bits below it).  Cold ids keep the row's order.
+constexpr int kListShards = 16;
+
+struct ListRoom {
+  uint64_t region, grant;  // lines of a shard's region; lines drawn at once
+  int rows;                // vertices of a wave: 16, 32 or 64
+  int together;            // log2 of the neighbouring vertices it takes at a time
+  int64_t nbatch;
+};
+
+__global__ __launch_bounds__(64) void k_rank_lists(int64_t nv, const int64_t* __restrict__ off,
+                                                   const uint64_t* __restrict__ oc, const uint32_t* __restrict__ rank,
+                                                   const uint32_t* __restrict__ part, ListRoom lr,
+                                                   uint4* __restrict__ lists, RankRec* __restrict__ rec,
+                                                   uint64_t* __restrict__ counters) {
+  constexpr int kGroups = 8;  // pairs of 64-bit words per lane
+  __shared__ ulonglong2 s_bits[kGroups * kWave];
+  __shared__ uint16_t s_pre[kGroups * kWave];
+  __shared__ uint16_t s_mark[kRankMarks];
+  const int lane = threadIdx.x;
+  unsigned long long* bits = reinterpret_cast<unsigned long long*>(s_bits);
+#pragma unroll
+  for (int i = 0; i < kGroups; i++) s_bits[i * kWave + lane] = make_ulonglong2(0, 0);
+  uint64_t room_at = 0, room_end = 0;  // lines drawn, not yet used (lane 0)
+  int shard = (int)(blockIdx.x & (kListShards - 1));
+  auto draw = [&](uint64_t lines) -> uint64_t {
+    if (lines <= room_end - room_at) {
+      room_at += lines;
+      return room_at - lines;
+    }
+    const uint64_t ask = lines * 4 > lr.grant ? lines : lr.grant;  // leaves less than a quarter of a grant
+    for (int k = 0; k < kListShards; k++) {  // a full region: the next one
+      const uint64_t b = atomicAdd((unsigned long long*)&counters[kNumSlots + shard * kNumSums + kSumLists],
+                                   (unsigned long long)ask);
+      if (b + ask <= lr.region) {
+        const uint64_t at = (uint64_t)shard * lr.region + b;
+        if (ask > lines) {
+          room_at = at + lines;
+          room_end = at + ask;
+        }
+        return at;
+      }
+      shard = (shard + 1) & (kListShards - 1);
+    }
+    return kNoRank;  // only for input that is no simple graph
+  };
+  uint64_t edges = 0;
+  for (int64_t batch = blockIdx.x; batch < lr.nbatch; batch += gridDim.x) {  // uniform
+    // Group g of the wave's is group (g * a prime) mod the number of groups.
+    const uint64_t groups = ((uint64_t)nv + (1u << lr.together) - 1) >> lr.together;
+    const uint64_t g = (uint64_t)batch * (uint64_t)(lr.rows >> lr.together) + (uint64_t)(lane >> lr.together);
+    const int64_t u = g < groups && lane < lr.rows ? (int64_t)((g * 2654435761ull % groups) << lr.together) | (lane & ((1 << lr.together) - 1)) : nv;
+    const bool live = u < nv;
+    uint32_t d = 0, h = 0, hc = 0, cc = 0, a0 = 0, ru = 0;
+    if (live) {
+      const uint64_t q = oc[u];
+      d = (uint32_t)q;
+      h = (uint32_t)(q >> 32);
+      a0 = (uint32_t)off[u];
+      ru = rank[u];
+      if (d >= 2) {  // a list of one id has no pair
+        hc = min((h + 7) >> 3, 8192u);  // (the clamps hold for any input that is a simple graph)
+        cc = min((d - h + 3) >> 2, 65535u);
+      }
+    }
+    edges += d;
+    const uint32_t room = list_room(hc + cc);
+    // lines: bits 0-31; lists of four, two, one chunk: 10 bits each from 32 on
+    const int64_t mine = room >= 8 ? (int64_t)(room >> 3) : room == 4 ? 1ll << 32 : room == 2 ? 1ll << 42 : room == 1 ? 1ll << 52 : 0ll;
+    const int64_t inc = wave_incl_scan_i64(mine), at = inc - mine, total = readlane64(inc, kWave - 1);
+    auto field = [](int64_t v, int sh) -> uint32_t { return (uint32_t)(v >> sh) & 1023u; };
+    const uint32_t n8 = (uint32_t)total, n4 = field(total, 32), n2 = field(total, 42), n1 = field(total, 52);
+    const uint32_t chunks = 8 * n8 + 4 * n4 + 2 * n2 + n1;
+    uint32_t base = 0;
+    if (chunks) {  // uniform
+      if (lane == 0) base = (uint32_t)draw((chunks + 7) >> 3);
+      base = __builtin_amdgcn_readfirstlane(base);
+    }
+    uint32_t start = 0;
+    if (room) {
+      if (base == kNoRank) {
+        d = hc = cc = 0;
+      } else {
+        const uint32_t b4 = 8 * n8, b2 = b4 + 4 * n4, b1 = b2 + 2 * n2;
+        start = 8 * base + (room >= 8   ? 8 * (uint32_t)at
+                            : room == 4 ? b4 + 4 * field(at, 32)
+                            : room == 2 ? b2 + 2 * field(at, 42)
+                                        : b1 + field(at, 52));
+      }
+    }
+    const bool alone = live && d <= kLaneList;
+    if (alone && d < 2) {
+      uint4* to = reinterpret_cast<uint4*>(rec + ru);
+      to[0] = to[1] = make_uint4(0, 0, 0, 0);
+    }
+    if (__builtin_amdgcn_ballot_w64(alone && d >= 2)) {  // uniform
+      uint64_t lo = ~0ull, hi = ~0ull;
+      uint32_t least = kHot, nh = 0, nc = 0;
+      uint4* hot = lists + start;
+      uint32_t* cold = reinterpret_cast<uint32_t*>(lists + start + hc);
+      const uint32_t n = alone && d >= 2 ? d : 0;
+      for (uint32_t i0 = 0; __builtin_amdgcn_ballot_w64(i0 < n); i0 += 8) {
+        uint32_t w[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) w[i] = i0 + i < n ? part[a0 + i0 + i] : kNoRank;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+          if (w[i] < kHot) {
+            hi = (hi << 16) | (lo >> 48);
+            lo = (lo << 16) | w[i];
+            least = min(least, w[i]);
+            if ((++nh & 7) == 0) {
+              hot[(nh >> 3) - 1] = make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+              lo = hi = ~0ull;
+            }
+          } else if (i0 + i < n) {
+            cold[nc++] = w[i];
+          }
+        }
+      }
+      if (n) {
+        if (nh & 7) hot[nh >> 3] = make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+        for (; nc & 3; nc++) cold[nc] = kNoRank;
+        static_assert(kLaneList <= 32, "four marks");
+        const uint32_t m = least | (least << 16);  // not sorted: all of it or nothing is below v
+        uint4* to = reinterpret_cast<uint4*>(rec + ru);
+        to[0] = make_uint4(start, hc | (cc << 16), m, m);
+        to[1] = make_uint4(~0u, ~0u, ~0u, ~0u);
+      }
+    }
+    uint64_t todo = __builtin_amdgcn_ballot_w64(live && d > kLaneList);
+    uint32_t ra = 0, rd = 0, rs = 0, rr = 0, rw = kNoRank;  // the next row: first entry, ids, list, rank; its first ids
+    auto pop = [&]() {
+      const int src = __builtin_ctzll(todo);
+      todo &= todo - 1;
+      ra = __builtin_amdgcn_readlane(a0, src);
+      rd = __builtin_amdgcn_readlane(d, src);
+      rs = __builtin_amdgcn_readlane(start, src);
+      rr = __builtin_amdgcn_readlane(ru, src);
+      rw = part[ra + lane];  // more than 32 ids and, in a simple graph, as many behind; the array is padded
+    };
+    bool more = todo != 0;
+    if (more) pop();
+    while (more) {  // uniform
+      const uint32_t dd = rd, st = rs, rk = rr, w0 = (uint32_t)lane < rd ? rw : kNoRank;
+      const uint32_t* ids = part + ra;
+      more = todo != 0;
+      if (more) pop();  // the next row's ids fly while this one is written
+      auto id = [&](uint32_t i) -> uint32_t { return i == 0 ? w0 : i + lane < dd ? ids[i + lane] : kNoRank; };
+      if (lane < kRankMarks) s_mark[lane] = 0xffff;
+      uint32_t hh = 0, place = 0;
+      if (dd <= kWave) {
+        const uint64_t hm = __builtin_amdgcn_ballot_w64(w0 < kHot);
+        hh = (uint32_t)__popcll(hm);
+        for (uint64_t m = hm; m; m &= m - 1)
+          place += (uint32_t)__builtin_amdgcn_readlane((int)w0, __builtin_ctzll(m)) < w0 ? 1u : 0u;
+      } else {
+        uint32_t top = 0;  // groups in use
+        for (uint32_t i = 0; i < dd; i += kWave) {
+          const uint32_t w = id(i);
+          if (w < kHot) {
+            atomicOr(&bits[w >> 6], 1ull << (w & 63));
+            top = max(top, (w >> 13) + 1);
+          }
+        }
+        wave_lds_fence();
+#pragma unroll 1
+        for (uint32_t k = 0; k < (uint32_t)kGroups; k++) {
+          if (__builtin_amdgcn_ballot_w64(top > k) == 0) break;
+          const ulonglong2 t = s_bits[k * kWave + lane];
+          const uint32_t n = (uint32_t)(__popcll(t.x) + __popcll(t.y));
+          const uint32_t upto = wave_incl_scan_u32(n);
+          s_pre[k * kWave + lane] = (uint16_t)(hh + upto - n);
+          hh += __builtin_amdgcn_readlane(upto, kWave - 1);
+        }
+      }
+      wave_lds_fence();
+      const uint32_t hcc = min((hh + 7) >> 3, 8192u), ccc = min((dd - hh + 3) >> 2, 65535u);
+      const uint32_t seg = 8 * max(mark_step(hcc), 1u);               // ids per segment
+      const uint32_t inv = (uint32_t)(((1ull << 32) + seg - 1) / seg);  // r / seg for r < 2^16
+      uint16_t* hl = reinterpret_cast<uint16_t*>(lists + st);
+      uint32_t* cl = reinterpret_cast<uint32_t*>(lists + st + hcc);
+      uint32_t ncold = 0;
+      for (uint32_t i = 0; i < dd; i += kWave) {
+        const uint32_t w = id(i);
+        const bool cold = i + lane < dd && w >= kHot;
+        const uint64_t cm = __builtin_amdgcn_ballot_w64(cold);
+        if (w < kHot) {
+          uint32_t r = place;
+          if (dd > kWave) {
+            const ulonglong2 t = s_bits[w >> 7];
+            const uint64_t below = (1ull << (w & 63)) - 1ull;
+            r = s_pre[w >> 7] + (uint32_t)((w & 64) ? __popcll(t.x) + __popcll(t.y & below) : __popcll(t.x & below));
+          }
+          if (r < 8 * hcc) hl[r] = (uint16_t)w;
+          const uint32_t k = __umulhi(r, inv);
+          if (k * seg == r && k < kRankMarks) s_mark[k] = (uint16_t)w;
+        } else if (cold) {
+          const uint32_t r = ncold + lanes_below(cm);
+          if (r < 4 * ccc) cl[r] = w;
+        }
+        ncold += (uint32_t)__popcll(cm);
+      }
+      wave_lds_fence();
+      if (dd > kWave)
+        for (uint32_t i = 0; i < dd; i += kWave) {
+          const uint32_t w = id(i);
+          if (w < kHot) bits[w >> 6] = 0ull;
+        }
+      if ((uint32_t)lane < 8 * hcc - min(hh, 8 * hcc)) hl[hh + lane] = 0xffff;
+      if ((uint32_t)lane < 4 * ccc - min(dd - hh, 4 * ccc)) cl[dd - hh + lane] = kNoRank;
+      if (lane < 8) {
+        const uint32_t m = lane >= 2 ? (uint32_t)s_mark[2 * lane - 4] | ((uint32_t)s_mark[2 * lane - 3] << 16) : 0u;
+        reinterpret_cast<uint32_t*>(rec + rk)[lane] = lane == 0 ? st : lane == 1 ? hcc | (ccc << 16) : m;
+      }
+      wave_lds_fence();
+    }
+  }
+  edges = wave_sum_u64(edges);
+  if (lane == 0) add_sum(counters, kSumEdges, edges);
+}
+
+// ---------------------------------------------------------------------------
+// One wave per chunk of S entries.  For every row v with N(v) not empty and
+// larger neighbours u in the chunk: N(v)'s hot ids become a bit map in LDS and
+// the u's hot prefixes are streamed through it; a cold v with cold ids hashes
+// these in the same LDS and streams the u's cold lists.
+//
+// 64 items (u's) are taken at once, one per lane, their 16-byte chunks numbered
+// through and dealt out one per lane and step, so every lane has a chunk
+// whatever the lists' lengths (a list per group of 4-16 lanes left 62 % of the
+// lanes without one at R-MAT s24: 27.4 ms against 21.9).  Chunk c belongs to item (number of items that
+// start at 1 .. c): lane b keeps the bits of the starts in chunks 64 b + 1 ..
+// 64 b + 64, so a step needs two readlanes and a masked bit count.
+constexpr int kStreamBlocks = kWave;  // 64-chunk blocks that the bits cover
+
+template <typename F>
+__device__ __forceinline__ void stream_lists(uint32_t start, uint32_t n, uint32_t* s_adj, unsigned long long* s_bit,
+                                             int lane, const uint4* __restrict__ lists, uint32_t pad, F&& probe) {
+  const uint32_t inc = wave_incl_scan_u32(n);
+  const uint32_t all = __builtin_amdgcn_readlane(inc, kWave - 1);
+  if (all == 0) return;  // uniform
+  auto load = [&](uint32_t at, bool on) -> uint4 {
+    uint4 v = make_uint4(pad, pad, pad, pad);
+    if (on) v = lists[at];
+    return v;
+  };
+  const uint64_t some = __builtin_amdgcn_ballot_w64(n > 0);
+  if (all <= kStreamBlocks * kWave) {
+    const uint32_t p = inc - n;
+    wave_lds_fence();
+    s_bit[lane] = 0ull;
+    if (n > 0) s_adj[lanes_below(some)] = start - p;
+    wave_lds_fence();
+    if (n > 0 && p > 0) atomicOr(&s_bit[(p - 1) >> 6], 1ull << ((p - 1) & 63));
+    wave_lds_fence();
+    const int64_t my = (int64_t)s_bit[lane];
+    const int steps = (int)((all + kWave - 1) / kWave);
+    uint32_t before = 0;
+    auto next = [&](int b) -> uint4 {
+      const uint64_t m = (uint64_t)readlane64(my, b);
+      const uint32_t c = (uint32_t)b * kWave + lane;
+      const uint32_t at = s_adj[before + lanes_below(m)] + c;
+      before += (uint32_t)__popcll(m);
+      return load(at, c < all);
+    };
+    // Two buffers by hand: the next step's loads are in flight while one is probed.
+    uint4 va = next(0), vb;
+    for (int b = 1;; b += 2) {
+      if (b < steps) vb = next(b);
+      probe(va);
+      if (b >= steps) break;
+      if (b + 1 < steps) va = next(b + 1);
+      probe(vb);
+      if (b + 1 >= steps) break;
+    }
+  } else {  // long lists: the whole wave on one item at a time
+    for (uint64_t left = some; left; left &= left - 1) {
+      const int k = __builtin_ctzll(left);
+      const uint32_t s0 = __builtin_amdgcn_readlane(start, k), nk = __builtin_amdgcn_readlane(n, k);
+      uint4 va = load(s0 + lane, (uint32_t)lane < nk), vb;
+      for (uint32_t c = kWave;; c += 2 * kWave) {
+        if (c < nk) vb = load(s0 + c + lane, c + lane < nk);
+        probe(va);
+        if (c >= nk) break;
+        if (c + kWave < nk) va = load(s0 + c + kWave + lane, c + kWave + lane < nk);
+        probe(vb);
+        if (c + kWave >= nk) break;
+      }
+    }
+  }
+}
+
+template <int LOGB>
+__device__ __forceinline__ void cold_table_clear(int4* tab, int lane) {
+#pragma unroll
+  for (int i = 0; i < (1 << LOGB) / kWave; i++) tab[lane + kWave * i] = make_int4(kEmpty, kEmpty, kEmpty, kEmpty);
+  wave_lds_fence();
+}
+
+struct Head {  // a record
+  uint4 a, b;
+};
+
+__global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const int64_t* __restrict__ off,
+                                                   const uint32_t* __restrict__ rank, const uint64_t* __restrict__ oc,
+                                                   const uint32_t* __restrict__ part, const RankRec* __restrict__ rec,
+                                                   const uint4* __restrict__ lists, const int32_t* __restrict__ crows,
+                                                   int64_t S, uint64_t* __restrict__ counters) {
+  constexpr int kWords = 2048;
+  constexpr int kColdSmall = 6, kColdBig = 9;  // hash buckets (log2) for up to 128 and up to 1024 cold ids
+  __shared__ uint4 s_mem[kWords / 4];
+  __shared__ unsigned long long s_bit[kStreamBlocks];
+  __shared__ uint32_t s_adj[kWave];
+  uint32_t* s_bm = reinterpret_cast<uint32_t*>(s_mem);
+  int4* s_tab = reinterpret_cast<int4*>(s_mem);
+  const int lane = threadIdx.x;
+  const int64_t c = blockIdx.x;
+  const int64_t eb = c * S, ee = min(ne, eb + S);
+  int64_t rlo = crows[2 * c], rhi = crows[2 * c + 1];
+  rlo = rlo < 0 ? 0 : (rlo > nv - 1 ? nv - 1 : rlo);
+  rhi = rhi < rlo ? rlo : (rhi > nv - 1 ? nv - 1 : rhi);
+  auto clear_words = [&](int quads) {  // 16-byte pieces from the front
+    for (int i = lane; i < quads; i += kWave) s_mem[i] = make_uint4(0, 0, 0, 0);
+  };
+  clear_words(kWords / 4);
+  wave_lds_fence();
+  auto tiny_rows = [&](bool tiny, uint32_t a0, uint32_t is, uint32_t items, uint32_t d) -> uint32_t {
+    const uint32_t n = tiny ? items : 0;
+    const uint32_t inc = wave_incl_scan_u32(n), p = inc - n;
+    const uint32_t all = __builtin_amdgcn_readlane(inc, kWave - 1);
+    const uint64_t some = __builtin_amdgcn_ballot_w64(n > 0);
+    wave_lds_fence();
+    s_bit[lane] = 0ull;
+    if (n > 0) s_adj[lanes_below(some)] = (uint32_t)lane;
+    wave_lds_fence();
+    if (n > 0 && p > 0) atomicOr(&s_bit[(p - 1) >> 6], 1ull << ((p - 1) & 63));
+    wave_lds_fence();
+    const int64_t my = (int64_t)s_bit[lane];
+    uint32_t before = 0, acc = 0;
+    for (uint32_t b = 0; b * kWave < all; b++) {
+      const uint64_t m = (uint64_t)readlane64(my, (int)b);
+      const uint32_t c = b * kWave + lane;
+      const int row = (int)s_adj[before + lanes_below(m)];
+      before += (uint32_t)__popcll(m);
+      const uint32_t entry = (uint32_t)__shfl((int)(is - p), row, kWave) + c;
+      const uint32_t first = (uint32_t)__shfl((int)a0, row, kWave), nd = (uint32_t)__shfl((int)d, row, kWave);
+      uint32_t x[kTinyRow];
+      uint2 r = make_uint2(0, 0);
+#pragma unroll
+      for (int i = 0; i < kTinyRow; i++) x[i] = kNoRank - 1;  // matches no id and no padding
+      if (c < all) {
+        const uint32_t ur = part[entry];
+#pragma unroll
+        for (int i = 0; i < kTinyRow; i++)
+          if ((uint32_t)i < nd) x[i] = part[first + i];
+        if (ur != kNoRank) r = *reinterpret_cast<const uint2*>(rec + ur);
+      }
+      const uint32_t hc = r.y & 0xffffu, cc = r.y >> 16;
+      for (uint32_t k = 0; __builtin_amdgcn_ballot_w64(k < hc); k++) {
+        if (k < hc) {
+          const uint4 q = lists[r.x + k];
+          const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            const uint32_t lo = w[j] & 0xffffu, hi = w[j] >> 16;
+            const uint32_t lo2 = lo < kHot ? lo : kNoRank, hi2 = hi < kHot ? hi : kNoRank;
+#pragma unroll
+            for (int i = 0; i < kTinyRow; i++) acc += (x[i] == lo2 ? 1u : 0u) + (x[i] == hi2 ? 1u : 0u);
+          }
+        }
+      }
+      for (uint32_t k = 0; __builtin_amdgcn_ballot_w64(k < cc); k++) {
+        if (k < cc) {
+          const uint4 q = lists[r.x + hc + k];
+          const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+          for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int i = 0; i < kTinyRow; i++) acc += x[i] == w[j] ? 1u : 0u;
+        }
+      }
+    }
+    return acc;
+  };
+  uint64_t hits = 0;
+  for (int64_t rb = rlo; rb <= rhi; rb += kWave) {
+    const int64_t r = rb + lane;
+    int64_t a0 = 0, is = 0, ie = 0;
+    uint32_t d = 0, h = 0, v = 0;
+    if (r <= rhi) {
+      const uint64_t q = oc[r];
+      a0 = off[r];
+      ie = min(off[r + 1], ee);
+      v = rank[r];
+      d = (uint32_t)q;
+      h = (uint32_t)(q >> 32);
+      is = max(a0 + (int64_t)d, eb);
+    }
+    const bool work = d > 0 && is < ie;
+    // Rows of few ids and few items: their items are taken together, one lane
+    // per item, every id of N(v) compared with every id of u's list.
+    const bool tiny = work && d <= kTinyRow && ie - is <= kWave;
+    if (__builtin_amdgcn_ballot_w64(tiny)) hits += tiny_rows(tiny, (uint32_t)a0, (uint32_t)is, (uint32_t)(ie - is), d);
+    uint64_t todo = __builtin_amdgcn_ballot_w64(work && !tiny);
+    // Row by row; the next row's ids and items are loaded before the current
+    // row's map is built, its items' records before the current lists stream.
+    uint32_t b0 = 0, s0 = 0, s1 = 0, dd = 0, hh = 0, vv = 0;
+    auto pop = [&]() {
+      const int src = __builtin_ctzll(todo);
+      todo &= todo - 1;
+      b0 = __builtin_amdgcn_readlane((uint32_t)a0, src);
+      s0 = __builtin_amdgcn_readlane((uint32_t)is, src);
+      s1 = __builtin_amdgcn_readlane((uint32_t)ie, src);
+      dd = __builtin_amdgcn_readlane(d, src);
+      hh = __builtin_amdgcn_readlane(h, src);
+      vv = __builtin_amdgcn_readlane(v, src);
+    };
+    auto item = [&](uint32_t e) -> uint32_t { return e + lane < s1 ? part[e + lane] : kNoRank; };
+    auto head = [&](uint32_t ur) -> Head {
+      Head x{make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)};
+      if (ur != kNoRank) {
+        const uint4* q = reinterpret_cast<const uint4*>(rec + ur);
+        x.a = q[0];
+        x.b = q[1];
+      }
+      return x;
+    };
+    if (todo == 0) continue;  // uniform
+    pop();
+    uint32_t w0 = (uint32_t)lane < dd ? part[b0 + lane] : kNoRank;
+    Head x = head(item(s0));
+    for (;;) {  // uniform
+      const uint32_t cb = b0, cs0 = s0, cs1 = s1, cd = dd, ch = hh, cv = vv, w = w0;
+      const bool more = todo != 0;
+      uint32_t un = kNoRank;
+      if (more) {
+        pop();
+        w0 = (uint32_t)lane < dd ? part[b0 + lane] : kNoRank;
+        un = item(s0);
+      }
+      auto id = [&](uint32_t i) -> uint32_t { return i == 0 ? w : i + lane < cd ? part[cb + i + lane] : kNoRank; };
+      // Hot chunks of the item whose record is h that hold every id below v.
+      auto prefix = [&](const Head& h) -> uint32_t {
+        const uint32_t hot = h.a.y & 0xffffu;
+        const uint32_t mk[kRankMarks / 2] = {h.a.z, h.a.w, h.b.x, h.b.y, h.b.z, h.b.w};
+        uint32_t segs = 0;  // segments that start below v
+#pragma unroll
+        for (int t = 0; t < kRankMarks / 2; t++) segs += ((mk[t] & 0xffffu) < cv ? 1u : 0u) + ((mk[t] >> 16) < cv ? 1u : 0u);
+        return min(segs * mark_step(hot), hot);
+      };
+      const bool cold = ch < cd && cv > kHot;  // cold ids below a cold v
+      const uint32_t st = x.a.x, len = x.a.y, n = prefix(x);  // the first 64 items
+      if (ch > 0)
+        for (uint32_t i = 0; i < cd; i += kWave) {
+          const uint32_t y = id(i);
+          if (y < kHot) atomicOr(&s_bm[y >> 5], 1u << (y & 31));
+        }
+      if (more) x = head(un);
+      auto items = [&](uint32_t e) -> uint32_t { return e + lane < cs1 ? part[e + lane] : kNoRank; };
+      if (ch > 0) {
+        uint32_t acc = 0;
+        auto probe = [&](const uint4 q) {
+          const uint32_t y[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            const uint32_t lo = s_bm[(y[j] >> 5) & 2047u], hi = s_bm[y[j] >> 21];
+            acc += (lo >> (y[j] & 31)) & 1u;
+            acc += (hi >> ((y[j] >> 16) & 31)) & 1u;
+          }
+        };
+        Head y = cs0 + kWave < cs1 ? head(items(cs0 + kWave)) : Head{};
+        stream_lists(st, n, s_adj, s_bit, lane, lists, 0xffffffffu, probe);
+        for (uint32_t e = cs0 + kWave; e < cs1; e += kWave) {
+          const uint32_t sty = y.a.x, ny = prefix(y);
+          if (e + kWave < cs1) y = head(items(e + kWave));
+          stream_lists(sty, ny, s_adj, s_bit, lane, lists, 0xffffffffu, probe);
+        }
+        hits += acc;
+        wave_lds_fence();
+        if (cd <= 8 * kWave) {
+          for (uint32_t i = 0; i < cd; i += kWave) {
+            const uint32_t y = id(i);
+            if (y < kHot) s_bm[y >> 5] = 0;
+          }
+        } else {
+          clear_words(kWords / 4);
+        }
+        wave_lds_fence();
+      }
+      if (cold) {
+        uint32_t acc = 0;
+        // Cold ids [first, first + room) of N(v), in row order, hashed.
+        auto pass = [&](auto logb, uint32_t first, uint32_t room) {
+          constexpr int L = decltype(logb)::value;
+          cold_table_clear<L>(s_tab, lane);
+          bool passed = false;
+          uint32_t seen = 0;
+          for (uint32_t i = 0; i < cd; i += kWave) {
+            const uint32_t y = id(i);
+            const bool in = i + lane < cd && y >= kHot;
+            const uint64_t m = __builtin_amdgcn_ballot_w64(in);
+            const uint32_t at = seen + lanes_below(m);
+            if (in && at >= first && at - first < room) passed |= wave_tab_insert<L>(s_tab, (int32_t)y);
+            seen += (uint32_t)__popcll(m);
+          }
+          const bool spl = __builtin_amdgcn_ballot_w64(passed) != 0;
+          wave_lds_fence();
+          auto probe = [&](const uint4 q) {
+            const int32_t y[4] = {(int32_t)q.x, (int32_t)q.y, (int32_t)q.z, (int32_t)q.w};
+            int4 t[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) t[j] = s_tab[wave_bucket<L>(y[j])];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+              bool hit = bucket_miss(t[j], y[j]) == 0;
+              if (spl && !hit && bucket_spilled(t[j]) && y[j] != -1)
+                hit = wave_tab_continue<L>(s_tab, wave_bucket<L>(y[j]), y[j]);
+              acc += hit ? 1u : 0u;
+            }
+          };
+          stream_lists(st + (len & 0xffffu), len >> 16, s_adj, s_bit, lane, lists, kNoRank, probe);
+          for (uint32_t e = cs0 + kWave; e < cs1; e += kWave) {
+            const uint32_t ur = items(e);
+            uint2 y = make_uint2(0, 0);
+            if (ur != kNoRank) y = *reinterpret_cast<const uint2*>(rec + ur);
+            stream_lists(y.x + (y.y & 0xffffu), y.y >> 16, s_adj, s_bit, lane, lists, kNoRank, probe);
+          }
+          wave_lds_fence();
+          clear_words(1 << L);
+          wave_lds_fence();
+        };
+        const uint32_t ncold = cd - ch;
+        if (ncold <= (2u << kColdSmall)) {
+          pass(std::integral_constant<int, kColdSmall>{}, 0u, ncold);
+        } else {
+          for (uint32_t f = 0; f < ncold; f += 2u << kColdBig) pass(std::integral_constant<int, kColdBig>{}, f, 2u << kColdBig);
+        }
+        hits += acc;
+      }
+      if (!more) break;
+    }
+  }
+  hits = wave_sum_u64(hits);
+  if (lane == 0) add_sum(counters, kSumTotal, hits);
+}
+
+// ---------------------------------------------------------------------------
+static unsigned rank_grid(int64_t n, int per, int64_t cap) {
+  int64_t g = (n + per - 1) / per;
+  g = g < 1 ? 1 : g > cap ? cap : g;
+  return (unsigned)g;
+}
+
+// Room for the lists of a simple graph, in 128-byte lines: |E+| = ne / 2 ids; a
+// list of d >= 2 ids is given at most min(d, d / 4 + 9.25) chunks (hot and cold
+// parts rounded up to chunks, then to list_room), a wave's lists at a time
+// rounded up to a line.  Grants but a wave's last are used to three quarters.
+// A region is left for the next when a request does not fit, so each may lose
+// one request: a grant, or 64 of the longest lists (at most 1.02 sqrt(ne) ids,
+// since out-neighbours have about the vertex's degree or more).
+static ListRoom rank_list_room(const xt_ctx* ctx, int64_t nv, int64_t ne, int64_t* lines) {
+  ListRoom r;
+  const int64_t waves = (int64_t)ctx->num_cus * 16;
+  r.rows = kWave;
+  while (r.rows > 16 && nv / r.rows < waves) r.rows >>= 1;
+  // Four neighbours read a quarter of a line of each vertex array: all right
+  // while these stay in the 256 MB cache (20 bytes a vertex).
+  r.together = nv <= (1ll << 22) ? 2 : 4;
+  r.nbatch = (nv + r.rows - 1) / r.rows;
+  const int64_t nlists = nv < ne / 4 ? nv : ne / 4;
+  const int64_t chunks = ne / 8 + 10 * nlists < ne / 2 ? ne / 8 + 10 * nlists : ne / 2;
+  const int64_t need = chunks / 8 + r.nbatch + 1;
+  const int64_t grant = need / (waves * 32) < 8 ? 8 : need / (waves * 32);
+  const int64_t used = need + need / 3 + (r.nbatch < waves ? r.nbatch : waves) * grant;
+  const double longest = 1.05 * std::sqrt((double)ne) + 64.0;
+  const int64_t most = grant + (int64_t)(64.0 * (longest / 4 + 10) / 8) + 1;
+  r.grant = (uint64_t)grant;
+  r.region = (uint64_t)(used / kListShards + most + 1);
+  *lines = (int64_t)r.region * kListShards;
+  return r;
+}
+
+// Ranks, chunk starts of lists and entry indices fit their 32 bits.
+bool rank_fits(const xt_ctx* ctx, int64_t nv, int64_t ne) {
+  if (nv >= (1ll << 30) || ne >= (1ll << 32)) return false;
+  int64_t lines;
+  rank_list_room(ctx, nv, ne, &lines);
+  return lines < (1ll << 29);
+}
+
+// Entries per wave of k_rank_count.
+static int64_t rank_chunk(const xt_ctx* ctx, int64_t ne) {
+  int64_t S = kChunk;
+  while (S > 256 && ne / S < (int64_t)ctx->num_cus * 18 * 8) S >>= 1;
+  return S;
+}
+
+template <typename T>
+int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* off, const T* tails, hipStream_t st,
+               hipEvent_t split_done) {
+  const int64_t S = rank_chunk(ctx, ne);
+  const int64_t nch = (ne + S - 1) / S, nchunks = (ne + kChunk - 1) / kChunk;
+  XT_TRY(ensure(ctx, s.crows, (size_t)(2 * nch) * sizeof(int32_t)));
+  XT_TRY(ensure(ctx, s.rank, (size_t)nv * sizeof(uint32_t)));
+  XT_TRY(ensure(ctx, s.ocount, (size_t)nv * sizeof(uint64_t)));
+  XT_TRY(ensure(ctx, s.itcnt, (size_t)nv * sizeof(uint32_t)));
+  XT_TRY(ensure(ctx, s.rpart, (size_t)(ne + kWave) * sizeof(uint32_t)));  // a wave reads past a short row
+  int64_t lines;
+  const ListRoom lr = rank_list_room(ctx, nv, ne, &lines);
+  XT_TRY(ensure(ctx, s.rlists, (size_t)lines * 128));
+  XT_TRY(ensure(ctx, s.rrec, (size_t)nv * sizeof(RankRec)));
+  XT_TRY(ensure(ctx, s.rhist, (size_t)(2 * kRankClasses) * sizeof(uint32_t)));
+  uint64_t* counters = s.counters.as<uint64_t>();
+  uint32_t* hist = s.rhist.as<uint32_t>();
+  int32_t* crows = s.crows.as<int32_t>();
+  uint32_t* rank = s.rank.as<uint32_t>();
+  uint64_t* oc = s.ocount.as<uint64_t>();
+  uint32_t* part = s.rpart.as<uint32_t>();
+  uint4* lists = s.rlists.as<uint4>();
+  RankRec* rec = s.rrec.as<RankRec>();
+  XT_TRY(fill_u32(ctx, hist, 2 * kRankClasses, 0u, st));
+  hipLaunchKernelGGL(k_rank_prep, dim3(rank_grid(nv, 1024, 8192)), dim3(256), 0, st, nv, ne, off, S, crows, oc,
+                     s.itcnt.as<uint32_t>(), hist);
+  XT_HIP(ctx, hipGetLastError());
+  hipLaunchKernelGGL(k_rank_assign, dim3(rank_grid(nv, 256 * kAssignRun, 1ll << 31)), dim3(256), 0, st, nv, off,
+                     (const uint32_t*)hist, hist + kRankClasses, rank);
+  XT_HIP(ctx, hipGetLastError());
+  hipLaunchKernelGGL((k_rank_split<T>), dim3(xcd_grid(nchunks)), dim3(kBlock), 0, st, nv, ne, off, tails,
+                     (const uint32_t*)rank, (const int32_t*)crows, (int)(kChunk / S), part, oc,
+                     s.itcnt.as<uint32_t>(), counters);
+  XT_HIP(ctx, hipGetLastError());
+  hipLaunchKernelGGL(k_rank_lists, dim3(rank_grid(lr.nbatch, 1, (int64_t)ctx->num_cus * 16)), dim3(64), 0, st, nv, off,
+                     (const uint64_t*)oc, (const uint32_t*)rank, (const uint32_t*)part, lr, lists, rec, counters);
+  XT_HIP(ctx, hipGetLastError());
+  if (split_done) XT_HIP(ctx, hipEventRecord(split_done, st));
+  hipLaunchKernelGGL(k_rank_count, dim3((unsigned)nch), dim3(64), 0, st, nv, ne, off, (const uint32_t*)rank,
+                     (const uint64_t*)oc, (const uint32_t*)part, (const RankRec*)rec, (const uint4*)lists,
+                     (const int32_t*)crows, S, counters);
+  XT_HIP(ctx, hipGetLastError());
+  return XT_OK;
+}
+
+template int rank_count<int32_t>(xt_ctx*, Scratch&, int64_t, int64_t, const int64_t*, const int32_t*, hipStream_t,
+                                 hipEvent_t);
+template int rank_count<int64_t>(xt_ctx*, Scratch&, int64_t, int64_t, const int64_t*, const int64_t*, hipStream_t,
+                                 hipEvent_t);
+
+}  // namespace xt

@@ -180,13 +180,6 @@ __device__ __forceinline__ void load_run(const T* __restrict__ tails, int64_t e0
   for (int j = 0; j < kRun; j++) vals[j] = (e0 + j < ee) ? (int64_t)tails[e0 + j] : 0;
 }
 
-// Adds v to sum k of the shard that this workgroup adds to (shards after
-// `slots` slots, `sums` words apart).
-__device__ __forceinline__ void add_to_shard(uint64_t* counters, int slots, int shards, int sums, int k, uint64_t v) {
-  if (v)
-    atomicAdd((unsigned long long*)&counters[slots + (int)(blockIdx.x & (shards - 1)) * sums + k], (unsigned long long)v);
-}
-
 // SplitMix64 output function (Steele, Lea, Flood, OOPSLA 2014).
 __device__ __forceinline__ uint64_t mix64_dev(uint64_t z) {
   z += 0x9E3779B97F4A7C15ULL;

@@ -38,7 +38,6 @@ constexpr int64_t kBatchWaveMinEntries = int64_t(1) << 22;  // a batch
 
 // Counter slots in Scratch::counters (uint64).
 enum Slot : int {
-  kTotal = 0,          // global triangle count
   kBadIds = 3,         // neighbour ids outside [0, nv)
   kBadRows = 4,        // rows not strictly ascending
   kAsym = 5,           // entries without their reverse entry
@@ -47,9 +46,6 @@ enum Slot : int {
   kTileQueue = 8,      // next tile of the persistent group kernel
   kStatMinHeavy = 9,   // same sum over heavy edges only
   kStatHeavyEdges = 10,// number of heavy edges
-  kHeavyItems = 11,    // heavy edges listed under their owners by the counting pass
-  kOwned = 12,         // owned-range count: triangles whose minimum vertex is owned
-  kLocal = 13,         // ... and whose middle vertex is owned too
   kWaveQueue = 14,     // next wave tile of k_count_waves, one queue per XCD (14..21)
   kNumSlots = 32
 };
@@ -59,13 +55,22 @@ enum Slot : int {
 // address are made one after another, about 18 ns apart whatever the XCD: a
 // million workgroups on one address take 18 ms.
 enum Sum : int {
-  kSumTotal = 0,  // triangles (rank space)
+  kSumTotal = 0,  // global triangle count
+  kSumOwned,      // owned-range count: triangles whose minimum vertex is owned
+  kSumLocal,      // ... and whose middle vertex is owned too
+  kSumHeavy,      // heavy edges listed under their owners by the counting pass
   kSumEdges,      // oriented edges (rank space)
   kSumLists,      // 128-byte lines handed out of the shard's region (rank space)
   kNumSums = 16
 };
 constexpr int kShards = 64;
 constexpr int kNumCounters = kNumSlots + kShards * kNumSums;
+
+__device__ __forceinline__ void add_sum(uint64_t* counters, Sum k, uint64_t v) {
+  if (v)
+    atomicAdd((unsigned long long*)&counters[kNumSlots + (int)(blockIdx.x & (kShards - 1)) * kNumSums + k],
+              (unsigned long long)v);
+}
 
 inline uint64_t sum_of(const uint64_t* counters, Sum k) {
   uint64_t t = 0;
@@ -171,7 +176,7 @@ int orient(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* off, 
            hipStream_t st);
 
 // Intersection + reduction over the context's oriented CSR.  Adds the global
-// count to ctx counters[0]; per-vertex counts into pv when pv != nullptr.
+// count to the sum kSumTotal; per-vertex counts into pv when pv != nullptr.
 // Batch mode: gid (graph of each vertex) and gtotal (per-graph totals) non-null
 // and the intersection kernel drains a device tile queue with a fixed grid.
 // evs (nullable): two events recorded after the light-edge kernel and after
@@ -220,8 +225,7 @@ int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* o
                hipEvent_t split_done);
 
 // Whole single-graph count on the device (orientation + intersection).
-// may_rank: a plain total may be counted in rank space.  The total is the slot
-// kTotal plus the sum kSumTotal.
+// may_rank: a plain total may be counted in rank space.
 template <typename T>
 int count_device_csr(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* off, const T* tails,
                      uint32_t flags, hipStream_t st, bool timed, bool may_rank,
