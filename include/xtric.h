@@ -63,7 +63,8 @@ typedef struct xt_timing {
   double group_ms;    /* persistent group kernel: staged list x streamed lists */
   int64_t ne_plus;    /* oriented edges |E+| */
   int64_t n_heavy;    /* oriented edges intersected by the group kernel (rank space: all) */
-  int64_t n_tiles;    /* group tiles drawn from the device work queue (rank space: 0) */
+  int64_t n_tiles;    /* group tiles drawn from the device work queue (rank space: chunks of
+                         entries, a wave each) */
   int64_t n_wave_tiles; /* wave tiles (owners with short out-lists, k_count_waves) */
 } xt_timing;
 
@@ -74,11 +75,12 @@ int xt_ctx_create(int device, xt_ctx** out);
 int xt_ctx_destroy(xt_ctx* ctx);
 const char* xt_last_error(const xt_ctx* ctx);
 int xt_last_timing(const xt_ctx* ctx, xt_timing* out);
-/* Plain totals of one graph in degree orientation are counted in rank space
- * (vertices ranked by degree, lists of smaller ranks in 16 bits, bit maps in
- * LDS); the knobs below belong to the edge tiles that all other counts use, and
- * a context on which one of them is away from its default uses edge tiles for
- * plain totals too.
+/* Totals of one graph in degree orientation are counted in rank space (vertices
+ * ranked by degree, lists of smaller ranks in 16 bits, bit maps in LDS), and so
+ * are its per-vertex counts below 2^25 entries and, where the host passed in the
+ * offsets and no row is longer than 256, counts in id orientation.  The knobs
+ * below belong to the edge tiles that all other counts use; a context on which
+ * one of them is away from its default uses edge tiles for all of them.
  * Tuning knobs (set by xxtric_amd.autotune from measurements; 0 keeps the
  * current value): light_cut -- edges whose two out-lists are both at most this
  * long are intersected one per thread, the rest by the group kernel or wave

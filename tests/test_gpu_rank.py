@@ -1,5 +1,5 @@
-"""The count in rank space (plain totals in degree orientation, library default
-knobs) at the sizes where it can go wrong: lists around one chunk, one line and
+"""The count in rank space (totals and per-vertex counts, library default knobs)
+at the sizes where it can go wrong: lists around one chunk, one line and
 one wave, ranks on both sides of the 16-bit limit, more cold ids than one hash
 holds, rows across chunks, rows of many empty neighbours, labels in any order.
 Expected values: the oracle, closed forms, and the edge tiles (asked for by
@@ -19,12 +19,16 @@ def _say(*a):
     print("[case]", *a, flush=True)
 
 
-def _tiles(ctx, g):
+def _tiles(ctx, g, **kw):
     ctx.tune(small_cut=32)
     try:
-        return g.count()
+        return g.count(**kw)
     finally:
         ctx.tune(small_cut=-1)
+
+
+def _same(a, b):
+    return a[0] == b[0] and (a[1] == b[1]).all()
 
 
 def _circulant(n, k):
@@ -44,7 +48,11 @@ def test_list_lengths(ctx, n):
     _say("complete", n)
     off = np.arange(n + 1, dtype=np.int64) * (n - 1)
     cols = np.tile(np.arange(n, dtype=np.int64), n).reshape(n, n)
-    assert ctx.count_csr(off, cols[~np.eye(n, dtype=bool)].reshape(-1)) == n * (n - 1) * (n - 2) // 6
+    tails = cols[~np.eye(n, dtype=bool)].reshape(-1)
+    assert ctx.count_csr(off, tails) == n * (n - 1) * (n - 2) // 6
+    i = np.arange(n, dtype=np.int64)
+    tot, pv = ctx.count_csr(off, tails, per_vertex=True)   # from 512 ids on: beyond the slots in LDS
+    assert tot == n * (n - 1) * (n - 2) // 6 and (pv == (n - 1 - i) * (n - 2 - i) // 2).all()
 
 
 @pytest.mark.parametrize("n", [HOT - 1, HOT, HOT + 1, HOT + 2, HOT + 70])
@@ -52,7 +60,13 @@ def test_ranks_around_the_hot_limit(ctx, n):
     """All degrees equal, so any vertex may take the ranks on either side."""
     k = 5
     _say("circulant", n, k)
-    assert ctx.count_csr(*_circulant(n, k)) == n * k * (k - 1) // 2
+    off, tails = _circulant(n, k)
+    assert ctx.count_csr(off, tails) == n * k * (k - 1) // 2
+    for orient in ("degree", "id"):
+        _say(orient)
+        tot, pv = ctx.count_csr(off, tails, per_vertex=True, orient=orient)
+        assert tot == n * k * (k - 1) // 2 == int(pv.sum())
+        assert (pv[:n - 2 * k] [2 * k:] == k * (k - 1) // 2).all()  # rows that do not wrap
 
 
 @pytest.mark.parametrize("k,clique", [(34, 64), (110, 200), (600, 1150)])
@@ -68,6 +82,10 @@ def test_cold_lists(ctx, k, clique):
     exp = n * k * (k - 1) // 2 + clique * (clique - 1) * (clique - 2) // 6
     assert g.count() == exp
     assert ctx.timing()["ne_plus"] == len(tails) // 2
+    if len(tails) < 1 << 25:
+        tot, pv = g.count(per_vertex=True)
+        assert tot == exp and (pv[n:] == (clique - 1 - i) * (clique - 2 - i) // 2).all()
+        assert int(pv.sum(dtype=np.uint64)) == exp
     g.close()
 
 
@@ -93,6 +111,9 @@ def test_row_shapes(ctx, make):
     assert ctx.count_csr(off, tails) == exp
     g = ctx.graph(off, tails)
     assert g.count() == exp and _tiles(ctx, g) == exp
+    ref = O.count_reference(off, tails.astype(np.int32), per_vertex=True)
+    for orient in ("degree", "id"):
+        assert _same(g.count(per_vertex=True, orient=orient), ref) and g.count(orient=orient) == exp
     g.close()
 
 
@@ -102,9 +123,22 @@ def test_rmat_equals_the_edge_tiles(ctx, scale, permute):
     g = ctx.rmat(scale, 16, 5, permute)
     a = g.count()
     assert a == _tiles(ctx, g) == g.count(orient="id")
+    assert _same(g.count(per_vertex=True), _tiles(ctx, g, per_vertex=True))
     if scale <= 17:
         assert a == O.count_degree_ordered(*g.download())
     g.close()
+
+
+@pytest.mark.parametrize("orient", ["degree", "id"])
+@pytest.mark.parametrize("n", [70, 5000, 90000])
+def test_host_csr_per_vertex(ctx, n, orient):
+    """Short rows, also past the 16-bit limit (cold lists), against the reference restatement."""
+    import xxtric_amd
+    off, tails = xxtric_amd.rgg_generate(n, seed=3, connect=True, strict=True)
+    _say("rgg", n, orient)
+    exp = O.count_reference(off, tails.astype(np.int32), per_vertex=True)
+    assert _same(ctx.count_csr(off, tails, per_vertex=True, orient=orient), exp)
+    assert ctx.count_csr(off, tails, orient=orient) == exp[0]
 
 
 def test_device_csr_and_graph_sizes_in_a_row(ctx):

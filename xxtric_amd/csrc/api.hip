@@ -147,30 +147,50 @@ static int noalloc_init(xt_ctx* ctx, int device) {
   return XT_OK;
 }
 
-static int check_host_offsets(xt_ctx* ctx, int64_t nv, int64_t ne, const int64_t* off) {
+// max_degree (nullable) gets the longest row.
+static int check_host_offsets(xt_ctx* ctx, int64_t nv, int64_t ne, const int64_t* off, int64_t* max_degree) {
   if (nv < 0 || ne < 0 || !off) return set_err(ctx, XT_ERR_ARG, "negative size or null offsets");
   if (nv >= (1LL << 31) - 1) return set_err(ctx, XT_ERR_ARG, "nv must be below 2^31-1 (int32 device ids)");
   if (off[0] != 0 || off[nv] != ne) return set_err(ctx, XT_ERR_INPUT, "offsets must start at 0 and end at ne");
-  for (int64_t i = 0; i < nv; i++)
-    if (off[i] > off[i + 1]) return set_err(ctx, XT_ERR_INPUT, "offsets are not monotone");
+  int64_t least = 0, most = 0;
+  for (int64_t i = 0; i < nv; i++) {
+    const int64_t d = off[i + 1] - off[i];
+    least = d < least ? d : least;
+    most = d > most ? d : most;
+  }
+  if (least < 0) return set_err(ctx, XT_ERR_INPUT, "offsets are not monotone");
+  if (max_degree) *max_degree = most;
   return XT_OK;
 }
 
-// Whether a plain total in degree orientation is counted in rank space: at
-// every size (ms per count, rank space against edge tiles: RGG n = 64 0.03 and
-// 0.09, n = 100,000 0.07 and 0.14; G(n, p) of degree 64 on 200,000 0.46 and
-// 1.45; R-MAT s18 0.30 and 0.85, s22 6.4 and 12.3, s26 189 and 357).  The knobs
-// of the edge tiles, when set, ask for those.
-static bool ranks(const xt_ctx* ctx, int64_t nv, int64_t ne) {
+// Per-vertex counts go to rank space below this many entries: the credit of
+// every hit there costs more than in the edge tiles' hash table, the rest less
+// (ms, rank space against edge tiles: R-MAT s14 0.11 and 0.40, s18 0.88 and
+// 1.08, s20 4.1 and 4.2, s21 9.6 and 8.7; G(n, p) of degree 64 on 200,000 0.83
+// and 2.5).
+constexpr int64_t kRankPvEntries = int64_t(1) << 25;
+// In id orientation out-lists are as long as rows; where rows are long, one
+// wave's list or map waits for another (ms: RGG n = 200,000 0.18 and 0.31,
+// G(n, p) of degree 64 0.87 and 2.6, but R-MAT s14, rows to 3,700, 0.71 and 0.38).
+constexpr int64_t kRankIdDegree = 256;
+
+// Whether a count goes to rank space.  Plain totals in degree orientation do at
+// every size (ms, rank space against edge tiles: RGG n = 64 0.03 and 0.09,
+// n = 100,000 0.07 and 0.14; G(n, p) of degree 64 on 200,000 0.46 and 1.45;
+// R-MAT s18 0.30 and 0.85, s22 6.4 and 12.3, s26 189 and 357).  The knobs of the
+// edge tiles, when set, ask for those.
+static bool ranks(const xt_ctx* ctx, int64_t nv, int64_t ne, int mode, bool per_vertex, int64_t max_degree) {
+  if (mode == kOrientId && (max_degree < 0 || max_degree > kRankIdDegree)) return false;
+  if (per_vertex && ne >= kRankPvEntries) return false;
   const bool knobs = ctx->small_cut != 0 || ctx->wave_owner != -1 || ctx->group_blocks != 4 || ctx->group_round != 2 ||
                      ctx->group_hash != kHashMix || ctx->items_per_tile != 256 || ctx->tile_run != 16 ||
                      ctx->force_wide;
-  return !knobs && ne > 0 && rank_fits(ctx, nv, ne);
+  return !knobs && ne > 0 && rank_fits(ctx, nv, ne, mode);
 }
 
 template <typename T>
 int count_device_csr(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* off,
-                     const T* tails, uint32_t flags, hipStream_t st, bool timed, bool may_rank,
+                     const T* tails, uint32_t flags, hipStream_t st, bool timed, RankUse rank,
                      const OwnedRange* range) {
   const int mode = (flags & XT_ORIENT_ID) ? kOrientId : kOrientDegree;
   ctx->last_ranked = false;
@@ -181,9 +201,9 @@ int count_device_csr(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int6
     XT_TRY(ensure(ctx, s.pv, (size_t)(nv > 0 ? nv : 1) * sizeof(uint64_t)));
     pv = s.pv.as<uint64_t>();
   }
-  if (may_rank && !pv && !range && mode == kOrientDegree && ranks(ctx, nv, ne)) {
+  if (rank.may && !range && ranks(ctx, nv, ne, mode, pv != nullptr, rank.max_degree)) {
     if (timed) XT_HIP(ctx, hipEventRecord(ctx->ev[kEvStart], st));
-    XT_TRY(rank_count<T>(ctx, s, nv, ne, off, tails, st, timed ? ctx->ev[kEvOriented] : nullptr));
+    XT_TRY(rank_count<T>(ctx, s, nv, ne, off, tails, mode, pv, st, timed ? ctx->ev[kEvOriented] : nullptr));
     if (timed) XT_HIP(ctx, hipEventRecord(ctx->ev[kEvCounted], st));
     ctx->last_ranked = true;
     return XT_OK;
@@ -203,9 +223,9 @@ int count_device_csr(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int6
 }
 
 template int count_device_csr<int32_t>(xt_ctx*, Scratch&, int64_t, int64_t, const int64_t*, const int32_t*,
-                                       uint32_t, hipStream_t, bool, bool, const OwnedRange*);
+                                       uint32_t, hipStream_t, bool, RankUse, const OwnedRange*);
 template int count_device_csr<int64_t>(xt_ctx*, Scratch&, int64_t, int64_t, const int64_t*, const int64_t*,
-                                       uint32_t, hipStream_t, bool, bool, const OwnedRange*);
+                                       uint32_t, hipStream_t, bool, RankUse, const OwnedRange*);
 
 // Reads the count, the input-error slots and the timing after a count; sums
 // (nullable, kNumCounters words) gets all counters.
@@ -223,10 +243,12 @@ static int finish_count(xt_ctx* ctx, int64_t nv, uint32_t flags, hipStream_t st,
   int64_t nep = 0, nheavy = 0, ntiles = 0, nwave = 0;
   const bool ranked = ctx->last_ranked;
   const bool worked = nv > 0 && ctx->s.itcnt.p != nullptr && ctx->s.ooff.p != nullptr;
-  if (ranked)
+  if (ranked) {
     nep = nheavy = (int64_t)sum_of(h, kSumEdges);
-  else if (nv > 0)
+    ntiles = ctx->rank_chunks;
+  } else if (nv > 0) {
     XT_HIP(ctx, hipMemcpy(&nep, ctx->s.ooff.as<int64_t>() + nv, sizeof(int64_t), hipMemcpyDeviceToHost));
+  }
   const bool split = worked && nep > 0 && !ranked;  // the light/items/group phases ran
   if (split) {
     nheavy = (int64_t)sum_of(h, kSumHeavy);
@@ -541,7 +563,8 @@ int xt_count_csr(xt_ctx* ctx, int64_t nv, int64_t ne, const int64_t* offsets, co
     XT_HIP(ctx, hipSetDevice(ctx->device));
     if (!total || (ne > 0 && !tails)) return set_err(ctx, XT_ERR_ARG, "null output or tails");
     if (per_vertex && !(flags & XT_PER_VERTEX)) return set_err(ctx, XT_ERR_ARG, "per_vertex needs XT_PER_VERTEX");
-    XT_TRY(check_host_offsets(ctx, nv, ne, offsets));
+    int64_t max_degree = -1;
+    XT_TRY(check_host_offsets(ctx, nv, ne, offsets, &max_degree));
     hipStream_t st = ctx->stream;
     XT_TRY(ensure(ctx, ctx->s.in_off, (size_t)(nv + 1) * sizeof(int64_t)));
     XT_TRY(ensure(ctx, ctx->s.in_tails, (size_t)(ne > 0 ? ne : 1) * sizeof(int32_t)));
@@ -549,7 +572,7 @@ int xt_count_csr(xt_ctx* ctx, int64_t nv, int64_t ne, const int64_t* offsets, co
     int32_t* d_tails = ctx->s.in_tails.as<int32_t>();
     XT_TRY(upload_csr(ctx, nv, ne, offsets, tails, 8, d_off, d_tails, st));
     if (flags & XT_VALIDATE) XT_TRY(validate<int32_t>(ctx, nv, ne, d_off, d_tails, (flags & XT_CHECK_SYMMETRY) != 0, st));
-    XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, nv, ne, d_off, d_tails, flags, st, true, true));
+    XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, nv, ne, d_off, d_tails, flags, st, true, RankUse{true, max_degree}));
     return finish_count(ctx, nv, flags, st, true, total, per_vertex);
   });
 }
@@ -573,7 +596,7 @@ int xt_single_gpu_count(xt_ctx* ctx, int64_t nv, const int64_t* d_indices, const
     // Offsets must be a valid index (and rows sorted) before the chunked
     // kernels search them; the reference launcher assumes the same.
     XT_TRY(validate<int64_t>(ctx, nv, ne, d_indices, d_edge_list, false, st));
-    XT_TRY(count_device_csr<int64_t>(ctx, ctx->s, nv, ne, d_indices, d_edge_list, XT_ORIENT_DEGREE, st, false, true));
+    XT_TRY(count_device_csr<int64_t>(ctx, ctx->s, nv, ne, d_indices, d_edge_list, XT_ORIENT_DEGREE, st, false, RankUse{true, -1}));
     uint64_t bad = 0;
     XT_HIP(ctx, hipMemcpyAsync(&bad, ctx->s.counters.as<uint64_t>() + kBadIds, sizeof(bad),
                                hipMemcpyDeviceToHost, st));
@@ -618,7 +641,7 @@ int xt_single_gpu_count_noalloc(xt_ctx* ctx, int64_t nv, const int64_t* d_indice
     uint64_t* counters = s.counters.as<uint64_t>();
     auto run = [&]() -> int {
       XT_TRY(validate<int64_t>(ctx, nv, ne, d_indices, d_edge_list, false, st, counters));
-      XT_TRY(count_device_csr<int64_t>(ctx, s, nv, ne, d_indices, d_edge_list, XT_ORIENT_DEGREE, st, false, false));
+      XT_TRY(count_device_csr<int64_t>(ctx, s, nv, ne, d_indices, d_edge_list, XT_ORIENT_DEGREE, st, false, RankUse{false, -1}));
       uint64_t bad = 0;
       XT_HIP(ctx, hipMemcpyAsync(&bad, counters + kBadIds, sizeof(bad), hipMemcpyDeviceToHost, st));
       XT_HIP(ctx, hipStreamSynchronize(st));
@@ -673,8 +696,10 @@ int xt_graph_from_csr(xt_ctx* ctx, int64_t nv, int64_t ne, const int64_t* offset
     *out = nullptr;
     if (tails_bytes != 4 && tails_bytes != 8) return set_err(ctx, XT_ERR_ARG, "tails_bytes must be 4 or 8");
     if (ne > 0 && !tails) return set_err(ctx, XT_ERR_ARG, "null tails");
-    XT_TRY(check_host_offsets(ctx, nv, ne, offsets));
+    int64_t max_degree = -1;
+    XT_TRY(check_host_offsets(ctx, nv, ne, offsets, &max_degree));
     xt_graph* g = new xt_graph();
+    g->max_degree = (flags & XT_CLEAN) ? -1 : max_degree;  // cleaning adds reverse entries
     g->nv = nv;
     g->ne = ne;
     hipError_t e = hipMalloc(&g->off, (size_t)(nv + 1) * sizeof(int64_t));
@@ -932,7 +957,7 @@ int xt_graph_count(xt_ctx* ctx, xt_graph* g, uint32_t flags, uint64_t* total, ui
     XT_HIP(ctx, hipSetDevice(ctx->device));
     if (per_vertex && !(flags & XT_PER_VERTEX)) return set_err(ctx, XT_ERR_ARG, "per_vertex needs XT_PER_VERTEX");
     hipStream_t st = ctx->stream;
-    XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, g->nv, g->ne, g->off, g->tails, flags, st, true, true));
+    XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, g->nv, g->ne, g->off, g->tails, flags, st, true, RankUse{true, g->max_degree}));
     return finish_count(ctx, g->nv, flags, st, true, total, per_vertex);
   });
 }
@@ -949,11 +974,11 @@ int xt_graph_count_owned(xt_ctx* ctx, xt_graph* g, int64_t lo, int64_t hi, uint3
     // The owned-range count skips what cannot be owned, so the graph's total
     // takes a count of its own (run first: the timing kept is the owned count's).
     if (total) {
-      XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, g->nv, g->ne, g->off, g->tails, flags, st, true, true));
+      XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, g->nv, g->ne, g->off, g->tails, flags, st, true, RankUse{true, g->max_degree}));
       XT_TRY(finish_count(ctx, g->nv, flags, st, true, total, nullptr));
     }
     const OwnedRange range{lo, hi};
-    XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, g->nv, g->ne, g->off, g->tails, flags, st, true, false, &range));
+    XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, g->nv, g->ne, g->off, g->tails, flags, st, true, RankUse{false, -1}, &range));
     uint64_t h[kNumCounters];
     XT_TRY(finish_count(ctx, g->nv, flags, st, true, nullptr, nullptr, h));
     *owned = sum_of(h, kSumOwned);

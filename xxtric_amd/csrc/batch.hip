@@ -304,7 +304,7 @@ int batch_launch(xt_batch* b, int mode, uint32_t flags) {
     for (int64_t g = 0; g < G; g++) {
       const BatchGraph& r = b->graphs[g];
       XT_TRY(count_device_csr<int32_t>(ctx, b->s, r.nv, r.ne, b->loff + r.lobase, b->ltails + r.ebase,
-                                       flags & XT_ORIENT_ID, st, false, false));
+                                       flags & XT_ORIENT_ID, st, false, RankUse{false, -1}));
       hipLaunchKernelGGL(k_copy_total, dim3(1), dim3(64), 0, st,
                          (const uint64_t*)b->s.counters.as<uint64_t>(), b->ptotal + g);
       XT_HIP(ctx, hipGetLastError());

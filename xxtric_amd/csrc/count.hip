@@ -1874,7 +1874,7 @@ void carve(Scratch& s, unsigned char* base, int64_t nv, int64_t ne) {
 
 void release(Scratch& s) {
   DevBuf* bufs[] = {&s.deg, &s.dplus, &s.tailcnt, &s.qscan, &s.ooff, &s.otails, &s.counters,
-                    &s.oflags, &s.crows, &s.itcnt, &s.items, &s.tileoff, &s.tiledesc, &s.vrec, &s.pv, &s.rhist, &s.rank,
+                    &s.oflags, &s.crows, &s.itcnt, &s.items, &s.tileoff, &s.tiledesc, &s.vrec, &s.pv, &s.rhist, &s.rank, &s.rorig,
                     &s.ocount, &s.rpart, &s.rlists, &s.rrec, &s.scan_tmp, &s.in_off,
                     &s.in_tails};
   for (DevBuf* b : bufs) {

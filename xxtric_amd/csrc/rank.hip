@@ -44,6 +44,7 @@ constexpr uint32_t kHot = 65535;       // ranks below are hot; 65535 itself pads
 constexpr uint32_t kNoRank = ~0u;      // a self-loop or an id out of range; pads cold lists
 constexpr int kRankClasses = 896;      // degree classes: exact below 64, then 32 per octave
 constexpr int kRankMarks = 12;         // ids kept per list for finding prefixes
+constexpr int kRankMarksPv = 10;       // the same beside the vertex's label (per-vertex counts)
 constexpr int kAssignRun = 8;          // vertices per thread of k_rank_assign
 constexpr int kLaneList = 32;          // lists of up to this many ids are written by one lane, unsorted
 constexpr int kTinyRow = 8;            // rows of up to this many ids and 64 items: a lane per item
@@ -67,7 +68,12 @@ struct alignas(16) RankRec {
 };
 static_assert(sizeof(RankRec) == 32, "two 16-byte loads");
 
-__device__ __forceinline__ uint32_t mark_step(uint32_t hot) { return (hot + kRankMarks - 1) / kRankMarks; }
+// A per-vertex count keeps ten marks, and the vertex's label in the last word.
+template <bool PV>
+__device__ __forceinline__ uint32_t mark_step(uint32_t hot) {
+  constexpr uint32_t kMarks = PV ? kRankMarksPv : kRankMarks;
+  return (hot + kMarks - 1) / kMarks;
+}
 
 // 16-byte chunks a list of t chunks is given: it starts on a multiple of its size up
 // to eight chunks (a 128-byte line), so no list crosses more lines than it
@@ -82,7 +88,8 @@ __device__ __forceinline__ uint32_t list_room(uint32_t t) {
 // (crows[2c], crows[2c + 1]), each written by the row that holds the boundary.
 __global__ __launch_bounds__(256) void k_rank_prep(int64_t nv, int64_t ne, const int64_t* __restrict__ off, int64_t S,
                                                    int32_t* __restrict__ crows, uint64_t* __restrict__ oc,
-                                                   uint32_t* __restrict__ ic, uint32_t* __restrict__ hist) {
+                                                   uint32_t* __restrict__ ic, uint32_t* __restrict__ hist,
+                                                   unsigned long long* __restrict__ pv) {
   __shared__ uint32_t s_h[kRankClasses];
   for (int k = threadIdx.x; k < kRankClasses; k += 256) s_h[k] = 0;
   __syncthreads();
@@ -92,6 +99,7 @@ __global__ __launch_bounds__(256) void k_rank_prep(int64_t nv, int64_t ne, const
     const int64_t a = off[u], b = off[u + 1];
     oc[u] = 0;
     ic[u] = 0;
+    if (pv) pv[u] = 0;
     atomicAdd(&s_h[degree_class(b - a)], 1u);
     if (a < 0 || b > ne || a >= b) continue;
     for (int64_t c = (a + S - 1) / S; c * S < b; c++) crows[2 * c] = (int32_t)u;
@@ -108,7 +116,7 @@ __global__ __launch_bounds__(256) void k_rank_prep(int64_t nv, int64_t ne, const
 // inside a class is a valid total order).
 __global__ __launch_bounds__(256) void k_rank_assign(int64_t nv, const int64_t* __restrict__ off,
                                                      const uint32_t* __restrict__ hist, uint32_t* __restrict__ taken,
-                                                     uint32_t* __restrict__ rank) {
+                                                     uint32_t* __restrict__ rank, uint32_t* __restrict__ orig) {
   __shared__ uint32_t s_base[kRankClasses], s_n[kRankClasses];
   __shared__ int64_t s_scan[256 / kWave];
   constexpr int kPer = (kRankClasses + 255) / 256;
@@ -150,7 +158,22 @@ __global__ __launch_bounds__(256) void k_rank_assign(int64_t nv, const int64_t* 
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < kAssignRun; j++)
-    if (cls[j] >= 0) rank[u0 + 256 * j] = s_base[cls[j]] + loc[j];
+    if (cls[j] >= 0) {
+      const uint32_t r = s_base[cls[j]] + loc[j];
+      rank[u0 + 256 * j] = r;
+      if (orig) orig[r] = (uint32_t)(u0 + 256 * j);
+    }
+}
+
+// Ranks by descending label: u -> v iff u < v, the reference's rule.
+__global__ __launch_bounds__(256) void k_rank_by_label(int64_t nv, uint32_t* __restrict__ rank,
+                                                       uint32_t* __restrict__ orig) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; u < nv; u += stride) {
+    const uint32_t r = (uint32_t)(nv - 1 - u);
+    rank[u] = r;
+    if (orig) orig[u] = r;  // its own inverse
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -350,6 +373,7 @@ struct ListRoom {
   int64_t nbatch;
 };
 
+template <bool PV>
 __global__ __launch_bounds__(64) void k_rank_lists(int64_t nv, const int64_t* __restrict__ off,
                                                    const uint64_t* __restrict__ oc, const uint32_t* __restrict__ rank,
                                                    const uint32_t* __restrict__ part, ListRoom lr,
@@ -358,6 +382,7 @@ __global__ __launch_bounds__(64) void k_rank_lists(int64_t nv, const int64_t* __
   constexpr int kGroups = 8;  // pairs of 64-bit words per lane
   __shared__ ulonglong2 s_bits[kGroups * kWave];
   __shared__ uint16_t s_pre[kGroups * kWave];
+  constexpr uint32_t kMarks = PV ? kRankMarksPv : kRankMarks;
   __shared__ uint16_t s_mark[kRankMarks];
   const int lane = threadIdx.x;
   unsigned long long* bits = reinterpret_cast<unsigned long long*>(s_bits);
@@ -433,7 +458,8 @@ __global__ __launch_bounds__(64) void k_rank_lists(int64_t nv, const int64_t* __
     const bool alone = live && d <= kLaneList;
     if (alone && d < 2) {
       uint4* to = reinterpret_cast<uint4*>(rec + ru);
-      to[0] = to[1] = make_uint4(0, 0, 0, 0);
+      to[0] = make_uint4(0, 0, 0, 0);
+      to[1] = make_uint4(0, 0, 0, PV ? (uint32_t)u : 0u);
     }
     if (__builtin_amdgcn_ballot_w64(alone && d >= 2)) {  // uniform
       uint64_t lo = ~0ull, hi = ~0ull;
@@ -467,11 +493,12 @@ __global__ __launch_bounds__(64) void k_rank_lists(int64_t nv, const int64_t* __
         const uint32_t m = least | (least << 16);  // not sorted: all of it or nothing is below v
         uint4* to = reinterpret_cast<uint4*>(rec + ru);
         to[0] = make_uint4(start, hc | (cc << 16), m, m);
-        to[1] = make_uint4(~0u, ~0u, ~0u, ~0u);
+        to[1] = make_uint4(~0u, ~0u, ~0u, PV ? (uint32_t)u : ~0u);
       }
     }
     uint64_t todo = __builtin_amdgcn_ballot_w64(live && d > kLaneList);
-    uint32_t ra = 0, rd = 0, rs = 0, rr = 0, rw = kNoRank;  // the next row: first entry, ids, list, rank; its first ids
+    // The next row: first entry, ids, list, rank, label; its first ids.
+    uint32_t ra = 0, rd = 0, rs = 0, rr = 0, ro = 0, rw = kNoRank;
     auto pop = [&]() {
       const int src = __builtin_ctzll(todo);
       todo &= todo - 1;
@@ -479,12 +506,13 @@ __global__ __launch_bounds__(64) void k_rank_lists(int64_t nv, const int64_t* __
       rd = __builtin_amdgcn_readlane(d, src);
       rs = __builtin_amdgcn_readlane(start, src);
       rr = __builtin_amdgcn_readlane(ru, src);
+      if constexpr (PV) ro = __builtin_amdgcn_readlane((uint32_t)u, src);
       rw = part[ra + lane];  // more than 32 ids and, in a simple graph, as many behind; the array is padded
     };
     bool more = todo != 0;
     if (more) pop();
     while (more) {  // uniform
-      const uint32_t dd = rd, st = rs, rk = rr, w0 = (uint32_t)lane < rd ? rw : kNoRank;
+      const uint32_t dd = rd, st = rs, rk = rr, label = ro, w0 = (uint32_t)lane < rd ? rw : kNoRank;
       const uint32_t* ids = part + ra;
       more = todo != 0;
       if (more) pop();  // the next row's ids fly while this one is written
@@ -518,7 +546,7 @@ __global__ __launch_bounds__(64) void k_rank_lists(int64_t nv, const int64_t* __
       }
       wave_lds_fence();
       const uint32_t hcc = min((hh + 7) >> 3, 8192u), ccc = min((dd - hh + 3) >> 2, 65535u);
-      const uint32_t seg = 8 * max(mark_step(hcc), 1u);               // ids per segment
+      const uint32_t seg = 8 * max(mark_step<PV>(hcc), 1u);               // ids per segment
       const uint32_t inv = (uint32_t)(((1ull << 32) + seg - 1) / seg);  // r / seg for r < 2^16
       uint16_t* hl = reinterpret_cast<uint16_t*>(lists + st);
       uint32_t* cl = reinterpret_cast<uint32_t*>(lists + st + hcc);
@@ -536,7 +564,7 @@ __global__ __launch_bounds__(64) void k_rank_lists(int64_t nv, const int64_t* __
           }
           if (r < 8 * hcc) hl[r] = (uint16_t)w;
           const uint32_t k = __umulhi(r, inv);
-          if (k * seg == r && k < kRankMarks) s_mark[k] = (uint16_t)w;
+          if (k * seg == r && k < kMarks) s_mark[k] = (uint16_t)w;
         } else if (cold) {
           const uint32_t r = ncold + lanes_below(cm);
           if (r < 4 * ccc) cl[r] = w;
@@ -553,7 +581,8 @@ __global__ __launch_bounds__(64) void k_rank_lists(int64_t nv, const int64_t* __
       if ((uint32_t)lane < 4 * ccc - min(dd - hh, 4 * ccc)) cl[dd - hh + lane] = kNoRank;
       if (lane < 8) {
         const uint32_t m = lane >= 2 ? (uint32_t)s_mark[2 * lane - 4] | ((uint32_t)s_mark[2 * lane - 3] << 16) : 0u;
-        reinterpret_cast<uint32_t*>(rec + rk)[lane] = lane == 0 ? st : lane == 1 ? hcc | (ccc << 16) : m;
+        reinterpret_cast<uint32_t*>(rec + rk)[lane] =
+            lane == 0 ? st : lane == 1 ? hcc | (ccc << 16) : PV && lane == 7 ? label : m;
       }
       wave_lds_fence();
     }
@@ -576,9 +605,23 @@ __global__ __launch_bounds__(64) void k_rank_lists(int64_t nv, const int64_t* __
 // 64 b + 64, so a step needs two readlanes and a masked bit count.
 constexpr int kStreamBlocks = kWave;  // 64-chunk blocks that the bits cover
 
-template <typename F>
-__device__ __forceinline__ void stream_lists(uint32_t start, uint32_t n, uint32_t* s_adj, unsigned long long* s_bit,
-                                             int lane, const uint4* __restrict__ lists, uint32_t pad, F&& probe) {
+// LDS of one wave's streaming.
+struct StreamLds {
+  unsigned long long bit[kStreamBlocks];
+  uint32_t adj[kWave];  // per item with chunks: its list's start less its first chunk
+};
+// Per-vertex counts, per item: u's label and the hits credited to u.
+struct ItemLds {
+  uint32_t label[kWave];
+  uint32_t hits[kWave];
+};
+
+// probe(chunk, item): item is the chunk's index among the items with chunks.
+// PV: `label` is u's label; the hits that probe adds to items are added to pv.
+template <bool PV, typename F>
+__device__ __forceinline__ void stream_lists(uint32_t start, uint32_t n, uint32_t label, StreamLds& s, ItemLds* s_items,
+                                             int lane, const uint4* __restrict__ lists, uint32_t pad,
+                                             unsigned long long* __restrict__ pv, F&& probe) {
   const uint32_t inc = wave_incl_scan_u32(n);
   const uint32_t all = __builtin_amdgcn_readlane(inc, kWave - 1);
   if (all == 0) return;  // uniform
@@ -588,48 +631,63 @@ __device__ __forceinline__ void stream_lists(uint32_t start, uint32_t n, uint32_
     return v;
   };
   const uint64_t some = __builtin_amdgcn_ballot_w64(n > 0);
+  if constexpr (PV) {
+    wave_lds_fence();
+    if (n > 0) s_items->label[lanes_below(some)] = label;
+    s_items->hits[lane] = 0;
+    wave_lds_fence();
+  }
   if (all <= kStreamBlocks * kWave) {
     const uint32_t p = inc - n;
     wave_lds_fence();
-    s_bit[lane] = 0ull;
-    if (n > 0) s_adj[lanes_below(some)] = start - p;
+    s.bit[lane] = 0ull;
+    if (n > 0) s.adj[lanes_below(some)] = start - p;
     wave_lds_fence();
-    if (n > 0 && p > 0) atomicOr(&s_bit[(p - 1) >> 6], 1ull << ((p - 1) & 63));
+    if (n > 0 && p > 0) atomicOr(&s.bit[(p - 1) >> 6], 1ull << ((p - 1) & 63));
     wave_lds_fence();
-    const int64_t my = (int64_t)s_bit[lane];
+    const int64_t my = (int64_t)s.bit[lane];
     const int steps = (int)((all + kWave - 1) / kWave);
     uint32_t before = 0;
-    auto next = [&](int b) -> uint4 {
+    auto next = [&](int b, uint32_t& item) -> uint4 {
       const uint64_t m = (uint64_t)readlane64(my, b);
       const uint32_t c = (uint32_t)b * kWave + lane;
-      const uint32_t at = s_adj[before + lanes_below(m)] + c;
+      item = before + lanes_below(m);
+      const uint32_t at = s.adj[item] + c;
       before += (uint32_t)__popcll(m);
       return load(at, c < all);
     };
     // Two buffers by hand: the next step's loads are in flight while one is probed.
-    uint4 va = next(0), vb;
+    uint32_t ia = 0, ib = 0;
+    uint4 va = next(0, ia), vb;
     for (int b = 1;; b += 2) {
-      if (b < steps) vb = next(b);
-      probe(va);
+      if (b < steps) vb = next(b, ib);
+      probe(va, ia);
       if (b >= steps) break;
-      if (b + 1 < steps) va = next(b + 1);
-      probe(vb);
+      if (b + 1 < steps) va = next(b + 1, ia);
+      probe(vb, ib);
       if (b + 1 >= steps) break;
     }
   } else {  // long lists: the whole wave on one item at a time
-    for (uint64_t left = some; left; left &= left - 1) {
+    uint32_t item = 0;
+    for (uint64_t left = some; left; left &= left - 1, item++) {
       const int k = __builtin_ctzll(left);
       const uint32_t s0 = __builtin_amdgcn_readlane(start, k), nk = __builtin_amdgcn_readlane(n, k);
       uint4 va = load(s0 + lane, (uint32_t)lane < nk), vb;
       for (uint32_t c = kWave;; c += 2 * kWave) {
         if (c < nk) vb = load(s0 + c + lane, c + lane < nk);
-        probe(va);
+        probe(va, item);
         if (c >= nk) break;
         if (c + kWave < nk) va = load(s0 + c + kWave + lane, c + kWave + lane < nk);
-        probe(vb);
+        probe(vb, item);
         if (c + kWave >= nk) break;
       }
     }
+  }
+  if constexpr (PV) {
+    wave_lds_fence();
+    const uint32_t t = s_items->hits[lane];
+    if (t) atomicAdd(&pv[s_items->label[lane]], (unsigned long long)t);
+    wave_lds_fence();
   }
 }
 
@@ -644,16 +702,36 @@ struct Head {  // a record
   uint4 a, b;
 };
 
+// PV: every triangle is credited to its smallest label (xxtric.hpp:165).  A hit
+// w of the item u in v's map: with its place p among N(v)'s hot ids (count
+// before its word plus the bits below it) s_label[p] is w's label; if it is the
+// smallest, slot p counts it (added to pv when the row ends), otherwise u's item
+// counter or v's register does.  Places from kSlots on, cold hits and the rows of
+// few ids look labels up and add to pv directly.
+constexpr int kSlots = 512;
+struct PvLds {
+  uint16_t pre[1024];  // hot ids of N(v) before each 64-bit word of the map
+  uint32_t label[kSlots];
+  uint32_t hits[kSlots];
+  ItemLds items;
+};
+struct NoLds {};
+
+template <bool PV>
 __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const int64_t* __restrict__ off,
                                                    const uint32_t* __restrict__ rank, const uint64_t* __restrict__ oc,
                                                    const uint32_t* __restrict__ part, const RankRec* __restrict__ rec,
                                                    const uint4* __restrict__ lists, const int32_t* __restrict__ crows,
-                                                   int64_t S, uint64_t* __restrict__ counters) {
+                                                   int64_t S, uint64_t* __restrict__ counters,
+                                                   const uint32_t* __restrict__ orig,
+                                                   unsigned long long* __restrict__ pv) {
   constexpr int kWords = 2048;
   constexpr int kColdSmall = 6, kColdBig = 9;  // hash buckets (log2) for up to 128 and up to 1024 cold ids
   __shared__ uint4 s_mem[kWords / 4];
-  __shared__ unsigned long long s_bit[kStreamBlocks];
-  __shared__ uint32_t s_adj[kWave];
+  __shared__ StreamLds s_stream;
+  __shared__ typename std::conditional<PV, PvLds, NoLds>::type s_pv;
+  ItemLds* s_items = nullptr;
+  if constexpr (PV) s_items = &s_pv.items;
   uint32_t* s_bm = reinterpret_cast<uint32_t*>(s_mem);
   int4* s_tab = reinterpret_cast<int4*>(s_mem);
   const int lane = threadIdx.x;
@@ -666,29 +744,32 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
     for (int i = lane; i < quads; i += kWave) s_mem[i] = make_uint4(0, 0, 0, 0);
   };
   clear_words(kWords / 4);
+  if constexpr (PV)
+    for (int i = lane; i < kSlots; i += kWave) s_pv.hits[i] = 0;
   wave_lds_fence();
-  auto tiny_rows = [&](bool tiny, uint32_t a0, uint32_t is, uint32_t items, uint32_t d) -> uint32_t {
+  auto tiny_rows = [&](bool tiny, uint32_t a0, uint32_t is, uint32_t items, uint32_t d, uint32_t row0) -> uint32_t {
     const uint32_t n = tiny ? items : 0;
     const uint32_t inc = wave_incl_scan_u32(n), p = inc - n;
     const uint32_t all = __builtin_amdgcn_readlane(inc, kWave - 1);
     const uint64_t some = __builtin_amdgcn_ballot_w64(n > 0);
     wave_lds_fence();
-    s_bit[lane] = 0ull;
-    if (n > 0) s_adj[lanes_below(some)] = (uint32_t)lane;
+    s_stream.bit[lane] = 0ull;
+    if (n > 0) s_stream.adj[lanes_below(some)] = (uint32_t)lane;
     wave_lds_fence();
-    if (n > 0 && p > 0) atomicOr(&s_bit[(p - 1) >> 6], 1ull << ((p - 1) & 63));
+    if (n > 0 && p > 0) atomicOr(&s_stream.bit[(p - 1) >> 6], 1ull << ((p - 1) & 63));
     wave_lds_fence();
-    const int64_t my = (int64_t)s_bit[lane];
+    const int64_t my = (int64_t)s_stream.bit[lane];
     uint32_t before = 0, acc = 0;
     for (uint32_t b = 0; b * kWave < all; b++) {
       const uint64_t m = (uint64_t)readlane64(my, (int)b);
       const uint32_t c = b * kWave + lane;
-      const int row = (int)s_adj[before + lanes_below(m)];
+      const int row = (int)s_stream.adj[before + lanes_below(m)];
       before += (uint32_t)__popcll(m);
       const uint32_t entry = (uint32_t)__shfl((int)(is - p), row, kWave) + c;
       const uint32_t first = (uint32_t)__shfl((int)a0, row, kWave), nd = (uint32_t)__shfl((int)d, row, kWave);
       uint32_t x[kTinyRow];
       uint2 r = make_uint2(0, 0);
+      uint32_t two = 0;  // PV: the smaller of u's and v's label
 #pragma unroll
       for (int i = 0; i < kTinyRow; i++) x[i] = kNoRank - 1;  // matches no id and no padding
       if (c < all) {
@@ -697,29 +778,62 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
         for (int i = 0; i < kTinyRow; i++)
           if ((uint32_t)i < nd) x[i] = part[first + i];
         if (ur != kNoRank) r = *reinterpret_cast<const uint2*>(rec + ur);
+        if constexpr (PV)
+          if (ur != kNoRank) two = min(rec[ur].mark[5], row0 + (uint32_t)row);
       }
+      // PV: the ids w of a chunk that N(v) holds (bit j: id j), one credit each.
+      auto credit = [&](uint32_t found, auto&& w) {
+        acc += (uint32_t)__popc(found);
+        while (found) {
+          const int j = __builtin_ctz(found);
+          found &= found - 1;
+          atomicAdd(&pv[min(two, orig[w(j)])], 1ull);
+        }
+      };
       const uint32_t hc = r.y & 0xffffu, cc = r.y >> 16;
       for (uint32_t k = 0; __builtin_amdgcn_ballot_w64(k < hc); k++) {
         if (k < hc) {
           const uint4 q = lists[r.x + k];
           const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+          uint32_t found = 0;
 #pragma unroll
           for (int j = 0; j < 4; j++) {
             const uint32_t lo = w[j] & 0xffffu, hi = w[j] >> 16;
             const uint32_t lo2 = lo < kHot ? lo : kNoRank, hi2 = hi < kHot ? hi : kNoRank;
+            bool in_lo = false, in_hi = false;
 #pragma unroll
-            for (int i = 0; i < kTinyRow; i++) acc += (x[i] == lo2 ? 1u : 0u) + (x[i] == hi2 ? 1u : 0u);
+            for (int i = 0; i < kTinyRow; i++) {
+              if constexpr (PV) {
+                in_lo |= x[i] == lo2;
+                in_hi |= x[i] == hi2;
+              } else {
+                acc += (x[i] == lo2 ? 1u : 0u) + (x[i] == hi2 ? 1u : 0u);
+              }
+            }
+            found |= (in_lo ? 1u : 0u) << (2 * j) | (in_hi ? 1u : 0u) << (2 * j + 1);
           }
+          if constexpr (PV)
+            credit(found, [&](int j) { return ((j & 4) ? (j & 2 ? w[3] : w[2]) : (j & 2 ? w[1] : w[0])) >> (16 * (j & 1)) & 0xffffu; });
         }
       }
       for (uint32_t k = 0; __builtin_amdgcn_ballot_w64(k < cc); k++) {
         if (k < cc) {
           const uint4 q = lists[r.x + hc + k];
           const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+          uint32_t found = 0;
 #pragma unroll
-          for (int j = 0; j < 4; j++)
+          for (int j = 0; j < 4; j++) {
+            bool in = false;
 #pragma unroll
-            for (int i = 0; i < kTinyRow; i++) acc += x[i] == w[j] ? 1u : 0u;
+            for (int i = 0; i < kTinyRow; i++) {
+              if constexpr (PV)
+                in |= x[i] == w[j];
+              else
+                acc += x[i] == w[j] ? 1u : 0u;
+            }
+            found |= (in ? 1u : 0u) << j;
+          }
+          if constexpr (PV) credit(found, [&](int j) { return (j & 2) ? (j & 1 ? w[3] : w[2]) : (j & 1 ? w[1] : w[0]); });
         }
       }
     }
@@ -743,11 +857,12 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
     // Rows of few ids and few items: their items are taken together, one lane
     // per item, every id of N(v) compared with every id of u's list.
     const bool tiny = work && d <= kTinyRow && ie - is <= kWave;
-    if (__builtin_amdgcn_ballot_w64(tiny)) hits += tiny_rows(tiny, (uint32_t)a0, (uint32_t)is, (uint32_t)(ie - is), d);
+    if (__builtin_amdgcn_ballot_w64(tiny)) 
+      hits += tiny_rows(tiny, (uint32_t)a0, (uint32_t)is, (uint32_t)(ie - is), d, (uint32_t)rb);
     uint64_t todo = __builtin_amdgcn_ballot_w64(work && !tiny);
     // Row by row; the next row's ids and items are loaded before the current
     // row's map is built, its items' records before the current lists stream.
-    uint32_t b0 = 0, s0 = 0, s1 = 0, dd = 0, hh = 0, vv = 0;
+    uint32_t b0 = 0, s0 = 0, s1 = 0, dd = 0, hh = 0, vv = 0, vo = 0;
     auto pop = [&]() {
       const int src = __builtin_ctzll(todo);
       todo &= todo - 1;
@@ -757,6 +872,7 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
       dd = __builtin_amdgcn_readlane(d, src);
       hh = __builtin_amdgcn_readlane(h, src);
       vv = __builtin_amdgcn_readlane(v, src);
+      vo = (uint32_t)rb + (uint32_t)src;
     };
     auto item = [&](uint32_t e) -> uint32_t { return e + lane < s1 ? part[e + lane] : kNoRank; };
     auto head = [&](uint32_t ur) -> Head {
@@ -773,7 +889,7 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
     uint32_t w0 = (uint32_t)lane < dd ? part[b0 + lane] : kNoRank;
     Head x = head(item(s0));
     for (;;) {  // uniform
-      const uint32_t cb = b0, cs0 = s0, cs1 = s1, cd = dd, ch = hh, cv = vv, w = w0;
+      const uint32_t cb = b0, cs0 = s0, cs1 = s1, cd = dd, ch = hh, cv = vv, cl = vo, w = w0;
       const bool more = todo != 0;
       uint32_t un = kNoRank;
       if (more) {
@@ -788,38 +904,109 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
         const uint32_t mk[kRankMarks / 2] = {h.a.z, h.a.w, h.b.x, h.b.y, h.b.z, h.b.w};
         uint32_t segs = 0;  // segments that start below v
 #pragma unroll
-        for (int t = 0; t < kRankMarks / 2; t++) segs += ((mk[t] & 0xffffu) < cv ? 1u : 0u) + ((mk[t] >> 16) < cv ? 1u : 0u);
-        return min(segs * mark_step(hot), hot);
+        for (int t = 0; t < (PV ? kRankMarksPv : kRankMarks) / 2; t++) segs += ((mk[t] & 0xffffu) < cv ? 1u : 0u) + ((mk[t] >> 16) < cv ? 1u : 0u);
+        return min(segs * mark_step<PV>(hot), hot);
       };
       const bool cold = ch < cd && cv > kHot;  // cold ids below a cold v
-      const uint32_t st = x.a.x, len = x.a.y, n = prefix(x);  // the first 64 items
+      const uint32_t st = x.a.x, len = x.a.y, label = x.b.w, n = prefix(x);  // the first 64 items
+      uint32_t at_v = 0;  // PV: hits credited to v
       if (ch > 0)
         for (uint32_t i = 0; i < cd; i += kWave) {
           const uint32_t y = id(i);
           if (y < kHot) atomicOr(&s_bm[y >> 5], 1u << (y & 31));
         }
+      unsigned long long* s_map = reinterpret_cast<unsigned long long*>(s_mem);
+      auto place = [&](uint32_t y) -> uint32_t {  // of hot id y of N(v)
+        if constexpr (PV)
+          return s_pv.pre[y >> 6] + (uint32_t)__popcll(s_map[y >> 6] & ((1ull << (y & 63)) - 1ull));
+        else
+          return 0;
+      };
+      if constexpr (PV) {
+        if (ch > 0) {
+          wave_lds_fence();
+          if (cd <= kWave) {  // counts at the words in use, by comparing the ids
+            uint32_t less = 0;
+            for (uint64_t m = __builtin_amdgcn_ballot_w64(w < kHot); m; m &= m - 1)
+              less += ((uint32_t)__builtin_amdgcn_readlane((int)w, __builtin_ctzll(m)) >> 6) < (w >> 6) ? 1u : 0u;
+            if (w < kHot) s_pv.pre[w >> 6] = (uint16_t)less;
+          } else {
+            uint32_t base = 0;
+            for (int g = 0; g < 1024 / kWave && base < ch; g++) {
+              const uint32_t t = (uint32_t)__popcll(s_map[g * kWave + lane]);
+              const uint32_t upto = wave_incl_scan_u32(t);
+              s_pv.pre[g * kWave + lane] = (uint16_t)(base + upto - t);
+              base += __builtin_amdgcn_readlane(upto, kWave - 1);
+            }
+          }
+          wave_lds_fence();
+          for (uint32_t i = 0; i < cd; i += kWave) {
+            const uint32_t y = id(i);
+            if (y < kHot) {
+              const uint32_t p = place(y);
+              if (p < kSlots) s_pv.label[p] = orig[y];
+            }
+          }
+          wave_lds_fence();
+        }
+      }
       if (more) x = head(un);
       auto items = [&](uint32_t e) -> uint32_t { return e + lane < cs1 ? part[e + lane] : kNoRank; };
       if (ch > 0) {
         uint32_t acc = 0;
-        auto probe = [&](const uint4 q) {
+        auto probe = [&](const uint4 q, uint32_t item) {
           const uint32_t y[4] = {q.x, q.y, q.z, q.w};
+          uint32_t found = 0;
 #pragma unroll
           for (int j = 0; j < 4; j++) {
             const uint32_t lo = s_bm[(y[j] >> 5) & 2047u], hi = s_bm[y[j] >> 21];
-            acc += (lo >> (y[j] & 31)) & 1u;
-            acc += (hi >> ((y[j] >> 16) & 31)) & 1u;
+            const uint32_t t0 = (lo >> (y[j] & 31)) & 1u, t1 = (hi >> ((y[j] >> 16) & 31)) & 1u;
+            if constexpr (PV)
+              found |= t0 << (2 * j) | t1 << (2 * j + 1);
+            else
+              acc += t0 + t1;
+          }
+          if constexpr (PV) {
+            acc += (uint32_t)__popc(found);
+            const uint32_t lu = found ? s_pv.items.label[item] : 0;
+            const uint32_t two = min(lu, cl);
+            uint32_t rest = 0;  // hits credited to u or v
+            while (found) {
+              const int j = __builtin_ctz(found);
+              found &= found - 1;
+              const uint32_t z = ((j & 4) ? (j & 2 ? y[3] : y[2]) : (j & 2 ? y[1] : y[0])) >> (16 * (j & 1)) & 0xffffu;
+              const uint32_t p = place(z);
+              const uint32_t lw = p < kSlots ? s_pv.label[p] : orig[z];
+              if (lw > two)
+                rest++;
+              else if (p < kSlots)
+                atomicAdd(&s_pv.hits[p], 1u);
+              else
+                atomicAdd(&pv[lw], 1ull);
+            }
+            if (cl < lu)
+              at_v += rest;
+            else if (rest)
+              atomicAdd(&s_pv.items.hits[item], rest);
           }
         };
         Head y = cs0 + kWave < cs1 ? head(items(cs0 + kWave)) : Head{};
-        stream_lists(st, n, s_adj, s_bit, lane, lists, 0xffffffffu, probe);
+        stream_lists<PV>(st, n, label, s_stream, s_items, lane, lists, 0xffffffffu, pv, probe);
         for (uint32_t e = cs0 + kWave; e < cs1; e += kWave) {
-          const uint32_t sty = y.a.x, ny = prefix(y);
+          const uint32_t sty = y.a.x, ny = prefix(y), ly = y.b.w;
           if (e + kWave < cs1) y = head(items(e + kWave));
-          stream_lists(sty, ny, s_adj, s_bit, lane, lists, 0xffffffffu, probe);
+          stream_lists<PV>(sty, ny, ly, s_stream, s_items, lane, lists, 0xffffffffu, pv, probe);
         }
         hits += acc;
         wave_lds_fence();
+        if constexpr (PV)
+          for (uint32_t p = lane; p < min(ch, (uint32_t)kSlots); p += kWave) {
+            const uint32_t t = s_pv.hits[p];
+            if (t) {
+              atomicAdd(&pv[s_pv.label[p]], (unsigned long long)t);
+              s_pv.hits[p] = 0;
+            }
+          }
         if (cd <= 8 * kWave) {
           for (uint32_t i = 0; i < cd; i += kWave) {
             const uint32_t y = id(i);
@@ -848,7 +1035,7 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
           }
           const bool spl = __builtin_amdgcn_ballot_w64(passed) != 0;
           wave_lds_fence();
-          auto probe = [&](const uint4 q) {
+          auto probe = [&](const uint4 q, uint32_t item) {
             const int32_t y[4] = {(int32_t)q.x, (int32_t)q.y, (int32_t)q.z, (int32_t)q.w};
             int4 t[4];
 #pragma unroll
@@ -859,14 +1046,29 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
               if (spl && !hit && bucket_spilled(t[j]) && y[j] != -1)
                 hit = wave_tab_continue<L>(s_tab, wave_bucket<L>(y[j]), y[j]);
               acc += hit ? 1u : 0u;
+              if constexpr (PV) {
+                if (hit) {
+                  const uint32_t lu = s_pv.items.label[item], lw = orig[y[j]];
+                  if (lw < min(lu, cl))
+                    atomicAdd(&pv[lw], 1ull);
+                  else if (cl < lu)
+                    at_v++;
+                  else
+                    atomicAdd(&s_pv.items.hits[item], 1u);
+                }
+              }
             }
           };
-          stream_lists(st + (len & 0xffffu), len >> 16, s_adj, s_bit, lane, lists, kNoRank, probe);
+          stream_lists<PV>(st + (len & 0xffffu), len >> 16, label, s_stream, s_items, lane, lists, kNoRank, pv, probe);
           for (uint32_t e = cs0 + kWave; e < cs1; e += kWave) {
             const uint32_t ur = items(e);
             uint2 y = make_uint2(0, 0);
-            if (ur != kNoRank) y = *reinterpret_cast<const uint2*>(rec + ur);
-            stream_lists(y.x + (y.y & 0xffffu), y.y >> 16, s_adj, s_bit, lane, lists, kNoRank, probe);
+            uint32_t ly = 0;
+            if (ur != kNoRank) {
+              y = *reinterpret_cast<const uint2*>(rec + ur);
+              if constexpr (PV) ly = rec[ur].mark[5];
+            }
+            stream_lists<PV>(y.x + (y.y & 0xffffu), y.y >> 16, ly, s_stream, s_items, lane, lists, kNoRank, pv, probe);
           }
           wave_lds_fence();
           clear_words(1 << L);
@@ -879,6 +1081,10 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
           for (uint32_t f = 0; f < ncold; f += 2u << kColdBig) pass(std::integral_constant<int, kColdBig>{}, f, 2u << kColdBig);
         }
         hits += acc;
+      }
+      if constexpr (PV) {
+        const uint64_t t = wave_sum_u64(at_v);
+        if (lane == 0 && t) atomicAdd(&pv[cl], (unsigned long long)t);
       }
       if (!more) break;
     }
@@ -901,7 +1107,7 @@ static unsigned rank_grid(int64_t n, int per, int64_t cap) {
 // A region is left for the next when a request does not fit, so each may lose
 // one request: a grant, or 64 of the longest lists (at most 1.02 sqrt(ne) ids,
 // since out-neighbours have about the vertex's degree or more).
-static ListRoom rank_list_room(const xt_ctx* ctx, int64_t nv, int64_t ne, int64_t* lines) {
+static ListRoom rank_list_room(const xt_ctx* ctx, int64_t nv, int64_t ne, bool by_label, int64_t* lines) {
   ListRoom r;
   const int64_t waves = (int64_t)ctx->num_cus * 16;
   r.rows = kWave;
@@ -915,7 +1121,7 @@ static ListRoom rank_list_room(const xt_ctx* ctx, int64_t nv, int64_t ne, int64_
   const int64_t need = chunks / 8 + r.nbatch + 1;
   const int64_t grant = need / (waves * 32) < 8 ? 8 : need / (waves * 32);
   const int64_t used = need + need / 3 + (r.nbatch < waves ? r.nbatch : waves) * grant;
-  const double longest = 1.05 * std::sqrt((double)ne) + 64.0;
+  const double longest = by_label ? (double)nv : 1.05 * std::sqrt((double)ne) + 64.0;
   const int64_t most = grant + (int64_t)(64.0 * (longest / 4 + 10) / 8) + 1;
   r.grant = (uint64_t)grant;
   r.region = (uint64_t)(used / kListShards + most + 1);
@@ -923,11 +1129,16 @@ static ListRoom rank_list_room(const xt_ctx* ctx, int64_t nv, int64_t ne, int64_
   return r;
 }
 
+// Ranked by label a list may hold every vertex: a record's 16 bits of cold
+// chunks hold the lists of this many vertices.
+constexpr int64_t kLabelRankMax = 4 * 65535;
+
 // Ranks, chunk starts of lists and entry indices fit their 32 bits.
-bool rank_fits(const xt_ctx* ctx, int64_t nv, int64_t ne) {
-  if (nv >= (1ll << 30) || ne >= (1ll << 32)) return false;
+bool rank_fits(const xt_ctx* ctx, int64_t nv, int64_t ne, int mode) {
+  const bool by_label = mode == kOrientId;
+  if (nv >= (by_label ? kLabelRankMax : 1ll << 30) || ne >= (1ll << 32)) return false;
   int64_t lines;
-  rank_list_room(ctx, nv, ne, &lines);
+  rank_list_room(ctx, nv, ne, by_label, &lines);
   return lines < (1ll << 29);
 }
 
@@ -939,8 +1150,8 @@ static int64_t rank_chunk(const xt_ctx* ctx, int64_t ne) {
 }
 
 template <typename T>
-int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* off, const T* tails, hipStream_t st,
-               hipEvent_t split_done) {
+int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* off, const T* tails, int mode,
+               uint64_t* pv, hipStream_t st, hipEvent_t split_done) {
   const int64_t S = rank_chunk(ctx, ne);
   const int64_t nch = (ne + S - 1) / S, nchunks = (ne + kChunk - 1) / kChunk;
   XT_TRY(ensure(ctx, s.crows, (size_t)(2 * nch) * sizeof(int32_t)));
@@ -949,10 +1160,13 @@ int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* o
   XT_TRY(ensure(ctx, s.itcnt, (size_t)nv * sizeof(uint32_t)));
   XT_TRY(ensure(ctx, s.rpart, (size_t)(ne + kWave) * sizeof(uint32_t)));  // a wave reads past a short row
   int64_t lines;
-  const ListRoom lr = rank_list_room(ctx, nv, ne, &lines);
+  const ListRoom lr = rank_list_room(ctx, nv, ne, mode == kOrientId, &lines);
   XT_TRY(ensure(ctx, s.rlists, (size_t)lines * 128));
   XT_TRY(ensure(ctx, s.rrec, (size_t)nv * sizeof(RankRec)));
   XT_TRY(ensure(ctx, s.rhist, (size_t)(2 * kRankClasses) * sizeof(uint32_t)));
+  if (pv) XT_TRY(ensure(ctx, s.rorig, (size_t)nv * sizeof(uint32_t)));
+  uint32_t* orig = pv ? s.rorig.as<uint32_t>() : nullptr;
+  unsigned long long* pvp = reinterpret_cast<unsigned long long*>(pv);
   uint64_t* counters = s.counters.as<uint64_t>();
   uint32_t* hist = s.rhist.as<uint32_t>();
   int32_t* crows = s.crows.as<int32_t>();
@@ -963,29 +1177,46 @@ int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* o
   RankRec* rec = s.rrec.as<RankRec>();
   XT_TRY(fill_u32(ctx, hist, 2 * kRankClasses, 0u, st));
   hipLaunchKernelGGL(k_rank_prep, dim3(rank_grid(nv, 1024, 8192)), dim3(256), 0, st, nv, ne, off, S, crows, oc,
-                     s.itcnt.as<uint32_t>(), hist);
+                     s.itcnt.as<uint32_t>(), hist, pvp);
   XT_HIP(ctx, hipGetLastError());
-  hipLaunchKernelGGL(k_rank_assign, dim3(rank_grid(nv, 256 * kAssignRun, 1ll << 31)), dim3(256), 0, st, nv, off,
-                     (const uint32_t*)hist, hist + kRankClasses, rank);
+  if (mode == kOrientId)
+    hipLaunchKernelGGL(k_rank_by_label, dim3(rank_grid(nv, 256, 8192)), dim3(256), 0, st, nv, rank, orig);
+  else
+    hipLaunchKernelGGL(k_rank_assign, dim3(rank_grid(nv, 256 * kAssignRun, 1ll << 31)), dim3(256), 0, st, nv, off,
+                       (const uint32_t*)hist, hist + kRankClasses, rank, orig);
   XT_HIP(ctx, hipGetLastError());
   hipLaunchKernelGGL((k_rank_split<T>), dim3(xcd_grid(nchunks)), dim3(kBlock), 0, st, nv, ne, off, tails,
                      (const uint32_t*)rank, (const int32_t*)crows, (int)(kChunk / S), part, oc,
                      s.itcnt.as<uint32_t>(), counters);
   XT_HIP(ctx, hipGetLastError());
-  hipLaunchKernelGGL(k_rank_lists, dim3(rank_grid(lr.nbatch, 1, (int64_t)ctx->num_cus * 16)), dim3(64), 0, st, nv, off,
-                     (const uint64_t*)oc, (const uint32_t*)rank, (const uint32_t*)part, lr, lists, rec, counters);
+  const dim3 lgrid(rank_grid(lr.nbatch, 1, (int64_t)ctx->num_cus * 16));
+#define XT_RANK_LISTS(PV)                                                                                           \
+  hipLaunchKernelGGL((k_rank_lists<PV>), lgrid, dim3(64), 0, st, nv, off, (const uint64_t*)oc, (const uint32_t*)rank, \
+                     (const uint32_t*)part, lr, lists, rec, counters)
+  if (pv)
+    XT_RANK_LISTS(true);
+  else
+    XT_RANK_LISTS(false);
+#undef XT_RANK_LISTS
   XT_HIP(ctx, hipGetLastError());
   if (split_done) XT_HIP(ctx, hipEventRecord(split_done, st));
-  hipLaunchKernelGGL(k_rank_count, dim3((unsigned)nch), dim3(64), 0, st, nv, ne, off, (const uint32_t*)rank,
-                     (const uint64_t*)oc, (const uint32_t*)part, (const RankRec*)rec, (const uint4*)lists,
-                     (const int32_t*)crows, S, counters);
+#define XT_RANK_COUNT(PV)                                                                                            \
+  hipLaunchKernelGGL((k_rank_count<PV>), dim3((unsigned)nch), dim3(64), 0, st, nv, ne, off, (const uint32_t*)rank,     \
+                     (const uint64_t*)oc, (const uint32_t*)part, (const RankRec*)rec, (const uint4*)lists,            \
+                     (const int32_t*)crows, S, counters, (const uint32_t*)orig, pvp)
+  if (pv)
+    XT_RANK_COUNT(true);
+  else
+    XT_RANK_COUNT(false);
+#undef XT_RANK_COUNT
   XT_HIP(ctx, hipGetLastError());
+  ctx->rank_chunks = nch;
   return XT_OK;
 }
 
-template int rank_count<int32_t>(xt_ctx*, Scratch&, int64_t, int64_t, const int64_t*, const int32_t*, hipStream_t,
-                                 hipEvent_t);
-template int rank_count<int64_t>(xt_ctx*, Scratch&, int64_t, int64_t, const int64_t*, const int64_t*, hipStream_t,
-                                 hipEvent_t);
+template int rank_count<int32_t>(xt_ctx*, Scratch&, int64_t, int64_t, const int64_t*, const int32_t*, int, uint64_t*,
+                                 hipStream_t, hipEvent_t);
+template int rank_count<int64_t>(xt_ctx*, Scratch&, int64_t, int64_t, const int64_t*, const int64_t*, int, uint64_t*,
+                                 hipStream_t, hipEvent_t);
 
 }  // namespace xt

@@ -112,6 +112,7 @@ struct Scratch {
   // The count in rank space (rank.hip; it also uses crows, int32 pairs, and itcnt).
   DevBuf rhist;     // uint32[2*classes]   vertices per degree class, ranks handed out per class
   DevBuf rank;      // uint32[nv]          rank by descending degree
+  DevBuf rorig;     // uint32[nv]          label of every rank (per-vertex counts)
   DevBuf ocount;    // uint64[nv]          neighbours of smaller rank | those below 65535 << 32
   DevBuf rpart;     // uint32[ne]          rows as ranks, smaller ones first
   DevBuf rlists;    // 16 B chunks         lists of smaller ranks (hot 16-bit, cold 32-bit)
@@ -143,6 +144,7 @@ struct xt_ctx {
   int wave_owner = -1;       // wave tiles for owner lists up to this long; -1 default, 0 off
   int last_wave_owner = 0;  // wave-owner cut of the last count (tiles [tileoff[nv], tileoff[2nv]) when > 0)
   bool last_ranked = false;  // the last count ran in rank space
+  int64_t rank_chunks = 0;   // and its chunks of entries, a wave each
   bool force_wide = false;  // use the 64-bit offset layout of graphs with >= 2^32 entries everywhere
   int fail_allocs = 0;      // failure injection: scratch allocations left to fail
 };
@@ -152,6 +154,7 @@ struct xt_graph {
   int64_t ne = 0;
   int64_t* off = nullptr;   // int64[nv+1]
   int32_t* tails = nullptr; // int32[ne]
+  int64_t max_degree = -1;  // longest row where the host has seen the offsets, else -1
 };
 
 namespace xt {
@@ -216,19 +219,25 @@ template <typename T>
 int validate(xt_ctx* ctx, int64_t nv, int64_t ne, const int64_t* off, const T* tails,
              bool symmetry, hipStream_t st, uint64_t* counters = nullptr);
 
-// The plain total of one graph counted in rank space: adds to the sums
-// kSumTotal and kSumEdges.  split_done (nullable) is recorded
-// once the lists stand.  Only for sizes that rank_fits() accepts.
-bool rank_fits(const xt_ctx* ctx, int64_t nv, int64_t ne);
+struct RankUse {
+  bool may;
+  int64_t max_degree;
+};
+
+// The total (pv == nullptr) or the per-vertex counts (and the total) of one
+// graph counted in rank space: adds to the sums kSumTotal and kSumEdges and
+// writes pv[nv].  split_done (nullable) is recorded once the lists stand.  Only
+// for sizes that rank_fits() accepts.
+bool rank_fits(const xt_ctx* ctx, int64_t nv, int64_t ne, int mode);
 template <typename T>
-int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* off, const T* tails, hipStream_t st,
-               hipEvent_t split_done);
+int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* off, const T* tails, int mode,
+               uint64_t* pv, hipStream_t st, hipEvent_t split_done);
 
 // Whole single-graph count on the device (orientation + intersection).
-// may_rank: a plain total may be counted in rank space.
+// rank: whether it may be counted in rank space, and the longest row (-1: unknown).
 template <typename T>
 int count_device_csr(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* off, const T* tails,
-                     uint32_t flags, hipStream_t st, bool timed, bool may_rank,
+                     uint32_t flags, hipStream_t st, bool timed, RankUse rank,
                      const OwnedRange* range = nullptr);
 
 // Device generators.
