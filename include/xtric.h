@@ -75,8 +75,8 @@ int xt_ctx_create(int device, xt_ctx** out);
 int xt_ctx_destroy(xt_ctx* ctx);
 const char* xt_last_error(const xt_ctx* ctx);
 int xt_last_timing(const xt_ctx* ctx, xt_timing* out);
-/* Totals of one graph in degree orientation are counted in rank space (vertices
- * ranked by degree, lists of smaller ranks in 16 bits, bit maps in LDS), and so
+/* Totals and owned ranges of one graph in degree orientation are counted in rank
+ * space (vertices ranked by degree, lists of smaller ranks in 16 bits, bit maps in LDS), and so
  * are its per-vertex counts below 2^25 entries and, where the host passed in the
  * offsets and no row is longer than 256, counts in id orientation.  The knobs
  * below belong to the edge tiles that all other counts use; a context on which
@@ -252,9 +252,9 @@ int xt_graph_count(xt_ctx* ctx, xt_graph* g, uint32_t flags, uint64_t* total,
  * *owned, and into *local those whose middle vertex is owned too (the rank
  * counts these itself; the others it forwards as (v, w) pairs to the middle
  * vertex's rank, xxtric.hpp:189-204).  *total (nullable) gets every triangle
- * of g, from a second, plain count.  The owned count skips edges whose smaller
- * endpoint is below lo and streams, per edge, only the ids of the shorter
- * list that can complete an owned triangle.  The count is the same on g and on its slice for [lo, hi).  flags
+ * of g, from a second, plain count.  The owned count leaves out the vertices
+ * below lo and reads, where neither end of an edge is owned, only the owned ids
+ * of a list.  The count is the same on g and on its slice for [lo, hi).  flags
  * selects the orientation; XT_PER_VERTEX is rejected. */
 int xt_graph_slice(xt_ctx* ctx, const xt_graph* g, int64_t lo, int64_t hi, xt_graph** out);
 int xt_graph_count_owned(xt_ctx* ctx, xt_graph* g, int64_t lo, int64_t hi, uint32_t flags,

@@ -1,4 +1,4 @@
-"""The count in rank space (totals and per-vertex counts, library default knobs)
+"""The count in rank space (totals, per-vertex counts and owned ranges, library default knobs)
 at the sizes where it can go wrong: lists around one chunk, one line and
 one wave, ranks on both sides of the 16-bit limit, more cold ids than one hash
 holds, rows across chunks, rows of many empty neighbours, labels in any order.
@@ -139,6 +139,33 @@ def test_host_csr_per_vertex(ctx, n, orient):
     exp = O.count_reference(off, tails.astype(np.int32), per_vertex=True)
     assert _same(ctx.count_csr(off, tails, per_vertex=True, orient=orient), exp)
     assert ctx.count_csr(off, tails, orient=orient) == exp[0]
+
+
+@pytest.mark.parametrize("make", ["rgg90000", "circulant", "rmat17", "rmat13 unpermuted"])
+def test_owned_ranges(ctx, make):
+    """Owned ranges at the ends, in the middle, empty and whole, with cold lists: the owned
+    count against the per-vertex counts, both against the edge tiles."""
+    import xxtric_amd
+    if make == "rgg90000":
+        g = ctx.graph(*xxtric_amd.rgg_generate(90000, seed=5, connect=True, strict=True))
+    elif make == "circulant":
+        g = ctx.graph(*_circulant(HOT + 300, 40))
+    else:
+        g = ctx.rmat(int(make[4:6]), 16, 4, make == "rmat17")
+    _, pv = g.count(per_vertex=True)
+    n = g.nv
+    for lo, hi in ((0, n // 8), (n // 3, n // 2), (n - n // 8, n), (0, n), (7, 7), (n - 1, n), (100, 164)):
+        _say(make, lo, hi)
+        owned, local, _ = g.count_owned(lo, hi, total=False)
+        ne_plus = ctx.timing()["ne_plus"]
+        assert owned == int(pv[lo:hi].sum(dtype=np.uint64))
+        ctx.tune(small_cut=32)
+        try:
+            assert (owned, local) == g.count_owned(lo, hi, total=False)[:2]
+            assert ne_plus == ctx.timing()["ne_plus"]
+        finally:
+            ctx.tune(small_cut=-1)
+    g.close()
 
 
 def test_device_csr_and_graph_sizes_in_a_row(ctx):

@@ -201,9 +201,9 @@ int count_device_csr(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int6
     XT_TRY(ensure(ctx, s.pv, (size_t)(nv > 0 ? nv : 1) * sizeof(uint64_t)));
     pv = s.pv.as<uint64_t>();
   }
-  if (rank.may && !range && ranks(ctx, nv, ne, mode, pv != nullptr, rank.max_degree)) {
+  if (rank.may && ranks(ctx, nv, ne, mode, pv != nullptr, rank.max_degree)) {
     if (timed) XT_HIP(ctx, hipEventRecord(ctx->ev[kEvStart], st));
-    XT_TRY(rank_count<T>(ctx, s, nv, ne, off, tails, mode, pv, st, timed ? ctx->ev[kEvOriented] : nullptr));
+    XT_TRY(rank_count<T>(ctx, s, nv, ne, off, tails, mode, pv, range, st, timed ? ctx->ev[kEvOriented] : nullptr));
     if (timed) XT_HIP(ctx, hipEventRecord(ctx->ev[kEvCounted], st));
     ctx->last_ranked = true;
     return XT_OK;
@@ -978,7 +978,7 @@ int xt_graph_count_owned(xt_ctx* ctx, xt_graph* g, int64_t lo, int64_t hi, uint3
       XT_TRY(finish_count(ctx, g->nv, flags, st, true, total, nullptr));
     }
     const OwnedRange range{lo, hi};
-    XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, g->nv, g->ne, g->off, g->tails, flags, st, true, RankUse{false, -1}, &range));
+    XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, g->nv, g->ne, g->off, g->tails, flags, st, true, RankUse{true, g->max_degree}, &range));
     uint64_t h[kNumCounters];
     XT_TRY(finish_count(ctx, g->nv, flags, st, true, nullptr, nullptr, h));
     *owned = sum_of(h, kSumOwned);

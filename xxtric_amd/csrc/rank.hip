@@ -40,11 +40,23 @@
 
 namespace xt {
 
+// What is counted: the total; per vertex (each triangle credited to its smallest
+// label); or, for an owned label range [lo, hi), the triangles whose smallest
+// label is owned and, of those, the ones whose middle label is owned too.  With
+// labels below lo left out, these are the triangles with one, and with two, of
+// their vertices owned.
+constexpr int kTotal = 0;
+constexpr int kPerVertex = 1;
+constexpr int kRange = 2;
+
 constexpr uint32_t kHot = 65535;       // ranks below are hot; 65535 itself pads 16-bit lists
 constexpr uint32_t kNoRank = ~0u;      // a self-loop or an id out of range; pads cold lists
 constexpr int kRankClasses = 896;      // degree classes: exact below 64, then 32 per octave
 constexpr int kRankMarks = 12;         // ids kept per list for finding prefixes
 constexpr int kRankMarksPv = 10;       // the same beside the vertex's label (per-vertex counts)
+constexpr int kMarksOwned = 3;         // owned-range counts: of the owned ids
+constexpr int kMarksRest = 7;          // ... and of the others
+constexpr uint32_t kOwnedBit = 1u << 31;  // on a rank: its label is owned (ranks are below 2^30)
 constexpr int kAssignRun = 8;          // vertices per thread of k_rank_assign
 constexpr int kLaneList = 32;          // lists of up to this many ids are written by one lane, unsorted
 constexpr int kTinyRow = 8;            // rows of up to this many ids and 64 items: a lane per item
@@ -69,11 +81,14 @@ struct alignas(16) RankRec {
 static_assert(sizeof(RankRec) == 32, "two 16-byte loads");
 
 // A per-vertex count keeps ten marks, and the vertex's label in the last word.
-template <bool PV>
-__device__ __forceinline__ uint32_t mark_step(uint32_t hot) {
-  constexpr uint32_t kMarks = PV ? kRankMarksPv : kRankMarks;
-  return (hot + kMarks - 1) / kMarks;
+// An owned-range count has four parts, each with its own chunks: owned hot ids,
+// other hot ids, owned cold ids, other cold ids; its record holds {start,
+// chunks 0 | 1 << 16, chunks 2 | 3 << 16, three marks of part 0 and seven of part 1}.
+template <int MODE>
+constexpr uint32_t hot_marks() {
+  return MODE == kPerVertex ? kRankMarksPv : kRankMarks;
 }
+__device__ __forceinline__ uint32_t mark_step(uint32_t hot, uint32_t marks) { return (hot + marks - 1) / marks; }
 
 // 16-byte chunks a list of t chunks is given: it starts on a multiple of its size up
 // to eight chunks (a 128-byte line), so no list crosses more lines than it
@@ -89,7 +104,7 @@ __device__ __forceinline__ uint32_t list_room(uint32_t t) {
 __global__ __launch_bounds__(256) void k_rank_prep(int64_t nv, int64_t ne, const int64_t* __restrict__ off, int64_t S,
                                                    int32_t* __restrict__ crows, uint64_t* __restrict__ oc,
                                                    uint32_t* __restrict__ ic, uint32_t* __restrict__ hist,
-                                                   unsigned long long* __restrict__ pv) {
+                                                   unsigned long long* __restrict__ pv, uint64_t* __restrict__ oc1) {
   __shared__ uint32_t s_h[kRankClasses];
   for (int k = threadIdx.x; k < kRankClasses; k += 256) s_h[k] = 0;
   __syncthreads();
@@ -100,6 +115,7 @@ __global__ __launch_bounds__(256) void k_rank_prep(int64_t nv, int64_t ne, const
     oc[u] = 0;
     ic[u] = 0;
     if (pv) pv[u] = 0;
+    if (oc1) oc1[u] = 0;
     atomicAdd(&s_h[degree_class(b - a)], 1u);
     if (a < 0 || b > ne || a >= b) continue;
     for (int64_t c = (a + S - 1) / S; c * S < b; c++) crows[2 * c] = (int32_t)u;
@@ -186,15 +202,23 @@ __global__ __launch_bounds__(256) void k_rank_by_label(int64_t nv, uint32_t* __r
 // and last row, which may continue in another chunk, take their places by
 // atomics.  Entries that are no edge (self-loops, ids out of range) go to the
 // back as kNoRank.
-template <typename T>
+//
+// RANGE: labels below rlo are left out (their rows are empty, entries of them no
+// edges); ranks of owned labels carry kOwnedBit, and oc1[u] counts the owned ones
+// of N(u) as oc[u] counts all.
+template <typename T, bool RANGE>
 __global__ __launch_bounds__(kBlock) void k_rank_split(int64_t nv, int64_t ne, const int64_t* __restrict__ off,
                                                        const T* __restrict__ tails, const uint32_t* __restrict__ rank,
                                                        const int32_t* __restrict__ crows, int per,
                                                        uint32_t* __restrict__ part, uint64_t* __restrict__ oc,
-                                                       uint32_t* __restrict__ ic, uint64_t* __restrict__ counters) {
+                                                       uint32_t* __restrict__ ic, uint64_t* __restrict__ counters,
+                                                       uint64_t* __restrict__ oc1, int64_t rlo, int64_t rhi) {
+  // Of the entries before each entry: smaller ranks | hot ones << 16 and, RANGE,
+  // owned ones << 32 | owned hot ones << 48.
+  using Pre = typename std::conditional<RANGE, uint64_t, uint32_t>::type;
   __shared__ alignas(16) int16_t s_end[kChunk];       // first entry of a row: where the row ends (clamped); 0 elsewhere
   __shared__ uint32_t s_rk[kChunk];       // and its rank; later the chunk's entries in their new order
-  __shared__ uint32_t s_pre[kChunk + 1];  // smaller ranks before each entry | hot ones << 16
+  __shared__ Pre s_pre[kChunk + 1];
   __shared__ int64_t s_scan[kBlock / kWave];
   __shared__ int s_last[kBlock / kWave];
   __shared__ uint32_t s_ob[2], s_ib[2];   // places taken by the first and the last row
@@ -219,7 +243,7 @@ __global__ __launch_bounds__(kBlock) void k_rank_split(int64_t nv, int64_t ne, c
   const bool live = i0 < n;
   *reinterpret_cast<int4*>(&s_end[i0]) = make_int4(0, 0, 0, 0);
   uint32_t rv[kPerThread];
-  uint32_t bad = 0;
+  uint32_t bad = 0, own = 0, out = 0;  // RANGE: entries of owned labels, of labels left out
   if (live) {
     int64_t vals[kPerThread];
     load_run<T>(tails, eb + i0, eb + n, vals);
@@ -229,6 +253,10 @@ __global__ __launch_bounds__(kBlock) void k_rank_split(int64_t nv, int64_t ne, c
       if (in && !ok) bad++;
       const uint32_t r = rank[ok ? vals[j] : 0];
       rv[j] = ok ? r : kNoRank;
+      if constexpr (RANGE) {
+        own |= (ok && vals[j] >= rlo && vals[j] < rhi ? 1u : 0u) << j;
+        out |= (ok && vals[j] < rlo ? 1u : 0u) << j;
+      }
     }
   }
   if (bad) atomicAdd((unsigned long long*)&counters[kBadIds], (unsigned long long)bad);
@@ -238,7 +266,7 @@ __global__ __launch_bounds__(kBlock) void k_rank_split(int64_t nv, int64_t ne, c
     const int ro = rel(o0), re = rel(o1);
     if (re > 0 && ro < n && o1 > o0) {
       s_end[max(ro, 0)] = (int16_t)re;
-      s_rk[max(ro, 0)] = rank[ulo + k];
+      s_rk[max(ro, 0)] = rank[ulo + k] | (RANGE && ulo + k < rlo ? kOwnedBit : 0u);  // RANGE: a row left out
     }
     if (k == 0) {
       s_rng[0] = ro < 0 || re > n ? min(re, n) : 0;
@@ -276,12 +304,17 @@ __global__ __launch_bounds__(kBlock) void k_rank_split(int64_t nv, int64_t ne, c
   if (ends[0]) at = i0;
   at = max(at, 0);  // entry 0 is marked whenever the offsets are an index
   uint32_t small = 0, hot = 0;
+  uint64_t edges = 0;  // RANGE: all of them, as other counts report
   if (live) {
     uint32_t ru = s_rk[at];
 #pragma unroll
     for (int j = 0; j < kPerThread; j++) {
       if (i0 + j < n) {
         if (ends[j]) ru = s_rk[i0 + j];
+        if constexpr (RANGE) {
+          edges += rv[j] < (ru & ~kOwnedBit) ? 1u : 0u;
+          if ((out >> j & 1u) || (ru & kOwnedBit)) rv[j] = kNoRank;
+        }
         if (rv[j] < ru) {
           small |= 1u << j;
           if (rv[j] < kHot) hot |= 1u << j;
@@ -291,34 +324,50 @@ __global__ __launch_bounds__(kBlock) void k_rank_split(int64_t nv, int64_t ne, c
       }
     }
   }
+  auto counts = [&](uint32_t m) -> Pre {  // of the entries in m; a chunk's fields stay below 2^16
+    Pre p = (Pre)(uint32_t)(__popc(small & m) | (__popc(hot & m) << 16));
+    if constexpr (RANGE)
+      p |= (Pre)(uint32_t)(__popc(small & own & m) | (__popc(hot & own & m) << 16)) << 32;
+    return p;
+  };
   int64_t total;
-  const int64_t pre =
-      block_excl_scan_i64<kBlock>((int64_t)(__popc(small) | (__popc(hot) << 16)), s_scan, &total);  // < 2^28: fields do not meet
+  const int64_t pre = block_excl_scan_i64<kBlock>((int64_t)counts(~0u), s_scan, &total);
   if (live) {
 #pragma unroll
     for (int j = 0; j < kPerThread; j++)
-      if (i0 + j < n) {
-        const uint32_t m = (1u << j) - 1u;
-        s_pre[i0 + j] = (uint32_t)pre + (uint32_t)(__popc(small & m) | (__popc(hot & m) << 16));
-      }
+      if (i0 + j < n) s_pre[i0 + j] = (Pre)pre + counts((1u << j) - 1u);
   }
-  if (tid == 0) s_pre[n] = (uint32_t)total;
+  if constexpr (RANGE) {
+    edges = wave_sum_u64(edges);
+    if (lane == 0) add_sum(counters, kSumEdges, edges);
+#pragma unroll
+    for (int j = 0; j < kPerThread; j++)
+      if (own >> j & 1u && rv[j] != kNoRank) rv[j] |= kOwnedBit;
+  }
+  if (tid == 0) s_pre[n] = (Pre)total;
   __syncthreads();  // s_rk is read: its place takes the new order
   for (int64_t k = tid; k < span; k += kBlock) {
     const int64_t o0 = off[ulo + k], o1 = off[ulo + k + 1];
     const int ro = rel(o0), re = rel(o1);
     if (re <= 0 || ro >= n || o1 <= o0) continue;
     const int a = max(ro, 0), b = min(re, n);
-    const uint32_t q = s_pre[b] - s_pre[a];
-    const uint32_t outs = q & 0xffffu;
+    const Pre q = s_pre[b] - s_pre[a];
+    const uint32_t outs = (uint32_t)q & 0xffffu, hots = (uint32_t)q >> 16;
+    uint32_t q1 = 0;
+    if constexpr (RANGE) q1 = (uint32_t)(q >> 32);
     if (ro >= 0 && re <= n) {
-      oc[ulo + k] = (uint64_t)outs | ((uint64_t)(q >> 16) << 32);
+      oc[ulo + k] = (uint64_t)outs | ((uint64_t)hots << 32);
+      if constexpr (RANGE) oc1[ulo + k] = (uint64_t)(q1 & 0xffffu) | ((uint64_t)(q1 >> 16) << 32);
     } else {
       const int s = k == 0 ? 0 : 1;
       const uint32_t ins = (uint32_t)(b - a) - outs;
       s_ob[s] = outs ? (uint32_t)atomicAdd((unsigned long long*)&oc[ulo + k],
-                                           (unsigned long long)outs | ((unsigned long long)(q >> 16) << 32))
+                                           (unsigned long long)outs | ((unsigned long long)hots << 32))
                      : 0u;
+      if constexpr (RANGE)
+        if (q1)
+          atomicAdd((unsigned long long*)&oc1[ulo + k],
+                    (unsigned long long)(q1 & 0xffffu) | ((unsigned long long)(q1 >> 16) << 32));
       s_ib[s] = ins ? atomicAdd(&ic[ulo + k], ins) : 0u;
     }
   }
@@ -334,15 +383,15 @@ __global__ __launch_bounds__(kBlock) void k_rank_split(int64_t nv, int64_t ne, c
           nxt = ends[j];
         }
         const bool first = cur == 0 && s_rng[2];  // continues from an earlier chunk
-        const uint32_t before = (s_pre[i] - s_pre[cur]) & 0xffffu;
-        const bool out = (small >> j) & 1u;
+        const uint32_t before = (uint32_t)(s_pre[i] - s_pre[cur]) & 0xffffu;
+        const bool front = (small >> j) & 1u;
         if (!first && nxt <= n) {
-          s_part[out ? cur + (int)before : nxt - 1 - (i - cur - (int)before)] = rv[j];
+          s_part[front ? cur + (int)before : nxt - 1 - (i - cur - (int)before)] = rv[j];
         } else {
           const int s = first || uhi == ulo ? 0 : 1;
           const int64_t u = s == 0 ? ulo : uhi;
-          part[out ? off[u] + (int64_t)s_ob[s] + before
-                   : off[u + 1] - 1 - (int64_t)s_ib[s] - (int64_t)(i - cur - (int)before)] = rv[j];
+          part[front ? off[u] + (int64_t)s_ob[s] + before
+                     : off[u + 1] - 1 - (int64_t)s_ib[s] - (int64_t)(i - cur - (int)before)] = rv[j];
         }
       }
     }
@@ -373,16 +422,18 @@ struct ListRoom {
   int64_t nbatch;
 };
 
-template <bool PV>
+template <int MODE>
 __global__ __launch_bounds__(64) void k_rank_lists(int64_t nv, const int64_t* __restrict__ off,
-                                                   const uint64_t* __restrict__ oc, const uint32_t* __restrict__ rank,
+                                                   const uint64_t* __restrict__ oc, const uint64_t* __restrict__ oc1,
+                                                   const uint32_t* __restrict__ rank,
                                                    const uint32_t* __restrict__ part, ListRoom lr,
                                                    uint4* __restrict__ lists, RankRec* __restrict__ rec,
                                                    uint64_t* __restrict__ counters) {
   constexpr int kGroups = 8;  // pairs of 64-bit words per lane
   __shared__ ulonglong2 s_bits[kGroups * kWave];
   __shared__ uint16_t s_pre[kGroups * kWave];
-  constexpr uint32_t kMarks = PV ? kRankMarksPv : kRankMarks;
+  constexpr bool PV = MODE == kPerVertex, RANGE = MODE == kRange;
+  constexpr int kParts = RANGE ? 2 : 1;  // hot parts (and as many cold ones)
   __shared__ uint16_t s_mark[kRankMarks];
   const int lane = threadIdx.x;
   unsigned long long* bits = reinterpret_cast<unsigned long long*>(s_bits);
@@ -418,7 +469,8 @@ __global__ __launch_bounds__(64) void k_rank_lists(int64_t nv, const int64_t* __
     const uint64_t g = (uint64_t)batch * (uint64_t)(lr.rows >> lr.together) + (uint64_t)(lane >> lr.together);
     const int64_t u = g < groups && lane < lr.rows ? (int64_t)((g * 2654435761ull % groups) << lr.together) | (lane & ((1 << lr.together) - 1)) : nv;
     const bool live = u < nv;
-    uint32_t d = 0, h = 0, hc = 0, cc = 0, a0 = 0, ru = 0;
+    uint32_t d = 0, h = 0, a0 = 0, ru = 0;
+    uint32_t hc = 0, cc = 0;  // hot and cold chunks; RANGE: two parts each, part 1 << 16
     if (live) {
       const uint64_t q = oc[u];
       d = (uint32_t)q;
@@ -426,12 +478,22 @@ __global__ __launch_bounds__(64) void k_rank_lists(int64_t nv, const int64_t* __
       a0 = (uint32_t)off[u];
       ru = rank[u];
       if (d >= 2) {  // a list of one id has no pair
-        hc = min((h + 7) >> 3, 8192u);  // (the clamps hold for any input that is a simple graph)
-        cc = min((d - h + 3) >> 2, 65535u);
+        auto hot_chunks = [](uint32_t n) { return min((n + 7) >> 3, 8192u); };  // (the clamps hold for
+        auto cold_chunks = [](uint32_t n) { return min((n + 3) >> 2, 65535u); };  // any simple graph)
+        if constexpr (RANGE) {
+          const uint64_t q1 = oc1[u];
+          const uint32_t d1 = (uint32_t)q1, h1 = (uint32_t)(q1 >> 32);
+          hc = hot_chunks(h1) | hot_chunks(h - h1) << 16;
+          cc = cold_chunks(d1 - h1) | cold_chunks((d - d1) - (h - h1)) << 16;
+        } else {
+          hc = hot_chunks(h);
+          cc = cold_chunks(d - h);
+        }
       }
     }
-    edges += d;
-    const uint32_t room = list_room(hc + cc);
+    if constexpr (!RANGE) edges += d;
+    auto both = [](uint32_t c) -> uint32_t { return RANGE ? (c & 0xffffu) + (c >> 16) : c; };
+    const uint32_t room = list_room(both(hc) + both(cc));
     // lines: bits 0-31; lists of four, two, one chunk: 10 bits each from 32 on
     const int64_t mine = room >= 8 ? (int64_t)(room >> 3) : room == 4 ? 1ll << 32 : room == 2 ? 1ll << 42 : room == 1 ? 1ll << 52 : 0ll;
     const int64_t inc = wave_incl_scan_i64(mine), at = inc - mine, total = readlane64(inc, kWave - 1);
@@ -461,7 +523,38 @@ __global__ __launch_bounds__(64) void k_rank_lists(int64_t nv, const int64_t* __
       to[0] = make_uint4(0, 0, 0, 0);
       to[1] = make_uint4(0, 0, 0, PV ? (uint32_t)u : 0u);
     }
-    if (__builtin_amdgcn_ballot_w64(alone && d >= 2)) {  // uniform
+    if constexpr (RANGE) {
+      if (alone && d >= 2) {  // part by part: hot ids, padding, cold ids, padding
+        uint16_t* hot[2] = {reinterpret_cast<uint16_t*>(lists + start),
+                            reinterpret_cast<uint16_t*>(lists + start + (hc & 0xffffu))};
+        uint32_t* cold[2] = {reinterpret_cast<uint32_t*>(lists + start + both(hc)),
+                             reinterpret_cast<uint32_t*>(lists + start + both(hc) + (cc & 0xffffu))};
+        uint32_t nh[2] = {0, 0}, nc[2] = {0, 0}, least[2] = {kHot, kHot};
+        for (uint32_t i = 0; i < d; i++) {
+          const uint32_t w = part[a0 + i], r = w & ~kOwnedBit;
+          const bool rest = !(w & kOwnedBit);
+#pragma unroll
+          for (int p = 0; p < 2; p++) {
+            if (rest != (p == 1)) continue;
+            if (r < kHot) {
+              hot[p][nh[p]++] = (uint16_t)r;
+              least[p] = min(least[p], r);
+            } else {
+              cold[p][nc[p]++] = r;
+            }
+          }
+        }
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+          for (; nh[p] & 7; nh[p]++) hot[p][nh[p]] = 0xffff;
+          for (; nc[p] & 3; nc[p]++) cold[p][nc[p]] = kNoRank;
+        }
+        // Not sorted: all of a part or nothing of it is below v.
+        uint4* to = reinterpret_cast<uint4*>(rec + ru);
+        to[0] = make_uint4(start, hc, cc, least[0] | (least[0] << 16));
+        to[1] = make_uint4(least[0] | (least[1] << 16), least[1] | (least[1] << 16), least[1] | 0xffff0000u, ~0u);
+      }
+    } else if (__builtin_amdgcn_ballot_w64(alone && d >= 2)) {  // uniform
       uint64_t lo = ~0ull, hi = ~0ull;
       uint32_t least = kHot, nh = 0, nc = 0;
       uint4* hot = lists + start;
@@ -497,8 +590,8 @@ __global__ __launch_bounds__(64) void k_rank_lists(int64_t nv, const int64_t* __
       }
     }
     uint64_t todo = __builtin_amdgcn_ballot_w64(live && d > kLaneList);
-    // The next row: first entry, ids, list, rank, label; its first ids.
-    uint32_t ra = 0, rd = 0, rs = 0, rr = 0, ro = 0, rw = kNoRank;
+    // The next row: first entry, ids, list, rank, label, chunks; its first ids.
+    uint32_t ra = 0, rd = 0, rs = 0, rr = 0, ro = 0, rhc = 0, rcc = 0, rw = kNoRank;
     auto pop = [&]() {
       const int src = __builtin_ctzll(todo);
       todo &= todo - 1;
@@ -507,88 +600,115 @@ __global__ __launch_bounds__(64) void k_rank_lists(int64_t nv, const int64_t* __
       rs = __builtin_amdgcn_readlane(start, src);
       rr = __builtin_amdgcn_readlane(ru, src);
       if constexpr (PV) ro = __builtin_amdgcn_readlane((uint32_t)u, src);
+      rhc = __builtin_amdgcn_readlane(hc, src);
+      rcc = __builtin_amdgcn_readlane(cc, src);
       rw = part[ra + lane];  // more than 32 ids and, in a simple graph, as many behind; the array is padded
     };
     bool more = todo != 0;
     if (more) pop();
     while (more) {  // uniform
-      const uint32_t dd = rd, st = rs, rk = rr, label = ro, w0 = (uint32_t)lane < rd ? rw : kNoRank;
+      const uint32_t dd = rd, st = rs, rk = rr, label = ro, hcs = rhc, ccs = rcc, w0 = (uint32_t)lane < rd ? rw : kNoRank;
       const uint32_t* ids = part + ra;
       more = todo != 0;
       if (more) pop();  // the next row's ids fly while this one is written
-      auto id = [&](uint32_t i) -> uint32_t { return i == 0 ? w0 : i + lane < dd ? ids[i + lane] : kNoRank; };
+      auto raw = [&](uint32_t i) -> uint32_t { return i == 0 ? w0 : i + lane < dd ? ids[i + lane] : kNoRank; };
       if (lane < kRankMarks) s_mark[lane] = 0xffff;
-      uint32_t hh = 0, place = 0;
-      if (dd <= kWave) {
-        const uint64_t hm = __builtin_amdgcn_ballot_w64(w0 < kHot);
-        hh = (uint32_t)__popcll(hm);
-        for (uint64_t m = hm; m; m &= m - 1)
-          place += (uint32_t)__builtin_amdgcn_readlane((int)w0, __builtin_ctzll(m)) < w0 ? 1u : 0u;
-      } else {
-        uint32_t top = 0;  // groups in use
-        for (uint32_t i = 0; i < dd; i += kWave) {
-          const uint32_t w = id(i);
-          if (w < kHot) {
-            atomicOr(&bits[w >> 6], 1ull << (w & 63));
-            top = max(top, (w >> 13) + 1);
+      uint32_t mark0 = 0, hot0 = 0, cold0 = both(hcs);  // where the part's marks and chunks start
+#pragma unroll
+      for (int part_no = 0; part_no < kParts; part_no++) {
+        const uint32_t hcc = RANGE ? (hcs >> (16 * part_no)) & 0xffffu : hcs;
+        const uint32_t ccc = RANGE ? (ccs >> (16 * part_no)) & 0xffffu : ccs;
+        const uint32_t marks = !RANGE ? hot_marks<MODE>() : part_no == 0 ? kMarksOwned : kMarksRest;
+        // The part's rank at i + lane, kNoRank where it has none.
+        auto id = [&](uint32_t i) -> uint32_t {
+          const uint32_t w = raw(i);
+          if constexpr (RANGE)
+            return w != kNoRank && (w & kOwnedBit ? 0 : 1) == part_no ? w & ~kOwnedBit : kNoRank;
+          else
+            return w;
+        };
+        uint32_t hh = 0, place = 0;
+        if (dd <= kWave) {
+          const uint32_t w = id(0);
+          const uint64_t hm = __builtin_amdgcn_ballot_w64(w < kHot);
+          hh = (uint32_t)__popcll(hm);
+          for (uint64_t m = hm; m; m &= m - 1)
+            place += (uint32_t)__builtin_amdgcn_readlane((int)w, __builtin_ctzll(m)) < w ? 1u : 0u;
+        } else {
+          uint32_t top = 0;  // groups in use
+          for (uint32_t i = 0; i < dd; i += kWave) {
+            const uint32_t w = id(i);
+            if (w < kHot) {
+              atomicOr(&bits[w >> 6], 1ull << (w & 63));
+              top = max(top, (w >> 13) + 1);
+            }
+          }
+          wave_lds_fence();
+#pragma unroll 1
+          for (uint32_t k = 0; k < (uint32_t)kGroups; k++) {
+            if (__builtin_amdgcn_ballot_w64(top > k) == 0) break;
+            const ulonglong2 t = s_bits[k * kWave + lane];
+            const uint32_t n = (uint32_t)(__popcll(t.x) + __popcll(t.y));
+            const uint32_t upto = wave_incl_scan_u32(n);
+            s_pre[k * kWave + lane] = (uint16_t)(hh + upto - n);
+            hh += __builtin_amdgcn_readlane(upto, kWave - 1);
           }
         }
         wave_lds_fence();
-#pragma unroll 1
-        for (uint32_t k = 0; k < (uint32_t)kGroups; k++) {
-          if (__builtin_amdgcn_ballot_w64(top > k) == 0) break;
-          const ulonglong2 t = s_bits[k * kWave + lane];
-          const uint32_t n = (uint32_t)(__popcll(t.x) + __popcll(t.y));
-          const uint32_t upto = wave_incl_scan_u32(n);
-          s_pre[k * kWave + lane] = (uint16_t)(hh + upto - n);
-          hh += __builtin_amdgcn_readlane(upto, kWave - 1);
-        }
-      }
-      wave_lds_fence();
-      const uint32_t hcc = min((hh + 7) >> 3, 8192u), ccc = min((dd - hh + 3) >> 2, 65535u);
-      const uint32_t seg = 8 * max(mark_step<PV>(hcc), 1u);               // ids per segment
-      const uint32_t inv = (uint32_t)(((1ull << 32) + seg - 1) / seg);  // r / seg for r < 2^16
-      uint16_t* hl = reinterpret_cast<uint16_t*>(lists + st);
-      uint32_t* cl = reinterpret_cast<uint32_t*>(lists + st + hcc);
-      uint32_t ncold = 0;
-      for (uint32_t i = 0; i < dd; i += kWave) {
-        const uint32_t w = id(i);
-        const bool cold = i + lane < dd && w >= kHot;
-        const uint64_t cm = __builtin_amdgcn_ballot_w64(cold);
-        if (w < kHot) {
-          uint32_t r = place;
-          if (dd > kWave) {
-            const ulonglong2 t = s_bits[w >> 7];
-            const uint64_t below = (1ull << (w & 63)) - 1ull;
-            r = s_pre[w >> 7] + (uint32_t)((w & 64) ? __popcll(t.x) + __popcll(t.y & below) : __popcll(t.x & below));
-          }
-          if (r < 8 * hcc) hl[r] = (uint16_t)w;
-          const uint32_t k = __umulhi(r, inv);
-          if (k * seg == r && k < kMarks) s_mark[k] = (uint16_t)w;
-        } else if (cold) {
-          const uint32_t r = ncold + lanes_below(cm);
-          if (r < 4 * ccc) cl[r] = w;
-        }
-        ncold += (uint32_t)__popcll(cm);
-      }
-      wave_lds_fence();
-      if (dd > kWave)
+        const uint32_t seg = 8 * max(mark_step(hcc, marks), 1u);          // ids per segment
+        const uint32_t inv = (uint32_t)(((1ull << 32) + seg - 1) / seg);  // r / seg for r < 2^16
+        uint16_t* hl = reinterpret_cast<uint16_t*>(lists + st + hot0);
+        uint32_t* cl = reinterpret_cast<uint32_t*>(lists + st + cold0);
+        uint32_t ncold = 0;
         for (uint32_t i = 0; i < dd; i += kWave) {
           const uint32_t w = id(i);
-          if (w < kHot) bits[w >> 6] = 0ull;
+          const bool cold = w >= kHot && w != kNoRank;
+          const uint64_t cm = __builtin_amdgcn_ballot_w64(cold);
+          if (w < kHot) {
+            uint32_t r = place;
+            if (dd > kWave) {
+              const ulonglong2 t = s_bits[w >> 7];
+              const uint64_t below = (1ull << (w & 63)) - 1ull;
+              r = s_pre[w >> 7] + (uint32_t)((w & 64) ? __popcll(t.x) + __popcll(t.y & below) : __popcll(t.x & below));
+            }
+            if (r < 8 * hcc) hl[r] = (uint16_t)w;
+            const uint32_t k = __umulhi(r, inv);
+            if (k * seg == r && k < marks) s_mark[mark0 + k] = (uint16_t)w;
+          } else if (cold) {
+            const uint32_t r = ncold + lanes_below(cm);
+            if (r < 4 * ccc) cl[r] = w;
+          }
+          ncold += (uint32_t)__popcll(cm);
         }
-      if ((uint32_t)lane < 8 * hcc - min(hh, 8 * hcc)) hl[hh + lane] = 0xffff;
-      if ((uint32_t)lane < 4 * ccc - min(dd - hh, 4 * ccc)) cl[dd - hh + lane] = kNoRank;
+        wave_lds_fence();
+        if (dd > kWave)
+          for (uint32_t i = 0; i < dd; i += kWave) {
+            const uint32_t w = id(i);
+            if (w < kHot) bits[w >> 6] = 0ull;
+          }
+        if ((uint32_t)lane < 8 * hcc - min(hh, 8 * hcc)) hl[hh + lane] = 0xffff;
+        if ((uint32_t)lane < 4 * ccc - min(ncold, 4 * ccc)) cl[ncold + lane] = kNoRank;
+        mark0 += marks;
+        hot0 += hcc;
+        cold0 += ccc;
+        wave_lds_fence();
+      }
       if (lane < 8) {
-        const uint32_t m = lane >= 2 ? (uint32_t)s_mark[2 * lane - 4] | ((uint32_t)s_mark[2 * lane - 3] << 16) : 0u;
-        reinterpret_cast<uint32_t*>(rec + rk)[lane] =
-            lane == 0 ? st : lane == 1 ? hcc | (ccc << 16) : PV && lane == 7 ? label : m;
+        constexpr int kFirst = RANGE ? 3 : 2;  // words before the marks
+        const uint32_t m = lane >= kFirst ? (uint32_t)s_mark[2 * (lane - kFirst)] | ((uint32_t)s_mark[2 * (lane - kFirst) + 1] << 16) : 0u;
+        reinterpret_cast<uint32_t*>(rec + rk)[lane] = lane == 0   ? st
+                                                      : lane == 1 ? (RANGE ? hcs : hcs | (ccs << 16))
+                                                      : RANGE && lane == 2 ? ccs
+                                                      : PV && lane == 7    ? label
+                                                                           : m;
       }
       wave_lds_fence();
     }
   }
-  edges = wave_sum_u64(edges);
-  if (lane == 0) add_sum(counters, kSumEdges, edges);
+  if constexpr (!RANGE) {
+    edges = wave_sum_u64(edges);
+    if (lane == 0) add_sum(counters, kSumEdges, edges);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -610,15 +730,17 @@ struct StreamLds {
   unsigned long long bit[kStreamBlocks];
   uint32_t adj[kWave];  // per item with chunks: its list's start less its first chunk
 };
-// Per-vertex counts, per item: u's label and the hits credited to u.
+// Per item: u's label and the hits credited to u (per-vertex counts), or a mask
+// of the hits that count as local (owned ranges).
 struct ItemLds {
   uint32_t label[kWave];
   uint32_t hits[kWave];
 };
 
 // probe(chunk, item): item is the chunk's index among the items with chunks.
-// PV: `label` is u's label; the hits that probe adds to items are added to pv.
-template <bool PV, typename F>
+// kPerVertex: `label` is u's label; the hits that probe adds to items are added
+// to pv.  kRange: `label` is kept for probe.
+template <int MODE, typename F>
 __device__ __forceinline__ void stream_lists(uint32_t start, uint32_t n, uint32_t label, StreamLds& s, ItemLds* s_items,
                                              int lane, const uint4* __restrict__ lists, uint32_t pad,
                                              unsigned long long* __restrict__ pv, F&& probe) {
@@ -631,10 +753,10 @@ __device__ __forceinline__ void stream_lists(uint32_t start, uint32_t n, uint32_
     return v;
   };
   const uint64_t some = __builtin_amdgcn_ballot_w64(n > 0);
-  if constexpr (PV) {
+  if constexpr (MODE != kTotal) {
     wave_lds_fence();
     if (n > 0) s_items->label[lanes_below(some)] = label;
-    s_items->hits[lane] = 0;
+    if constexpr (MODE == kPerVertex) s_items->hits[lane] = 0;
     wave_lds_fence();
   }
   if (all <= kStreamBlocks * kWave) {
@@ -683,7 +805,7 @@ __device__ __forceinline__ void stream_lists(uint32_t start, uint32_t n, uint32_
       }
     }
   }
-  if constexpr (PV) {
+  if constexpr (MODE == kPerVertex) {
     wave_lds_fence();
     const uint32_t t = s_items->hits[lane];
     if (t) atomicAdd(&pv[s_items->label[lane]], (unsigned long long)t);
@@ -715,31 +837,40 @@ struct PvLds {
   uint32_t hits[kSlots];
   ItemLds items;
 };
+struct RangeLds {
+  ItemLds items;
+};
 struct NoLds {};
 
-template <bool PV>
+// kRange: a triangle with its labels above rlo counts as owned when one of its
+// vertices is owned, as local when two are.  Of u's list the owned ids are
+// streamed for every item, the others only where u or v is owned (rank 0 of 8
+// of R-MAT s23: 20.3 ms in edge tiles, 12.5 here, 6.1 of them in this kernel
+// against 9.2 for the total).
+template <int MODE>
 __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const int64_t* __restrict__ off,
                                                    const uint32_t* __restrict__ rank, const uint64_t* __restrict__ oc,
                                                    const uint32_t* __restrict__ part, const RankRec* __restrict__ rec,
                                                    const uint4* __restrict__ lists, const int32_t* __restrict__ crows,
                                                    int64_t S, uint64_t* __restrict__ counters,
                                                    const uint32_t* __restrict__ orig,
-                                                   unsigned long long* __restrict__ pv) {
+                                                   unsigned long long* __restrict__ pv, int64_t rlo, int64_t rhi) {
+  constexpr bool PV = MODE == kPerVertex, RANGE = MODE == kRange;
   constexpr int kWords = 2048;
   constexpr int kColdSmall = 6, kColdBig = 9;  // hash buckets (log2) for up to 128 and up to 1024 cold ids
   __shared__ uint4 s_mem[kWords / 4];
   __shared__ StreamLds s_stream;
-  __shared__ typename std::conditional<PV, PvLds, NoLds>::type s_pv;
+  __shared__ typename std::conditional<PV, PvLds, typename std::conditional<RANGE, RangeLds, NoLds>::type>::type s_pv;
   ItemLds* s_items = nullptr;
-  if constexpr (PV) s_items = &s_pv.items;
+  if constexpr (MODE != kTotal) s_items = &s_pv.items;
   uint32_t* s_bm = reinterpret_cast<uint32_t*>(s_mem);
   int4* s_tab = reinterpret_cast<int4*>(s_mem);
   const int lane = threadIdx.x;
   const int64_t c = blockIdx.x;
   const int64_t eb = c * S, ee = min(ne, eb + S);
-  int64_t rlo = crows[2 * c], rhi = crows[2 * c + 1];
-  rlo = rlo < 0 ? 0 : (rlo > nv - 1 ? nv - 1 : rlo);
-  rhi = rhi < rlo ? rlo : (rhi > nv - 1 ? nv - 1 : rhi);
+  int64_t row_lo = crows[2 * c], row_hi = crows[2 * c + 1];
+  row_lo = row_lo < 0 ? 0 : (row_lo > nv - 1 ? nv - 1 : row_lo);
+  row_hi = row_hi < row_lo ? row_lo : (row_hi > nv - 1 ? nv - 1 : row_hi);
   auto clear_words = [&](int quads) {  // 16-byte pieces from the front
     for (int i = lane; i < quads; i += kWave) s_mem[i] = make_uint4(0, 0, 0, 0);
   };
@@ -747,6 +878,9 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
   if constexpr (PV)
     for (int i = lane; i < kSlots; i += kWave) s_pv.hits[i] = 0;
   wave_lds_fence();
+  uint64_t hits = 0, local = 0;  // local: kRange
+  auto strip = [](uint32_t w) -> uint32_t { return RANGE && w != kNoRank ? w & ~kOwnedBit : w; };
+  auto owned = [&](uint32_t label) -> bool { return (int64_t)label >= rlo && (int64_t)label < rhi; };
   auto tiny_rows = [&](bool tiny, uint32_t a0, uint32_t is, uint32_t items, uint32_t d, uint32_t row0) -> uint32_t {
     const uint32_t n = tiny ? items : 0;
     const uint32_t inc = wave_incl_scan_u32(n), p = inc - n;
@@ -769,17 +903,24 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
       const uint32_t first = (uint32_t)__shfl((int)a0, row, kWave), nd = (uint32_t)__shfl((int)d, row, kWave);
       uint32_t x[kTinyRow];
       uint2 r = make_uint2(0, 0);
-      uint32_t two = 0;  // PV: the smaller of u's and v's label
+      uint32_t two = 0;  // PV: the smaller of u's and v's label; RANGE: how many of the two are owned
+      uint32_t cold2 = 0;  // RANGE: the cold parts' chunks
 #pragma unroll
       for (int i = 0; i < kTinyRow; i++) x[i] = kNoRank - 1;  // matches no id and no padding
       if (c < all) {
         const uint32_t ur = part[entry];
 #pragma unroll
         for (int i = 0; i < kTinyRow; i++)
-          if ((uint32_t)i < nd) x[i] = part[first + i];
-        if (ur != kNoRank) r = *reinterpret_cast<const uint2*>(rec + ur);
-        if constexpr (PV)
-          if (ur != kNoRank) two = min(rec[ur].mark[5], row0 + (uint32_t)row);
+          if ((uint32_t)i < nd) x[i] = strip(part[first + i]);
+        if (ur != kNoRank) {
+          const RankRec* q = rec + strip(ur);
+          r = *reinterpret_cast<const uint2*>(q);
+          if constexpr (PV) two = min(q->mark[5], row0 + (uint32_t)row);
+          if constexpr (RANGE) {
+            cold2 = q->mark[0];
+            two = (ur & kOwnedBit ? 1u : 0u) + (owned(row0 + (uint32_t)row) ? 1u : 0u);
+          }
+        }
       }
       // PV: the ids w of a chunk that N(v) holds (bit j: id j), one credit each.
       auto credit = [&](uint32_t found, auto&& w) {
@@ -790,61 +931,79 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
           atomicAdd(&pv[min(two, orig[w(j)])], 1ull);
         }
       };
-      const uint32_t hc = r.y & 0xffffu, cc = r.y >> 16;
-      for (uint32_t k = 0; __builtin_amdgcn_ballot_w64(k < hc); k++) {
-        if (k < hc) {
-          const uint4 q = lists[r.x + k];
-          const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-          uint32_t found = 0;
+      // One hot and one cold part: cnt chunks from `from`, every id compared with
+      // every id of N(v); every lane its own item's.
+      auto hot_part = [&](uint32_t from, uint32_t cnt) -> uint32_t {
+        uint32_t acc = 0;
+        for (uint32_t k = 0; __builtin_amdgcn_ballot_w64(k < cnt); k++) {
+          if (k < cnt) {
+            const uint4 q = lists[from + k];
+            const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+            uint32_t found = 0;
 #pragma unroll
-          for (int j = 0; j < 4; j++) {
-            const uint32_t lo = w[j] & 0xffffu, hi = w[j] >> 16;
-            const uint32_t lo2 = lo < kHot ? lo : kNoRank, hi2 = hi < kHot ? hi : kNoRank;
-            bool in_lo = false, in_hi = false;
+            for (int j = 0; j < 4; j++) {
+              const uint32_t lo = w[j] & 0xffffu, hi = w[j] >> 16;
+              const uint32_t lo2 = lo < kHot ? lo : kNoRank, hi2 = hi < kHot ? hi : kNoRank;
+              bool in_lo = false, in_hi = false;
 #pragma unroll
-            for (int i = 0; i < kTinyRow; i++) {
-              if constexpr (PV) {
-                in_lo |= x[i] == lo2;
-                in_hi |= x[i] == hi2;
-              } else {
-                acc += (x[i] == lo2 ? 1u : 0u) + (x[i] == hi2 ? 1u : 0u);
+              for (int i = 0; i < kTinyRow; i++) {
+                if constexpr (PV) {
+                  in_lo |= x[i] == lo2;
+                  in_hi |= x[i] == hi2;
+                } else {
+                  acc += (x[i] == lo2 ? 1u : 0u) + (x[i] == hi2 ? 1u : 0u);
+                }
               }
+              found |= (in_lo ? 1u : 0u) << (2 * j) | (in_hi ? 1u : 0u) << (2 * j + 1);
             }
-            found |= (in_lo ? 1u : 0u) << (2 * j) | (in_hi ? 1u : 0u) << (2 * j + 1);
+            if constexpr (PV)
+              credit(found, [&](int j) { return ((j & 4) ? (j & 2 ? w[3] : w[2]) : (j & 2 ? w[1] : w[0])) >> (16 * (j & 1)) & 0xffffu; });
           }
-          if constexpr (PV)
-            credit(found, [&](int j) { return ((j & 4) ? (j & 2 ? w[3] : w[2]) : (j & 2 ? w[1] : w[0])) >> (16 * (j & 1)) & 0xffffu; });
         }
-      }
-      for (uint32_t k = 0; __builtin_amdgcn_ballot_w64(k < cc); k++) {
-        if (k < cc) {
-          const uint4 q = lists[r.x + hc + k];
-          const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-          uint32_t found = 0;
+        return acc;
+      };
+      auto cold_part = [&](uint32_t from, uint32_t cnt) -> uint32_t {
+        uint32_t acc = 0;
+        for (uint32_t k = 0; __builtin_amdgcn_ballot_w64(k < cnt); k++) {
+          if (k < cnt) {
+            const uint4 q = lists[from + k];
+            const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+            uint32_t found = 0;
 #pragma unroll
-          for (int j = 0; j < 4; j++) {
-            bool in = false;
+            for (int j = 0; j < 4; j++) {
+              bool in = false;
 #pragma unroll
-            for (int i = 0; i < kTinyRow; i++) {
-              if constexpr (PV)
-                in |= x[i] == w[j];
-              else
-                acc += x[i] == w[j] ? 1u : 0u;
+              for (int i = 0; i < kTinyRow; i++) {
+                if constexpr (PV)
+                  in |= x[i] == w[j];
+                else
+                  acc += x[i] == w[j] ? 1u : 0u;
+              }
+              found |= (in ? 1u : 0u) << j;
             }
-            found |= (in ? 1u : 0u) << j;
+            if constexpr (PV) credit(found, [&](int j) { return (j & 2) ? (j & 1 ? w[3] : w[2]) : (j & 1 ? w[1] : w[0]); });
           }
-          if constexpr (PV) credit(found, [&](int j) { return (j & 2) ? (j & 1 ? w[3] : w[2]) : (j & 1 ? w[1] : w[0]); });
         }
+        return acc;
+      };
+      if constexpr (RANGE) {
+        const uint32_t h0 = r.y & 0xffffu, h1 = r.y >> 16, c0 = cold2 & 0xffffu, c1 = cold2 >> 16;
+        const uint32_t a = hot_part(r.x, h0) + cold_part(r.x + h0 + h1, c0);  // owned ids
+        const uint32_t o = hot_part(r.x + h0, two ? h1 : 0) + cold_part(r.x + h0 + h1 + c0, two ? c1 : 0);
+        acc += a + o;
+        local += (two ? a : 0) + (two == 2 ? o : 0);
+      } else {
+        const uint32_t hc = r.y & 0xffffu, cc = r.y >> 16;
+        acc += hot_part(r.x, hc) + cold_part(r.x + hc, cc);
       }
     }
     return acc;
   };
-  uint64_t hits = 0;
-  for (int64_t rb = rlo; rb <= rhi; rb += kWave) {
+  for (int64_t rb = row_lo; rb <= row_hi; rb += kWave) {
     const int64_t r = rb + lane;
     int64_t a0 = 0, is = 0, ie = 0;
     uint32_t d = 0, h = 0, v = 0;
-    if (r <= rhi) {
+    if (r <= row_hi) {
       const uint64_t q = oc[r];
       a0 = off[r];
       ie = min(off[r + 1], ee);
@@ -878,7 +1037,7 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
     auto head = [&](uint32_t ur) -> Head {
       Head x{make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)};
       if (ur != kNoRank) {
-        const uint4* q = reinterpret_cast<const uint4*>(rec + ur);
+        const uint4* q = reinterpret_cast<const uint4*>(rec + strip(ur));
         x.a = q[0];
         x.b = q[1];
       }
@@ -886,29 +1045,47 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
     };
     if (todo == 0) continue;  // uniform
     pop();
-    uint32_t w0 = (uint32_t)lane < dd ? part[b0 + lane] : kNoRank;
-    Head x = head(item(s0));
+    uint32_t w0 = (uint32_t)lane < dd ? strip(part[b0 + lane]) : kNoRank;
+    uint32_t xu = item(s0);
+    Head x = head(xu);
     for (;;) {  // uniform
       const uint32_t cb = b0, cs0 = s0, cs1 = s1, cd = dd, ch = hh, cv = vv, cl = vo, w = w0;
       const bool more = todo != 0;
       uint32_t un = kNoRank;
       if (more) {
         pop();
-        w0 = (uint32_t)lane < dd ? part[b0 + lane] : kNoRank;
+        w0 = (uint32_t)lane < dd ? strip(part[b0 + lane]) : kNoRank;
         un = item(s0);
       }
-      auto id = [&](uint32_t i) -> uint32_t { return i == 0 ? w : i + lane < cd ? part[cb + i + lane] : kNoRank; };
+      auto id = [&](uint32_t i) -> uint32_t { return i == 0 ? w : i + lane < cd ? strip(part[cb + i + lane]) : kNoRank; };
       // Hot chunks of the item whose record is h that hold every id below v.
       auto prefix = [&](const Head& h) -> uint32_t {
         const uint32_t hot = h.a.y & 0xffffu;
         const uint32_t mk[kRankMarks / 2] = {h.a.z, h.a.w, h.b.x, h.b.y, h.b.z, h.b.w};
         uint32_t segs = 0;  // segments that start below v
 #pragma unroll
-        for (int t = 0; t < (PV ? kRankMarksPv : kRankMarks) / 2; t++) segs += ((mk[t] & 0xffffu) < cv ? 1u : 0u) + ((mk[t] >> 16) < cv ? 1u : 0u);
-        return min(segs * mark_step<PV>(hot), hot);
+        for (int t = 0; t < (int)hot_marks<MODE>() / 2; t++) segs += ((mk[t] & 0xffffu) < cv ? 1u : 0u) + ((mk[t] >> 16) < cv ? 1u : 0u);
+        return min(segs * mark_step(hot, hot_marks<MODE>()), hot);
       };
+      // kRange: the same of the owned ids and of the others.
+      auto prefix_owned = [&](const Head& h) -> uint32_t {
+        const uint32_t hot = h.a.y & 0xffffu;
+        const uint32_t segs = ((h.a.w & 0xffffu) < cv ? 1u : 0u) + ((h.a.w >> 16) < cv ? 1u : 0u) + ((h.b.x & 0xffffu) < cv ? 1u : 0u);
+        return min(segs * mark_step(hot, kMarksOwned), hot);
+      };
+      auto prefix_rest = [&](const Head& h) -> uint32_t {
+        const uint32_t hot = h.a.y >> 16;
+        const uint32_t mk[3] = {h.b.y, h.b.z, h.b.w};
+        uint32_t segs = (h.b.x >> 16) < cv ? 1u : 0u;
+#pragma unroll
+        for (int t = 0; t < 3; t++) segs += ((mk[t] & 0xffffu) < cv ? 1u : 0u) + ((mk[t] >> 16) < cv ? 1u : 0u);
+        return min(segs * mark_step(hot, kMarksRest), hot);
+      };
+      const bool v_own = RANGE && owned(cl);  // uniform
       const bool cold = ch < cd && cv > kHot;  // cold ids below a cold v
-      const uint32_t st = x.a.x, len = x.a.y, label = x.b.w, n = prefix(x);  // the first 64 items
+      const uint32_t st = x.a.x, len = x.a.y, len2 = x.a.z, label = x.b.w, u0 = xu;  // the first 64 items
+      const uint32_t n = RANGE ? prefix_owned(x) : prefix(x);
+      const uint32_t n_rest = RANGE && (v_own || (u0 & kOwnedBit && u0 != kNoRank)) ? prefix_rest(x) : 0;
       uint32_t at_v = 0;  // PV: hits credited to v
       if (ch > 0)
         for (uint32_t i = 0; i < cd; i += kWave) {
@@ -950,10 +1127,13 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
           wave_lds_fence();
         }
       }
-      if (more) x = head(un);
+      if (more) {
+        x = head(un);
+        xu = un;
+      }
       auto items = [&](uint32_t e) -> uint32_t { return e + lane < cs1 ? part[e + lane] : kNoRank; };
       if (ch > 0) {
-        uint32_t acc = 0;
+        uint32_t acc = 0, acc_local = 0;
         auto probe = [&](const uint4 q, uint32_t item) {
           const uint32_t y[4] = {q.x, q.y, q.z, q.w};
           uint32_t found = 0;
@@ -963,8 +1143,14 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
             const uint32_t t0 = (lo >> (y[j] & 31)) & 1u, t1 = (hi >> ((y[j] >> 16) & 31)) & 1u;
             if constexpr (PV)
               found |= t0 << (2 * j) | t1 << (2 * j + 1);
+            else if constexpr (RANGE)
+              found += t0 + t1;
             else
               acc += t0 + t1;
+          }
+          if constexpr (RANGE) {
+            acc += found;
+            acc_local += found & s_pv.items.label[item];
           }
           if constexpr (PV) {
             acc += (uint32_t)__popc(found);
@@ -990,13 +1176,33 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
               atomicAdd(&s_pv.items.hits[item], rest);
           }
         };
-        Head y = cs0 + kWave < cs1 ? head(items(cs0 + kWave)) : Head{};
-        stream_lists<PV>(st, n, label, s_stream, s_items, lane, lists, 0xffffffffu, pv, probe);
+        // kRange: hits of owned ids are local where u or v is owned, those of the
+        // others (streamed only there) where both are.
+        auto stream = [&](uint32_t ss, uint32_t nn, uint32_t nr, uint32_t hot2, uint32_t ll, uint32_t ur) {
+          if constexpr (RANGE) {
+            const bool u_own = ur != kNoRank && (ur & kOwnedBit);
+            stream_lists<MODE>(ss, nn, v_own || u_own ? ~0u : 0u, s_stream, s_items, lane, lists, 0xffffffffu, pv, probe);
+            stream_lists<MODE>(ss + (hot2 & 0xffffu), nr, v_own && u_own ? ~0u : 0u, s_stream, s_items, lane, lists,
+                               0xffffffffu, pv, probe);
+          } else {
+            stream_lists<MODE>(ss, nn, ll, s_stream, s_items, lane, lists, 0xffffffffu, pv, probe);
+          }
+        };
+        uint32_t yu = kNoRank;
+        if (cs0 + kWave < cs1) yu = items(cs0 + kWave);
+        Head y = head(yu);
+        stream(st, n, n_rest, len, label, u0);
         for (uint32_t e = cs0 + kWave; e < cs1; e += kWave) {
-          const uint32_t sty = y.a.x, ny = prefix(y), ly = y.b.w;
-          if (e + kWave < cs1) y = head(items(e + kWave));
-          stream_lists<PV>(sty, ny, ly, s_stream, s_items, lane, lists, 0xffffffffu, pv, probe);
+          const uint32_t sty = y.a.x, leny = y.a.y, ly = y.b.w, uy = yu;
+          const uint32_t ny = RANGE ? prefix_owned(y) : prefix(y);
+          const uint32_t nry = RANGE && (v_own || (uy & kOwnedBit && uy != kNoRank)) ? prefix_rest(y) : 0;
+          if (e + kWave < cs1) {
+            yu = items(e + kWave);
+            y = head(yu);
+          }
+          stream(sty, ny, nry, leny, ly, uy);
         }
+        local += acc_local;
         hits += acc;
         wave_lds_fence();
         if constexpr (PV)
@@ -1018,7 +1224,7 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
         wave_lds_fence();
       }
       if (cold) {
-        uint32_t acc = 0;
+        uint32_t acc = 0, acc_local = 0;
         // Cold ids [first, first + room) of N(v), in row order, hashed.
         auto pass = [&](auto logb, uint32_t first, uint32_t room) {
           constexpr int L = decltype(logb)::value;
@@ -1046,6 +1252,7 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
               if (spl && !hit && bucket_spilled(t[j]) && y[j] != -1)
                 hit = wave_tab_continue<L>(s_tab, wave_bucket<L>(y[j]), y[j]);
               acc += hit ? 1u : 0u;
+              if constexpr (RANGE) acc_local += hit ? s_pv.items.label[item] & 1u : 0u;
               if constexpr (PV) {
                 if (hit) {
                   const uint32_t lu = s_pv.items.label[item], lw = orig[y[j]];
@@ -1059,16 +1266,28 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
               }
             }
           };
-          stream_lists<PV>(st + (len & 0xffffu), len >> 16, label, s_stream, s_items, lane, lists, kNoRank, pv, probe);
+          auto stream = [&](uint32_t ss, uint32_t l1, uint32_t l2, uint32_t ll, uint32_t ur) {
+            if constexpr (RANGE) {
+              const bool u_own = ur != kNoRank && (ur & kOwnedBit);
+              const uint32_t c0 = ss + (l1 & 0xffffu) + (l1 >> 16);  // behind both hot parts
+              stream_lists<MODE>(c0, l2 & 0xffffu, v_own || u_own ? ~0u : 0u, s_stream, s_items, lane, lists, kNoRank, pv, probe);
+              stream_lists<MODE>(c0 + (l2 & 0xffffu), v_own || u_own ? l2 >> 16 : 0, v_own && u_own ? ~0u : 0u, s_stream,
+                                 s_items, lane, lists, kNoRank, pv, probe);
+            } else {
+              stream_lists<MODE>(ss + (l1 & 0xffffu), l1 >> 16, ll, s_stream, s_items, lane, lists, kNoRank, pv, probe);
+            }
+          };
+          stream(st, len, len2, label, u0);
           for (uint32_t e = cs0 + kWave; e < cs1; e += kWave) {
             const uint32_t ur = items(e);
-            uint2 y = make_uint2(0, 0);
+            uint4 y = make_uint4(0, 0, 0, 0);
             uint32_t ly = 0;
             if (ur != kNoRank) {
-              y = *reinterpret_cast<const uint2*>(rec + ur);
-              if constexpr (PV) ly = rec[ur].mark[5];
+              const RankRec* q = rec + strip(ur);
+              y = *reinterpret_cast<const uint4*>(q);
+              if constexpr (PV) ly = q->mark[5];
             }
-            stream_lists<PV>(y.x + (y.y & 0xffffu), y.y >> 16, ly, s_stream, s_items, lane, lists, kNoRank, pv, probe);
+            stream(y.x, y.y, y.z, ly, ur);
           }
           wave_lds_fence();
           clear_words(1 << L);
@@ -1081,6 +1300,7 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
           for (uint32_t f = 0; f < ncold; f += 2u << kColdBig) pass(std::integral_constant<int, kColdBig>{}, f, 2u << kColdBig);
         }
         hits += acc;
+        local += acc_local;
       }
       if constexpr (PV) {
         const uint64_t t = wave_sum_u64(at_v);
@@ -1090,7 +1310,11 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
     }
   }
   hits = wave_sum_u64(hits);
-  if (lane == 0) add_sum(counters, kSumTotal, hits);
+  if (lane == 0) add_sum(counters, RANGE ? kSumOwned : kSumTotal, hits);
+  if constexpr (RANGE) {
+    local = wave_sum_u64(local);
+    if (lane == 0) add_sum(counters, kSumLocal, local);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1102,12 +1326,12 @@ static unsigned rank_grid(int64_t n, int per, int64_t cap) {
 
 // Room for the lists of a simple graph, in 128-byte lines: |E+| = ne / 2 ids; a
 // list of d >= 2 ids is given at most min(d, d / 4 + 9.25) chunks (hot and cold
-// parts rounded up to chunks, then to list_room), a wave's lists at a time
+// parts rounded up to chunks, then to list_room; two parts each: d / 4 + 11.5), a wave's lists at a time
 // rounded up to a line.  Grants but a wave's last are used to three quarters.
 // A region is left for the next when a request does not fit, so each may lose
 // one request: a grant, or 64 of the longest lists (at most 1.02 sqrt(ne) ids,
 // since out-neighbours have about the vertex's degree or more).
-static ListRoom rank_list_room(const xt_ctx* ctx, int64_t nv, int64_t ne, bool by_label, int64_t* lines) {
+static ListRoom rank_list_room(const xt_ctx* ctx, int64_t nv, int64_t ne, bool by_label, int parts, int64_t* lines) {
   ListRoom r;
   const int64_t waves = (int64_t)ctx->num_cus * 16;
   r.rows = kWave;
@@ -1117,12 +1341,13 @@ static ListRoom rank_list_room(const xt_ctx* ctx, int64_t nv, int64_t ne, bool b
   r.together = nv <= (1ll << 22) ? 2 : 4;
   r.nbatch = (nv + r.rows - 1) / r.rows;
   const int64_t nlists = nv < ne / 4 ? nv : ne / 4;
-  const int64_t chunks = ne / 8 + 10 * nlists < ne / 2 ? ne / 8 + 10 * nlists : ne / 2;
+  const int64_t chunks = parts == 4 ? ne / 8 + 12 * nlists
+                         : ne / 8 + 10 * nlists < ne / 2 ? ne / 8 + 10 * nlists : ne / 2;
   const int64_t need = chunks / 8 + r.nbatch + 1;
   const int64_t grant = need / (waves * 32) < 8 ? 8 : need / (waves * 32);
   const int64_t used = need + need / 3 + (r.nbatch < waves ? r.nbatch : waves) * grant;
   const double longest = by_label ? (double)nv : 1.05 * std::sqrt((double)ne) + 64.0;
-  const int64_t most = grant + (int64_t)(64.0 * (longest / 4 + 10) / 8) + 1;
+  const int64_t most = grant + (int64_t)(64.0 * (longest / 4 + 12) / 8) + 1;
   r.grant = (uint64_t)grant;
   r.region = (uint64_t)(used / kListShards + most + 1);
   *lines = (int64_t)r.region * kListShards;
@@ -1138,7 +1363,7 @@ bool rank_fits(const xt_ctx* ctx, int64_t nv, int64_t ne, int mode) {
   const bool by_label = mode == kOrientId;
   if (nv >= (by_label ? kLabelRankMax : 1ll << 30) || ne >= (1ll << 32)) return false;
   int64_t lines;
-  rank_list_room(ctx, nv, ne, by_label, &lines);
+  rank_list_room(ctx, nv, ne, by_label, 4, &lines);
   return lines < (1ll << 29);
 }
 
@@ -1151,7 +1376,7 @@ static int64_t rank_chunk(const xt_ctx* ctx, int64_t ne) {
 
 template <typename T>
 int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* off, const T* tails, int mode,
-               uint64_t* pv, hipStream_t st, hipEvent_t split_done) {
+               uint64_t* pv, const OwnedRange* range, hipStream_t st, hipEvent_t split_done) {
   const int64_t S = rank_chunk(ctx, ne);
   const int64_t nch = (ne + S - 1) / S, nchunks = (ne + kChunk - 1) / kChunk;
   XT_TRY(ensure(ctx, s.crows, (size_t)(2 * nch) * sizeof(int32_t)));
@@ -1160,10 +1385,13 @@ int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* o
   XT_TRY(ensure(ctx, s.itcnt, (size_t)nv * sizeof(uint32_t)));
   XT_TRY(ensure(ctx, s.rpart, (size_t)(ne + kWave) * sizeof(uint32_t)));  // a wave reads past a short row
   int64_t lines;
-  const ListRoom lr = rank_list_room(ctx, nv, ne, mode == kOrientId, &lines);
+  const ListRoom lr = rank_list_room(ctx, nv, ne, mode == kOrientId, range ? 4 : 2, &lines);
   XT_TRY(ensure(ctx, s.rlists, (size_t)lines * 128));
   XT_TRY(ensure(ctx, s.rrec, (size_t)nv * sizeof(RankRec)));
   XT_TRY(ensure(ctx, s.rhist, (size_t)(2 * kRankClasses) * sizeof(uint32_t)));
+  if (range) XT_TRY(ensure(ctx, s.vrec, (size_t)nv * sizeof(uint64_t)));
+  uint64_t* oc1 = range ? s.vrec.as<uint64_t>() : nullptr;
+  const int64_t rlo = range ? range->lo : 0, rhi = range ? range->hi : 0;
   if (pv) XT_TRY(ensure(ctx, s.rorig, (size_t)nv * sizeof(uint32_t)));
   uint32_t* orig = pv ? s.rorig.as<uint32_t>() : nullptr;
   unsigned long long* pvp = reinterpret_cast<unsigned long long*>(pv);
@@ -1177,7 +1405,7 @@ int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* o
   RankRec* rec = s.rrec.as<RankRec>();
   XT_TRY(fill_u32(ctx, hist, 2 * kRankClasses, 0u, st));
   hipLaunchKernelGGL(k_rank_prep, dim3(rank_grid(nv, 1024, 8192)), dim3(256), 0, st, nv, ne, off, S, crows, oc,
-                     s.itcnt.as<uint32_t>(), hist, pvp);
+                     s.itcnt.as<uint32_t>(), hist, pvp, oc1);
   XT_HIP(ctx, hipGetLastError());
   if (mode == kOrientId)
     hipLaunchKernelGGL(k_rank_by_label, dim3(rank_grid(nv, 256, 8192)), dim3(256), 0, st, nv, rank, orig);
@@ -1185,29 +1413,39 @@ int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* o
     hipLaunchKernelGGL(k_rank_assign, dim3(rank_grid(nv, 256 * kAssignRun, 1ll << 31)), dim3(256), 0, st, nv, off,
                        (const uint32_t*)hist, hist + kRankClasses, rank, orig);
   XT_HIP(ctx, hipGetLastError());
-  hipLaunchKernelGGL((k_rank_split<T>), dim3(xcd_grid(nchunks)), dim3(kBlock), 0, st, nv, ne, off, tails,
-                     (const uint32_t*)rank, (const int32_t*)crows, (int)(kChunk / S), part, oc,
-                     s.itcnt.as<uint32_t>(), counters);
+#define XT_RANK_SPLIT(R)                                                                                             \
+  hipLaunchKernelGGL((k_rank_split<T, R>), dim3(xcd_grid(nchunks)), dim3(kBlock), 0, st, nv, ne, off, tails,            \
+                     (const uint32_t*)rank, (const int32_t*)crows, (int)(kChunk / S), part, oc,                       \
+                     s.itcnt.as<uint32_t>(), counters, oc1, rlo, rhi)
+  if (range)
+    XT_RANK_SPLIT(true);
+  else
+    XT_RANK_SPLIT(false);
+#undef XT_RANK_SPLIT
   XT_HIP(ctx, hipGetLastError());
   const dim3 lgrid(rank_grid(lr.nbatch, 1, (int64_t)ctx->num_cus * 16));
-#define XT_RANK_LISTS(PV)                                                                                           \
-  hipLaunchKernelGGL((k_rank_lists<PV>), lgrid, dim3(64), 0, st, nv, off, (const uint64_t*)oc, (const uint32_t*)rank, \
-                     (const uint32_t*)part, lr, lists, rec, counters)
+#define XT_RANK_LISTS(M)                                                                                             \
+  hipLaunchKernelGGL((k_rank_lists<M>), lgrid, dim3(64), 0, st, nv, off, (const uint64_t*)oc, (const uint64_t*)oc1,     \
+                     (const uint32_t*)rank, (const uint32_t*)part, lr, lists, rec, counters)
   if (pv)
-    XT_RANK_LISTS(true);
+    XT_RANK_LISTS(kPerVertex);
+  else if (range)
+    XT_RANK_LISTS(kRange);
   else
-    XT_RANK_LISTS(false);
+    XT_RANK_LISTS(kTotal);
 #undef XT_RANK_LISTS
   XT_HIP(ctx, hipGetLastError());
   if (split_done) XT_HIP(ctx, hipEventRecord(split_done, st));
-#define XT_RANK_COUNT(PV)                                                                                            \
-  hipLaunchKernelGGL((k_rank_count<PV>), dim3((unsigned)nch), dim3(64), 0, st, nv, ne, off, (const uint32_t*)rank,     \
+#define XT_RANK_COUNT(M)                                                                                             \
+  hipLaunchKernelGGL((k_rank_count<M>), dim3((unsigned)nch), dim3(64), 0, st, nv, ne, off, (const uint32_t*)rank,       \
                      (const uint64_t*)oc, (const uint32_t*)part, (const RankRec*)rec, (const uint4*)lists,            \
-                     (const int32_t*)crows, S, counters, (const uint32_t*)orig, pvp)
+                     (const int32_t*)crows, S, counters, (const uint32_t*)orig, pvp, rlo, rhi)
   if (pv)
-    XT_RANK_COUNT(true);
+    XT_RANK_COUNT(kPerVertex);
+  else if (range)
+    XT_RANK_COUNT(kRange);
   else
-    XT_RANK_COUNT(false);
+    XT_RANK_COUNT(kTotal);
 #undef XT_RANK_COUNT
   XT_HIP(ctx, hipGetLastError());
   ctx->rank_chunks = nch;
@@ -1215,8 +1453,8 @@ int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* o
 }
 
 template int rank_count<int32_t>(xt_ctx*, Scratch&, int64_t, int64_t, const int64_t*, const int32_t*, int, uint64_t*,
-                                 hipStream_t, hipEvent_t);
+                                 const OwnedRange*, hipStream_t, hipEvent_t);
 template int rank_count<int64_t>(xt_ctx*, Scratch&, int64_t, int64_t, const int64_t*, const int64_t*, int, uint64_t*,
-                                 hipStream_t, hipEvent_t);
+                                 const OwnedRange*, hipStream_t, hipEvent_t);
 
 }  // namespace xt

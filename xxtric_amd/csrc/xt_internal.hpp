@@ -178,17 +178,17 @@ template <typename T>
 int orient(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* off, const T* tails, int mode,
            hipStream_t st);
 
+// Owned vertex range [lo, hi) of a credit-by-range count.
+struct OwnedRange {
+  int64_t lo, hi;
+};
+
 // Intersection + reduction over the context's oriented CSR.  Adds the global
 // count to the sum kSumTotal; per-vertex counts into pv when pv != nullptr.
 // Batch mode: gid (graph of each vertex) and gtotal (per-graph totals) non-null
 // and the intersection kernel drains a device tile queue with a fixed grid.
 // evs (nullable): two events recorded after the light-edge kernel and after
 // the item lists are built.
-// Owned vertex range [lo, hi) of a credit-by-range count.
-struct OwnedRange {
-  int64_t lo, hi;
-};
-
 template <typename T>
 int count_oriented(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne_bound, const int64_t* in_off,
                    const T* in_tails, uint64_t* pv, const int32_t* gid, uint64_t* gtotal,
@@ -224,14 +224,14 @@ struct RankUse {
   int64_t max_degree;
 };
 
-// The total (pv == nullptr) or the per-vertex counts (and the total) of one
-// graph counted in rank space: adds to the sums kSumTotal and kSumEdges and
-// writes pv[nv].  split_done (nullable) is recorded once the lists stand.  Only
+// The total, the per-vertex counts (pv != nullptr: pv[nv] is written) or an
+// owned range of one graph counted in rank space: adds to the sums kSumTotal
+// (an owned range: kSumOwned and kSumLocal) and kSumEdges.  split_done (nullable) is recorded once the lists stand.  Only
 // for sizes that rank_fits() accepts.
 bool rank_fits(const xt_ctx* ctx, int64_t nv, int64_t ne, int mode);
 template <typename T>
 int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* off, const T* tails, int mode,
-               uint64_t* pv, hipStream_t st, hipEvent_t split_done);
+               uint64_t* pv, const OwnedRange* range, hipStream_t st, hipEvent_t split_done);
 
 // Whole single-graph count on the device (orientation + intersection).
 // rank: whether it may be counted in rank space, and the longest row (-1: unknown).
