@@ -26,7 +26,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 CXX = os.environ.get("CXX", "g++")
 ARCH = "gfx950"
 
-HIP_SOURCES = ["api.hip", "orient.hip", "count.hip", "rank.hip", "gen.hip", "batch.hip", "serve.hip"]
+HIP_SOURCES = ["api.hip", "orient.hip", "count.hip", "rank.hip", "gen.hip", "batch.hip", "batch_count.hip", "serve.hip"]
 HOST_SOURCES = ["ingest.cpp", "partition.cpp"]
 
 HIP_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC", "-Wall",

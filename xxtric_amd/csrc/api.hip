@@ -163,6 +163,11 @@ static int check_host_offsets(xt_ctx* ctx, int64_t nv, int64_t ne, const int64_t
   return XT_OK;
 }
 
+bool edge_tile_knobs(const xt_ctx* ctx) {
+  return ctx->small_cut != 0 || ctx->wave_owner != -1 || ctx->group_blocks != 4 || ctx->group_round != 2 ||
+         ctx->group_hash != kHashMix || ctx->items_per_tile != 256 || ctx->tile_run != 16 || ctx->force_wide;
+}
+
 // Per-vertex counts go to rank space below this many entries: the credit of
 // every hit there costs more than in the edge tiles' hash table, the rest less
 // (ms, rank space against edge tiles: R-MAT s14 0.11 and 0.40, s18 0.88 and
@@ -182,10 +187,7 @@ constexpr int64_t kRankIdDegree = 256;
 static bool ranks(const xt_ctx* ctx, int64_t nv, int64_t ne, int mode, bool per_vertex, int64_t max_degree) {
   if (mode == kOrientId && (max_degree < 0 || max_degree > kRankIdDegree)) return false;
   if (per_vertex && ne >= kRankPvEntries) return false;
-  const bool knobs = ctx->small_cut != 0 || ctx->wave_owner != -1 || ctx->group_blocks != 4 || ctx->group_round != 2 ||
-                     ctx->group_hash != kHashMix || ctx->items_per_tile != 256 || ctx->tile_run != 16 ||
-                     ctx->force_wide;
-  return !knobs && ne > 0 && rank_fits(ctx, nv, ne, mode);
+  return !edge_tile_knobs(ctx) && ne > 0 && rank_fits(ctx, nv, ne, mode);
 }
 
 template <typename T>

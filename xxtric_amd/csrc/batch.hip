@@ -3,12 +3,16 @@
 // Layout in HBM.  The graphs of a batch are stored twice:
 //   * union form: one block-diagonal CSR over all graphs (graph g owns vertex
 //     ids [vbase_g, vbase_g + nv_g) and entries [ebase_g, ebase_g + ne_g)),
-//     plus gid[v] = graph of vertex v.  The ordinary orientation kernels and
-//     the persistent intersection kernel run over it once, whatever the number
-//     of graphs: a tile (2048 oriented edges) maps to a (graph, edge range)
-//     piece of the batch, tiles are drawn from a device work queue, short-list
-//     edges are intersected by threads and long-list edges are binned to the
-//     wave-per-edge kernel.  Per-graph totals are reduced in LDS per tile.
+//     plus gid[v] = graph of vertex v and gbase[g] = vbase_g.  A batch whose
+//     graphs have at most 65,535 vertices is counted by the three kernels of
+//     batch_count.hip.  One with a larger graph, or with a knob of the edge
+//     tiles set, takes the single-graph pipeline over the union: the ordinary
+//     orientation kernels and the persistent intersection kernel run over it
+//     once, whatever the number of graphs: a tile (2048 oriented edges) maps to
+//     a (graph, edge range) piece of the batch, tiles are drawn from a device
+//     work queue, short-list edges are intersected by threads and long-list
+//     edges are binned to the wave-per-edge kernel.  Per-graph totals are
+//     reduced in LDS per tile.
 //   * local form: each graph's own CSR (ids 0..nv_g-1), used by the baseline
 //     that launches the single-graph pipeline once per graph.
 // All scratch is sized at creation so the pipeline can be captured once as a
@@ -29,12 +33,14 @@ int gen_er_rows(xt_ctx* ctx, Scratch& s, int64_t n, uint64_t seed, uint64_t thr6
                 int32_t* tails, int64_t cap, int64_t* ne_out, hipStream_t st);
 
 __global__ __launch_bounds__(256) void k_rebase(int64_t nv, int64_t ne, int64_t vbase, int64_t ebase,
-                                                int32_t g, const int64_t* __restrict__ loff,
+                                                int32_t g, int32_t* __restrict__ gbase,
+                                                const int64_t* __restrict__ loff,
                                                 const int32_t* __restrict__ ltails,
                                                 int64_t* __restrict__ goff, int32_t* __restrict__ gtails,
                                                 int32_t* __restrict__ gid) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   const int64_t n = nv + 1 > ne ? nv + 1 : ne;
+  if (blockIdx.x == 0 && threadIdx.x == 0) gbase[g] = (int32_t)vbase;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
     if (i <= nv) goff[vbase + i] = ebase + loff[i];
     if (i < nv) gid[vbase + i] = g;
@@ -50,6 +56,7 @@ constexpr int kRecWords = 6;
 constexpr int kRebaseRun = 8;
 
 __global__ __launch_bounds__(256) void k_rebase_many(int64_t ng, int64_t total, int32_t g0,
+                                                     int32_t* __restrict__ gbase,
                                                      const int64_t* __restrict__ rec,
                                                      const int64_t* __restrict__ loff,
                                                      const int32_t* __restrict__ ltails,
@@ -74,6 +81,7 @@ __global__ __launch_bounds__(256) void k_rebase_many(int64_t ng, int64_t total, 
       const int64_t* r = rec + j * kRecWords;
       const int64_t nv = r[0], ne = r[1], vbase = r[2], ebase = r[3], lobase = r[4];
       const int64_t k = i - r[5];
+      if (k == 0) gbase[g0 + (int32_t)j] = (int32_t)vbase;
       if (k <= nv) goff[vbase + k] = ebase + loff[lobase + k];
       if (k < nv) gid[vbase + k] = g0 + (int32_t)j;
       if (k < ne) gtails[ebase + k] = (int32_t)(vbase + ltails[ebase + k]);
@@ -102,6 +110,8 @@ struct xt_batch {
   int64_t* goff = nullptr;
   int32_t* gtails = nullptr;
   int32_t* gid = nullptr;
+  int32_t* gbase = nullptr;  // first vertex of each graph
+  int64_t max_nv = 0;        // vertices of the largest graph
   int64_t* loff = nullptr;
   int32_t* ltails = nullptr;
   uint64_t* gtotal = nullptr;
@@ -120,6 +130,7 @@ struct xt_batch {
   int exec_tile_run = -1;
   int exec_wave_owner = -2;
   int exec_group_hash = 0;
+  bool exec_small = false;
   // pinned host mirror of the local arena for staged host adds
   int64_t* h_loff = nullptr;
   int32_t* h_ltails = nullptr;
@@ -140,7 +151,7 @@ static void batch_free(xt_batch* b) {
   if (b->stream) (void)hipStreamSynchronize(b->stream);
   if (b->exec) (void)hipGraphExecDestroy(b->exec);
   if (b->graph) (void)hipGraphDestroy(b->graph);
-  void* ps[] = {b->goff, b->gtails, b->gid, b->loff, b->ltails, b->gtotal, b->ptotal, b->d_rec};
+  void* ps[] = {b->goff, b->gtails, b->gid, b->gbase, b->loff, b->ltails, b->gtotal, b->ptotal, b->d_rec};
   for (void* p : ps)
     if (p) (void)hipFree(p);
   void* hs[] = {b->h_loff, b->h_ltails, b->h_rec, b->h_totals};
@@ -170,11 +181,12 @@ static int batch_commit(xt_batch* b, int64_t nv, int64_t ne) {
   if (grid > 4096) grid = 4096;
   if (grid < 1) grid = 1;
   hipLaunchKernelGGL(k_rebase, dim3((unsigned)grid), dim3(256), 0, b->stream, nv, ne, rec.vbase,
-                     rec.ebase, g, (const int64_t*)(b->loff + rec.lobase),
+                     rec.ebase, g, b->gbase, (const int64_t*)(b->loff + rec.lobase),
                      (const int32_t*)(b->ltails + rec.ebase), b->goff, b->gtails, b->gid);
   XT_HIP(b->ctx, hipGetLastError());
   b->graphs.push_back(rec);
   b->V += nv;
+  if (nv > b->max_nv) b->max_nv = nv;
   b->E += ne;
   b->LO += nv + 1;
   b->pend_g = (int64_t)b->graphs.size();
@@ -223,7 +235,7 @@ static int batch_flush(xt_batch* b) {
   int64_t grid = (work + 256 * kRebaseRun - 1) / (256 * kRebaseRun);
   if (grid > 8192) grid = 8192;
   hipLaunchKernelGGL(k_rebase_many, dim3((unsigned)grid), dim3(256), 0, b->stream, ng, work,
-                     (int32_t)b->pend_g, (const int64_t*)b->d_rec, (const int64_t*)b->loff,
+                     (int32_t)b->pend_g, b->gbase, (const int64_t*)b->d_rec, (const int64_t*)b->loff,
                      (const int32_t*)b->ltails, b->goff, b->gtails, b->gid);
   XT_HIP(ctx, hipGetLastError());
   XT_HIP(ctx, hipEventRecord(b->ev_stage, b->stream));
@@ -232,12 +244,19 @@ static int batch_flush(xt_batch* b) {
   return XT_OK;
 }
 
+// Whether every graph's ids fit 16 bits and no knob asks for the edge tiles.
+static bool batch_is_small(const xt_batch* b) {
+  return !edge_tile_knobs(b->ctx) && batch_small_fits(b->max_nv, b->E);
+}
+
 // Launches the union pipeline on the batch stream (no synchronisation).
 static int batch_pipeline(xt_batch* b, uint32_t flags) {
   xt_ctx* ctx = b->ctx;
   hipStream_t st = b->stream;
   const int mode = (flags & XT_ORIENT_ID) ? kOrientId : kOrientDegree;
   const int64_t G = (int64_t)b->graphs.size();
+  if (batch_is_small(b))
+    return batch_small_count(ctx, b->s, b->V, b->E, G, b->goff, b->gtails, b->gid, b->gbase, b->gtotal, mode, st);
   XT_TRY(fill_u64(ctx, b->s.counters.as<uint64_t>(), kNumSlots, 0, st));
   XT_TRY(fill_u64(ctx, b->gtotal, G, 0, st));
   XT_TRY(orient<int32_t>(ctx, b->s, b->V, b->E, b->goff, b->gtails, mode, st));
@@ -264,7 +283,8 @@ int batch_launch(xt_batch* b, int mode, uint32_t flags) {
         b->exec_flags != flags || b->exec_small_cut != ctx->small_cut ||
         b->exec_group_blocks != ctx->group_blocks || b->exec_group_round != ctx->group_round ||
         b->exec_items_per_tile != ctx->items_per_tile || b->exec_tile_run != ctx->tile_run ||
-        b->exec_wave_owner != ctx->wave_owner || b->exec_group_hash != ctx->group_hash) {
+        b->exec_wave_owner != ctx->wave_owner || b->exec_group_hash != ctx->group_hash ||
+        b->exec_small != batch_is_small(b)) {
       if (b->exec) {
         XT_HIP(ctx, hipGraphExecDestroy(b->exec));
         b->exec = nullptr;
@@ -295,6 +315,7 @@ int batch_launch(xt_batch* b, int mode, uint32_t flags) {
       b->exec_tile_run = ctx->tile_run;
       b->exec_wave_owner = ctx->wave_owner;
       b->exec_group_hash = ctx->group_hash;
+      b->exec_small = batch_is_small(b);
     }
     XT_HIP(ctx, hipEventRecord(b->ev0, st));
     XT_HIP(ctx, hipGraphLaunch(b->exec, st));
@@ -416,6 +437,7 @@ int batch_stage_host(xt_batch* b, int64_t nv, int64_t ne, const int64_t* off, co
   if (ne > 0) std::memcpy(b->h_ltails + b->E, tails, (size_t)ne * sizeof(int32_t));
   b->graphs.push_back(BatchGraph{nv, ne, b->V, b->E, b->LO});
   b->V += nv;
+  if (nv > b->max_nv) b->max_nv = nv;
   b->E += ne;
   b->LO += nv + 1;
   return XT_OK;
@@ -431,6 +453,7 @@ int batch_stage_layout(xt_batch* b, int64_t nv, int64_t ne, int64_t** off_dst, i
   *tails_dst = b->h_ltails + b->E;
   b->graphs.push_back(BatchGraph{nv, ne, b->V, b->E, b->LO});
   b->V += nv;
+  if (nv > b->max_nv) b->max_nv = nv;
   b->E += ne;
   b->LO += nv + 1;
   return XT_OK;
@@ -449,6 +472,7 @@ const char* batch_stage_host_checked(xt_batch* b, int64_t nv, int64_t ne, const 
   if (bad) return bad;
   b->graphs.push_back(BatchGraph{nv, ne, b->V, b->E, b->LO});
   b->V += nv;
+  if (nv > b->max_nv) b->max_nv = nv;
   b->E += ne;
   b->LO += nv + 1;
   return nullptr;
@@ -484,6 +508,7 @@ int xt_batch_create(xt_ctx* ctx, int64_t max_vertices, int64_t max_edges, int64_
     if (e == hipSuccess) e = hipMalloc(&b->goff, (size_t)(max_vertices + 1) * sizeof(int64_t));
     if (e == hipSuccess) e = hipMalloc(&b->gtails, (size_t)max_edges * sizeof(int32_t));
     if (e == hipSuccess) e = hipMalloc(&b->gid, (size_t)max_vertices * sizeof(int32_t));
+    if (e == hipSuccess) e = hipMalloc(&b->gbase, (size_t)max_graphs * sizeof(int32_t));
     if (e == hipSuccess) e = hipMalloc(&b->loff, (size_t)(max_vertices + max_graphs) * sizeof(int64_t));
     if (e == hipSuccess) e = hipMalloc(&b->ltails, (size_t)max_edges * sizeof(int32_t));
     if (e == hipSuccess) e = hipMalloc(&b->gtotal, (size_t)max_graphs * sizeof(uint64_t));
@@ -494,6 +519,7 @@ int xt_batch_create(xt_ctx* ctx, int64_t max_vertices, int64_t max_edges, int64_
       return rc;
     }
     int rc = reserve(ctx, b->s, max_vertices, max_edges, false);
+    if (rc == XT_OK) rc = batch_small_reserve(ctx, b->s, max_vertices, max_edges);
     if (rc == XT_OK) rc = fill_u64(ctx, b->s.counters.as<uint64_t>(), kNumSlots, 0, b->stream);
     if (rc == XT_OK) {
       e = hipMemsetAsync(b->goff, 0, sizeof(int64_t), b->stream);
@@ -643,6 +669,7 @@ int xt_batch_clear(xt_batch* b) {
     XT_TRY(batch_stage_idle(b));
     b->graphs.clear();
     b->V = b->E = b->LO = 0;
+    b->max_nv = 0;
     b->pend_g = 0;
     return XT_OK;
   });

@@ -193,6 +193,16 @@ template <typename T>
 int count_oriented(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne_bound, const int64_t* in_off,
                    const T* in_tails, uint64_t* pv, const int32_t* gid, uint64_t* gtotal,
                    hipStream_t st, hipEvent_t* evs, const OwnedRange* range = nullptr);
+// The per-graph totals of a batch whose graphs have at most 65,535 vertices
+// (batch_small_fits): gbase[g] is the first vertex of graph g.
+bool batch_small_fits(int64_t max_graph_vertices, int64_t ne);
+int batch_small_reserve(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne);
+int batch_small_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, int64_t ng, const int64_t* off,
+                      const int32_t* tails, const int32_t* gid, const int32_t* gbase, uint64_t* gtotal, int mode,
+                      hipStream_t st);
+// Whether a knob of the edge tiles is away from its default: counts then use them.
+bool edge_tile_knobs(const xt_ctx* ctx);
+
 // Sums of min(d+(u), d+(v)) over the oriented edges of s (all, and those whose
 // longer list exceeds `cut`: 0 = the context's light cut for one graph).
 int alg_stats(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne_bound, hipStream_t st, int cut = 0);
