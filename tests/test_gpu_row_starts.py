@@ -38,3 +38,20 @@ def test_row_starts(ctx, nv, where):
     keys = np.unique(a * nv + b)
     assert (tails.astype(np.int64) == keys % nv).all() and len(tails) == len(keys)
     assert (np.asarray(off) == np.searchsorted(keys, np.arange(nv + 1, dtype=np.int64) * nv)).all()
+
+
+def test_builds_share_memory(ctx):
+    """Counts of edge lists on both sides of the memory that a context keeps for
+    builds, between graphs that outlive them."""
+    rng = np.random.default_rng(4)
+    kept = []
+    for nv, m in ((1000, 6000), (50, 0), (300_000, 900_000), (1000, 5000), (1 << 20, 9_000_000), (70_000, 400_000)):
+        u, v = rng.integers(0, nv, (2, m))
+        _say(nv, m)
+        total = ctx.count_edges(nv, u, v)
+        g = ctx.graph_from_edges(nv, u, v)
+        assert g.count() == total
+        kept.append((g, total))
+    for g, total in kept:
+        assert g.count() == total
+        g.close()

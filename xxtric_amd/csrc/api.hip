@@ -363,6 +363,7 @@ int xt_ctx_destroy(xt_ctx* ctx) {
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     release(ctx->s);
+    if (ctx->build.p) (void)hipFree(ctx->build.p);
     for (int i = 0; i < kNumEv; i++)
       if (ctx->ev[i]) (void)hipEventDestroy(ctx->ev[i]);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
@@ -770,6 +771,12 @@ int xt_graph_er(xt_ctx* ctx, int64_t n, uint64_t seed, uint64_t thr64, xt_graph*
   });
 }
 
+static int check_edges(xt_ctx* ctx, int64_t nv, int64_t m, const int64_t* src, const int64_t* dst) {
+  if (nv < 1 || nv >= (1LL << 31) - 1 || m < 0 || (m > 0 && (!src || !dst)))
+    return set_err(ctx, XT_ERR_ARG, "edge list: need 1 <= nv < 2^31-1, m >= 0 and both id arrays");
+  return XT_OK;
+}
+
 int xt_graph_from_edges(xt_ctx* ctx, int64_t nv, int64_t m, const int64_t* src, const int64_t* dst,
                         xt_graph** out) {
   return xt_guarded([&]() -> int {
@@ -777,10 +784,9 @@ int xt_graph_from_edges(xt_ctx* ctx, int64_t nv, int64_t m, const int64_t* src, 
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     XT_HIP(ctx, hipSetDevice(ctx->device));
     *out = nullptr;
-    if (nv < 1 || nv >= (1LL << 31) - 1 || m < 0 || (m > 0 && (!src || !dst)))
-      return set_err(ctx, XT_ERR_ARG, "edge list: need 1 <= nv < 2^31-1, m >= 0 and both id arrays");
+    XT_TRY(check_edges(ctx, nv, m, src, dst));
     xt_graph* g = new xt_graph();
-    const int rc = graph_from_edges(ctx, nv, m, src, dst, g);
+    const int rc = graph_from_edges(ctx, nv, m, src, dst, false, g);
     if (rc != XT_OK) {
       if (g->off) (void)hipFree(g->off);
       if (g->tails) (void)hipFree(g->tails);
@@ -922,10 +928,15 @@ int xt_count_edges(xt_ctx* ctx, int64_t nv, int64_t m, const int64_t* src, const
   return xt_guarded([&]() -> int {
     if (!ctx || !total) return XT_ERR_ARG;
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
-    xt_graph* g = nullptr;
-    XT_TRY(xt_graph_from_edges(ctx, nv, m, src, dst, &g));
-    const int rc = xt_graph_count(ctx, g, flags, total, per_vertex);
-    xt_graph_destroy(ctx, g);
+    XT_HIP(ctx, hipSetDevice(ctx->device));
+    XT_TRY(check_edges(ctx, nv, m, src, dst));
+    xt_graph g;
+    int rc = graph_from_edges(ctx, nv, m, src, dst, true, &g);
+    if (rc == XT_OK) rc = xt_graph_count(ctx, &g, flags, total, per_vertex);
+    if (!g.lent) {
+      if (g.off) (void)hipFree(g.off);
+      if (g.tails) (void)hipFree(g.tails);
+    }
     return rc;
   });
 }

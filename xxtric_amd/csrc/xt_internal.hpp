@@ -131,6 +131,7 @@ struct xt_ctx {
   std::string err;
   std::recursive_mutex mu;
   xt::Scratch s;
+  xt::DevBuf build;  // memory of graph builds (stream's work only)
   hipEvent_t ev[xt::kNumEv] = {};
   xt_timing timing = {};
   // Light edges: both out-lists at most this long; 0 picks kLightCut for one
@@ -155,6 +156,7 @@ struct xt_graph {
   int64_t* off = nullptr;   // int64[nv+1]
   int32_t* tails = nullptr; // int32[ne]
   int64_t max_degree = -1;  // longest row where the host has seen the offsets, else -1
+  bool lent = false;        // off and tails lie in the context's build memory
 };
 
 namespace xt {
@@ -255,7 +257,10 @@ int gen_rmat(xt_ctx* ctx, int scale, int edgefactor, const uint32_t thr[3], uint
              int permute, xt_graph* g);
 int gen_er(xt_ctx* ctx, int64_t n, uint64_t seed, uint64_t thr64, xt_graph* g);
 // Edge list (host pairs) -> symmetric, merged, self-loop-free CSR on the device.
-int graph_from_edges(xt_ctx* ctx, int64_t nv, int64_t m, const int64_t* src, const int64_t* dst, xt_graph* g);
+// With `borrow` g's arrays may lie in the context's build memory (g->lent), valid
+// until its next build.
+int graph_from_edges(xt_ctx* ctx, int64_t nv, int64_t m, const int64_t* src, const int64_t* dst, bool borrow,
+                     xt_graph* g);
 // A resident CSR rebuilt as a simple undirected graph in place: rows sorted,
 // duplicates merged, self-loops dropped, missing reverse entries added.
 int graph_clean(xt_ctx* ctx, xt_graph* g);
