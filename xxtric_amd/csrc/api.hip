@@ -168,12 +168,13 @@ bool edge_tile_knobs(const xt_ctx* ctx) {
          ctx->group_hash != kHashMix || ctx->items_per_tile != 256 || ctx->tile_run != 16 || ctx->force_wide;
 }
 
-// Per-vertex counts go to rank space below this many entries: the credit of
-// every hit there costs more than in the edge tiles' hash table, the rest less
-// (ms, rank space against edge tiles: R-MAT s14 0.11 and 0.40, s18 0.88 and
-// 1.08, s20 4.1 and 4.2, s21 9.6 and 8.7; G(n, p) of degree 64 on 200,000 0.83
-// and 2.5).
-constexpr int64_t kRankPvEntries = int64_t(1) << 25;
+// Per-vertex counts go to rank space below this many entries: above, hubs have
+// more hot neighbours than a wave has slots for, and their hits add to device
+// memory one by one (ms, rank space against edge tiles, the generator's labels in
+// brackets: R-MAT s14 0.11 and 0.43 (0.17 and 0.49), s18 0.80 and 1.09 (1.40 and
+// 1.78), s20 3.5 and 4.2 (4.4 and 4.9), s22 17.1 and 18.7 (17.0 and 21.1), s23
+// 40.0 and 37.7 (43.3 and 41.4); G(n, p) of degree 64 on 200,000 0.83 and 2.5).
+constexpr int64_t kRankPvEntries = int64_t(1) << 27;
 // In id orientation out-lists are as long as rows; where rows are long, one
 // wave's list or map waits for another (ms: RGG n = 200,000 0.18 and 0.31,
 // G(n, p) of degree 64 0.87 and 2.6, but R-MAT s14, rows to 3,700, 0.71 and 0.38).

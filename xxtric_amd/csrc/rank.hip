@@ -739,11 +739,12 @@ struct ItemLds {
 
 // probe(chunk, item): item is the chunk's index among the items with chunks.
 // kPerVertex: `label` is u's label; the hits that probe adds to items are added
-// to pv.  kRange: `label` is kept for probe.
-template <int MODE, typename F>
+// to pv, after done(), which ends what probe has put off.  kRange: `label` is
+// kept for probe.
+template <int MODE, typename F, typename G>
 __device__ __forceinline__ void stream_lists(uint32_t start, uint32_t n, uint32_t label, StreamLds& s, ItemLds* s_items,
                                              int lane, const uint4* __restrict__ lists, uint32_t pad,
-                                             unsigned long long* __restrict__ pv, F&& probe) {
+                                             unsigned long long* __restrict__ pv, F&& probe, G&& done) {
   const uint32_t inc = wave_incl_scan_u32(n);
   const uint32_t all = __builtin_amdgcn_readlane(inc, kWave - 1);
   if (all == 0) return;  // uniform
@@ -806,6 +807,7 @@ __device__ __forceinline__ void stream_lists(uint32_t start, uint32_t n, uint32_
     }
   }
   if constexpr (MODE == kPerVertex) {
+    done();
     wave_lds_fence();
     const uint32_t t = s_items->hits[lane];
     if (t) atomicAdd(&pv[s_items->label[lane]], (unsigned long long)t);
@@ -830,11 +832,20 @@ struct Head {  // a record
 // smallest, slot p counts it (added to pv when the row ends), otherwise u's item
 // counter or v's register does.  Places from kSlots on, cold hits and the rows of
 // few ids look labels up and add to pv directly.
-constexpr int kSlots = 512;
+// A lane has 0 to 8 hits of a chunk (2 on average at R-MAT s22), so the hits of a
+// step are put into a queue first and taken from it 128 at a time, two a lane
+// (R-MAT s22, this kernel: 20.5 ms with every lane its own hits one after another,
+// 15.2 with 64 at a time, 14.6 with 128).  What bounds it is the wait for LDS at
+// eight waves a compute unit, and the slots: with the generator's labels, where
+// hubs are credited, 512 take 27.9 ms, 1024 14.3, and 2048, with fewer waves, 21.7.
+constexpr int kSlots = 1024;
+constexpr int kQueue = 10 * kWave;  // a step's hits behind up to 127 older ones
 struct PvLds {
+  uint32_t queue[kQueue];  // hit | item << 16
   uint16_t pre[1024];  // hot ids of N(v) before each 64-bit word of the map
   uint32_t label[kSlots];
-  uint32_t hits[kSlots];
+  uint32_t hits[kSlots / 2];  // 16 bits each: a row's items in a chunk hit a place once each
+  static_assert(kChunk < 65536, "hits of a place");
   ItemLds items;
 };
 struct RangeLds {
@@ -876,7 +887,7 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
   };
   clear_words(kWords / 4);
   if constexpr (PV)
-    for (int i = lane; i < kSlots; i += kWave) s_pv.hits[i] = 0;
+    for (int i = lane; i < kSlots / 2; i += kWave) s_pv.hits[i] = 0;
   wave_lds_fence();
   uint64_t hits = 0, local = 0;  // local: kRange
   auto strip = [](uint32_t w) -> uint32_t { return RANGE && w != kNoRank ? w & ~kOwnedBit : w; };
@@ -1134,6 +1145,36 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
       auto items = [&](uint32_t e) -> uint32_t { return e + lane < cs1 ? part[e + lane] : kNoRank; };
       if (ch > 0) {
         uint32_t acc = 0, acc_local = 0;
+        uint32_t queued = 0;  // PV, uniform
+        // K queue entries a lane (kNoRank: none), their chains of LDS reads side by side.
+        auto credit = [&](const auto& e) {
+          if constexpr (PV) {
+            constexpr int K = sizeof(e) / sizeof(e[0]);
+            uint32_t lu[K], p[K], lw[K];
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+              lu[k] = s_pv.items.label[(e[k] >> 16) & 63u];
+              p[k] = place(e[k] & 0xffffu);
+            }
+#pragma unroll
+            for (int k = 0; k < K; k++) lw[k] = s_pv.label[min(p[k], (uint32_t)kSlots - 1)];
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+              if (e[k] == kNoRank) continue;
+              if (p[k] >= kSlots) lw[k] = orig[e[k] & 0xffffu];
+              if (lw[k] > min(lu[k], cl)) {
+                if (cl < lu[k])
+                  at_v++;
+                else
+                  atomicAdd(&s_pv.items.hits[e[k] >> 16], 1u);
+              } else if (p[k] < kSlots) {
+                atomicAdd(&s_pv.hits[p[k] >> 1], 1u << (16 * (p[k] & 1)));
+              } else {
+                atomicAdd(&pv[lw[k]], 1ull);
+              }
+            }
+          }
+        };
         auto probe = [&](const uint4 q, uint32_t item) {
           const uint32_t y[4] = {q.x, q.y, q.z, q.w};
           uint32_t found = 0;
@@ -1153,27 +1194,33 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
             acc_local += found & s_pv.items.label[item];
           }
           if constexpr (PV) {
-            acc += (uint32_t)__popc(found);
-            const uint32_t lu = found ? s_pv.items.label[item] : 0;
-            const uint32_t two = min(lu, cl);
-            uint32_t rest = 0;  // hits credited to u or v
-            while (found) {
-              const int j = __builtin_ctz(found);
-              found &= found - 1;
-              const uint32_t z = ((j & 4) ? (j & 2 ? y[3] : y[2]) : (j & 2 ? y[1] : y[0])) >> (16 * (j & 1)) & 0xffffu;
-              const uint32_t p = place(z);
-              const uint32_t lw = p < kSlots ? s_pv.label[p] : orig[z];
-              if (lw > two)
-                rest++;
-              else if (p < kSlots)
-                atomicAdd(&s_pv.hits[p], 1u);
-              else
-                atomicAdd(&pv[lw], 1ull);
+            const uint32_t n = (uint32_t)__popc(found), inc = wave_incl_scan_u32(n);
+            acc += n;
+            uint32_t at = queued + inc - n;
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+              if ((found >> j) & 1u) {
+                s_pv.queue[at] = (j & 1 ? y[j / 2] >> 16 : y[j / 2] & 0xffffu) | (item << 16);
+                at++;
+              }
             }
-            if (cl < lu)
-              at_v += rest;
-            else if (rest)
-              atomicAdd(&s_pv.items.hits[item], rest);
+            queued += __builtin_amdgcn_readlane(inc, kWave - 1);
+            wave_lds_fence();
+            while (queued >= 2 * kWave) {  // uniform
+              queued -= 2 * kWave;
+              const uint32_t e[2] = {s_pv.queue[queued + lane], s_pv.queue[queued + kWave + lane]};
+              credit(e);
+            }
+            wave_lds_fence();
+          }
+        };
+        auto done = [&]() {
+          if constexpr (PV) {
+            if (queued == 0) return;  // uniform
+            const uint32_t e[2] = {(uint32_t)lane < queued ? s_pv.queue[lane] : kNoRank,
+                                   kWave + lane < queued ? s_pv.queue[kWave + lane] : kNoRank};
+            credit(e);
+            queued = 0;
           }
         };
         // kRange: hits of owned ids are local where u or v is owned, those of the
@@ -1181,11 +1228,11 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
         auto stream = [&](uint32_t ss, uint32_t nn, uint32_t nr, uint32_t hot2, uint32_t ll, uint32_t ur) {
           if constexpr (RANGE) {
             const bool u_own = ur != kNoRank && (ur & kOwnedBit);
-            stream_lists<MODE>(ss, nn, v_own || u_own ? ~0u : 0u, s_stream, s_items, lane, lists, 0xffffffffu, pv, probe);
+            stream_lists<MODE>(ss, nn, v_own || u_own ? ~0u : 0u, s_stream, s_items, lane, lists, 0xffffffffu, pv, probe, done);
             stream_lists<MODE>(ss + (hot2 & 0xffffu), nr, v_own && u_own ? ~0u : 0u, s_stream, s_items, lane, lists,
-                               0xffffffffu, pv, probe);
+                               0xffffffffu, pv, probe, done);
           } else {
-            stream_lists<MODE>(ss, nn, ll, s_stream, s_items, lane, lists, 0xffffffffu, pv, probe);
+            stream_lists<MODE>(ss, nn, ll, s_stream, s_items, lane, lists, 0xffffffffu, pv, probe, done);
           }
         };
         uint32_t yu = kNoRank;
@@ -1206,12 +1253,11 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
         hits += acc;
         wave_lds_fence();
         if constexpr (PV)
-          for (uint32_t p = lane; p < min(ch, (uint32_t)kSlots); p += kWave) {
+          for (uint32_t p = lane; 2 * p < min(ch, (uint32_t)kSlots); p += kWave) {
             const uint32_t t = s_pv.hits[p];
-            if (t) {
-              atomicAdd(&pv[s_pv.label[p]], (unsigned long long)t);
-              s_pv.hits[p] = 0;
-            }
+            if (t & 0xffffu) atomicAdd(&pv[s_pv.label[2 * p]], (unsigned long long)(t & 0xffffu));
+            if (t >> 16) atomicAdd(&pv[s_pv.label[2 * p + 1]], (unsigned long long)(t >> 16));
+            if (t) s_pv.hits[p] = 0;
           }
         if (cd <= 8 * kWave) {
           for (uint32_t i = 0; i < cd; i += kWave) {
@@ -1270,11 +1316,11 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
             if constexpr (RANGE) {
               const bool u_own = ur != kNoRank && (ur & kOwnedBit);
               const uint32_t c0 = ss + (l1 & 0xffffu) + (l1 >> 16);  // behind both hot parts
-              stream_lists<MODE>(c0, l2 & 0xffffu, v_own || u_own ? ~0u : 0u, s_stream, s_items, lane, lists, kNoRank, pv, probe);
+              stream_lists<MODE>(c0, l2 & 0xffffu, v_own || u_own ? ~0u : 0u, s_stream, s_items, lane, lists, kNoRank, pv, probe, [] {});
               stream_lists<MODE>(c0 + (l2 & 0xffffu), v_own || u_own ? l2 >> 16 : 0, v_own && u_own ? ~0u : 0u, s_stream,
-                                 s_items, lane, lists, kNoRank, pv, probe);
+                                 s_items, lane, lists, kNoRank, pv, probe, [] {});
             } else {
-              stream_lists<MODE>(ss + (l1 & 0xffffu), l1 >> 16, ll, s_stream, s_items, lane, lists, kNoRank, pv, probe);
+              stream_lists<MODE>(ss + (l1 & 0xffffu), l1 >> 16, ll, s_stream, s_items, lane, lists, kNoRank, pv, probe, [] {});
             }
           };
           stream(st, len, len2, label, u0);
