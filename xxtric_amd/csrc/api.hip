@@ -198,7 +198,6 @@ int count_device_csr(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int6
   const int mode = (flags & XT_ORIENT_ID) ? kOrientId : kOrientDegree;
   ctx->last_ranked = false;
   XT_TRY(ensure(ctx, s.counters, kNumCounters * sizeof(uint64_t)));
-  XT_TRY(fill_u64(ctx, s.counters.as<uint64_t>(), kNumCounters, 0, st));
   uint64_t* pv = nullptr;
   if (flags & XT_PER_VERTEX) {
     XT_TRY(ensure(ctx, s.pv, (size_t)(nv > 0 ? nv : 1) * sizeof(uint64_t)));
@@ -211,6 +210,7 @@ int count_device_csr(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int6
     ctx->last_ranked = true;
     return XT_OK;
   }
+  XT_TRY(fill_u64(ctx, s.counters.as<uint64_t>(), kNumCounters, 0, st));
   // Grow every scratch buffer before the first event so no allocation (and
   // its implicit synchronisation) falls inside the timed window.
   XT_TRY(ensure(ctx, s.ooff, (size_t)(nv + 1) * sizeof(int64_t)));
@@ -234,15 +234,15 @@ template int count_device_csr<int64_t>(xt_ctx*, Scratch&, int64_t, int64_t, cons
 // (nullable, kNumCounters words) gets all counters.
 static int finish_count(xt_ctx* ctx, int64_t nv, uint32_t flags, hipStream_t st, bool timed,
                         uint64_t* total, uint64_t* per_vertex, uint64_t* sums = nullptr) {
-  uint64_t h[kNumCounters];
-  XT_HIP(ctx, hipMemcpyAsync(h, ctx->s.counters.p, sizeof(h), hipMemcpyDeviceToHost, st));
+  uint64_t* h = ctx->h_counters;
+  XT_HIP(ctx, hipMemcpyAsync(h, ctx->s.counters.p, kNumCounters * sizeof(uint64_t), hipMemcpyDeviceToHost, st));
   if (per_vertex && (flags & XT_PER_VERTEX) && nv > 0)
     XT_HIP(ctx, hipMemcpyAsync(per_vertex, ctx->s.pv.p, (size_t)nv * sizeof(uint64_t),
                                hipMemcpyDeviceToHost, st));
   XT_HIP(ctx, hipStreamSynchronize(st));
   if (h[kBadIds]) return set_err(ctx, XT_ERR_INPUT, "neighbour id out of range [0, nv)");
   if (total) *total = sum_of(h, kSumTotal);
-  if (sums) std::memcpy(sums, h, sizeof(h));
+  if (sums) std::memcpy(sums, h, kNumCounters * sizeof(uint64_t));
   int64_t nep = 0, nheavy = 0, ntiles = 0, nwave = 0;
   const bool ranked = ctx->last_ranked;
   const bool worked = nv > 0 && ctx->s.itcnt.p != nullptr && ctx->s.ooff.p != nullptr;
@@ -348,7 +348,13 @@ int xt_ctx_create(int device, xt_ctx** out) {
       delete ctx;
       return XT_ERR_NOMEM;
     }
+    if (hipHostMalloc((void**)&ctx->h_counters, kNumCounters * sizeof(uint64_t)) != hipSuccess) {
+      release(ctx->s);
+      delete ctx;
+      return XT_ERR_NOMEM;
+    }
     if (noalloc_init(ctx, device) != XT_OK) {
+      (void)hipHostFree(ctx->h_counters);
       release(ctx->s);
       delete ctx;
       return XT_ERR_HIP;
@@ -365,6 +371,7 @@ int xt_ctx_destroy(xt_ctx* ctx) {
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     release(ctx->s);
     if (ctx->build.p) (void)hipFree(ctx->build.p);
+    if (ctx->h_counters) (void)hipHostFree(ctx->h_counters);
     for (int i = 0; i < kNumEv; i++)
       if (ctx->ev[i]) (void)hipEventDestroy(ctx->ev[i]);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
@@ -592,24 +599,22 @@ int xt_single_gpu_count(xt_ctx* ctx, int64_t nv, const int64_t* d_indices, const
     if (nv >= (1LL << 31) - 1) return set_err(ctx, XT_ERR_ARG, "nv must be below 2^31-1 (int32 device ids)");
     if (nv == 0) return XT_OK;
     hipStream_t st = stream ? static_cast<hipStream_t>(stream) : ctx->stream;
-    int64_t ne = 0;
-    XT_HIP(ctx, hipMemcpyAsync(&ne, d_indices + nv, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+    XT_HIP(ctx, hipMemcpyAsync(ctx->h_counters, d_indices + nv, sizeof(int64_t), hipMemcpyDeviceToHost, st));
     XT_HIP(ctx, hipStreamSynchronize(st));
+    const int64_t ne = (int64_t)ctx->h_counters[0];
     if (ne < 0) return set_err(ctx, XT_ERR_INPUT, "negative edge count in d_indices[nv]");
     if (ne > 0 && !d_edge_list) return set_err(ctx, XT_ERR_ARG, "null d_edge_list");
     // Offsets must be a valid index (and rows sorted) before the chunked
     // kernels search them; the reference launcher assumes the same.
     XT_TRY(validate<int64_t>(ctx, nv, ne, d_indices, d_edge_list, false, st));
     XT_TRY(count_device_csr<int64_t>(ctx, ctx->s, nv, ne, d_indices, d_edge_list, XT_ORIENT_DEGREE, st, false, RankUse{true, -1}));
-    uint64_t bad = 0;
-    XT_HIP(ctx, hipMemcpyAsync(&bad, ctx->s.counters.as<uint64_t>() + kBadIds, sizeof(bad),
+    XT_TRY(launch_add_total(ctx, d_local_count, st));  // nothing if an id was out of range
+    XT_HIP(ctx, hipMemcpyAsync(ctx->h_counters, ctx->s.counters.as<uint64_t>() + kBadIds, sizeof(uint64_t),
                                hipMemcpyDeviceToHost, st));
-    XT_HIP(ctx, hipStreamSynchronize(st));
-    if (bad) return set_err(ctx, XT_ERR_INPUT, "neighbour id out of range [0, nv)");
-    XT_TRY(launch_add_total(ctx, d_local_count, st));
     // The add reads the context's counters, which the next call on this
     // context (on any stream) clears: it must be done before this returns.
     XT_HIP(ctx, hipStreamSynchronize(st));
+    if (ctx->h_counters[0]) return set_err(ctx, XT_ERR_INPUT, "neighbour id out of range [0, nv)");
     return XT_OK;
   });
 }
@@ -627,9 +632,9 @@ int xt_single_gpu_count_noalloc(xt_ctx* ctx, int64_t nv, const int64_t* d_indice
     NoAllocDevice& dev = g_noalloc[ctx->device];
     if (nv == 0) return XT_OK;
     hipStream_t st = stream ? static_cast<hipStream_t>(stream) : ctx->stream;
-    int64_t ne = 0;
-    XT_HIP(ctx, hipMemcpyAsync(&ne, d_indices + nv, sizeof(int64_t), hipMemcpyDeviceToHost, st));
+    XT_HIP(ctx, hipMemcpyAsync(ctx->h_counters, d_indices + nv, sizeof(int64_t), hipMemcpyDeviceToHost, st));
     XT_HIP(ctx, hipStreamSynchronize(st));
+    const int64_t ne = (int64_t)ctx->h_counters[0];
     if (ne < 0) return set_err(ctx, XT_ERR_INPUT, "negative edge count in d_indices[nv]");
     if (ne > 0 && !d_edge_list) return set_err(ctx, XT_ERR_ARG, "null d_edge_list");
     const size_t need = carve_bytes(nv, ne);
@@ -646,11 +651,11 @@ int xt_single_gpu_count_noalloc(xt_ctx* ctx, int64_t nv, const int64_t* d_indice
     auto run = [&]() -> int {
       XT_TRY(validate<int64_t>(ctx, nv, ne, d_indices, d_edge_list, false, st, counters));
       XT_TRY(count_device_csr<int64_t>(ctx, s, nv, ne, d_indices, d_edge_list, XT_ORIENT_DEGREE, st, false, RankUse{false, -1}));
-      uint64_t bad = 0;
-      XT_HIP(ctx, hipMemcpyAsync(&bad, counters + kBadIds, sizeof(bad), hipMemcpyDeviceToHost, st));
+      XT_TRY(launch_add_total(ctx, d_local_count, st, counters));  // nothing if an id was out of range
+      XT_HIP(ctx, hipMemcpyAsync(ctx->h_counters, counters + kBadIds, sizeof(uint64_t), hipMemcpyDeviceToHost, st));
       XT_HIP(ctx, hipStreamSynchronize(st));
-      if (bad) return set_err(ctx, XT_ERR_INPUT, "neighbour id out of range [0, nv)");
-      return launch_add_total(ctx, d_local_count, st, counters);
+      if (ctx->h_counters[0]) return set_err(ctx, XT_ERR_INPUT, "neighbour id out of range [0, nv)");
+      return XT_OK;
     };
     const int rc = run();
     // On every path, nothing queued by this call may still use the array

@@ -460,6 +460,7 @@ __global__ __launch_bounds__(kBlock) void k_validate(int64_t nv, int64_t ne,
                                                      uint64_t* __restrict__ counters) {
   __shared__ int64_t s_off[kOffCap + 1];
   __shared__ int64_t s_lohi[2];
+  if (counters[kBadOff]) return;  // whole grid: k_check_offsets found no index to walk
   const int64_t eb = (int64_t)blockIdx.x * kChunk;
   const int64_t ee = min(ne, eb + (int64_t)kChunk);
   const ChunkRows r = chunk_rows(off, nv, eb, ee, s_off, s_lohi);
@@ -486,7 +487,8 @@ __global__ __launch_bounds__(kBlock) void k_validate(int64_t nv, int64_t ne,
   if (asym) atomicAdd((unsigned long long*)&counters[kAsym], (unsigned long long)asym);
 }
 
-// Offsets check followed by the entry checks; reads the verdict back (syncs).
+// Offsets check followed by the entry checks (which do nothing where it failed);
+// reads the verdict back (syncs).
 template <typename T>
 int validate(xt_ctx* ctx, int64_t nv, int64_t ne, const int64_t* off, const T* tails,
              bool symmetry, hipStream_t st, uint64_t* counters) {
@@ -495,18 +497,16 @@ int validate(xt_ctx* ctx, int64_t nv, int64_t ne, const int64_t* off, const T* t
   hipLaunchKernelGGL(k_check_offsets, dim3(grid_for(nv, 256, 4096)), dim3(256), 0, st, nv, ne, off,
                      counters);
   XT_HIP(ctx, hipGetLastError());
-  uint64_t h[4];
-  XT_HIP(ctx, hipMemcpyAsync(h, counters + kBadIds, sizeof(h), hipMemcpyDeviceToHost, st));
-  XT_HIP(ctx, hipStreamSynchronize(st));
-  if (h[kBadOff - kBadIds]) return set_err(ctx, XT_ERR_INPUT, "offsets are not a valid CSR index");
   if (ne > 0) {
     const int64_t nchunks = (ne + kChunk - 1) / kChunk;
     hipLaunchKernelGGL((k_validate<T>), dim3((unsigned)nchunks), dim3(kBlock), 0, st, nv, ne, off,
                        tails, symmetry ? 1 : 0, counters);
     XT_HIP(ctx, hipGetLastError());
-    XT_HIP(ctx, hipMemcpyAsync(h, counters + kBadIds, sizeof(h), hipMemcpyDeviceToHost, st));
-    XT_HIP(ctx, hipStreamSynchronize(st));
   }
+  uint64_t* h = ctx->h_counters;
+  XT_HIP(ctx, hipMemcpyAsync(h, counters + kBadIds, 4 * sizeof(uint64_t), hipMemcpyDeviceToHost, st));
+  XT_HIP(ctx, hipStreamSynchronize(st));
+  if (h[kBadOff - kBadIds]) return set_err(ctx, XT_ERR_INPUT, "offsets are not a valid CSR index");
   if (h[0]) return set_err(ctx, XT_ERR_INPUT, "neighbour id out of range [0, nv)");
   if (h[1]) return set_err(ctx, XT_ERR_INPUT, "adjacency row not strictly ascending (unsorted or duplicate entries)");
   if (h[2]) return set_err(ctx, XT_ERR_INPUT, "adjacency is not symmetric");

@@ -97,6 +97,15 @@ __device__ __forceinline__ uint32_t list_room(uint32_t t) {
   return t <= 2 ? t : t <= 4 ? 4 : (t + 7) & ~7u;
 }
 
+// The counters and both halves of the class histogram cleared in one launch (a
+// launch is 5 to 8 us of a small count's 90).
+__global__ __launch_bounds__(256) void k_rank_clear(uint64_t* __restrict__ counters, uint32_t* __restrict__ hist) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < kNumCounters) counters[i] = 0;
+  if (i < kRankClasses) hist[i] = hist[kRankClasses + i] = 0;
+}
+static_assert(kNumCounters >= kRankClasses, "the grid covers both");
+
 // ---------------------------------------------------------------------------
 // Degree classes counted (one histogram per workgroup in LDS), per-row
 // counters cleared, and the first and last row of every S-entry chunk
@@ -1449,7 +1458,8 @@ int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* o
   uint32_t* part = s.rpart.as<uint32_t>();
   uint4* lists = s.rlists.as<uint4>();
   RankRec* rec = s.rrec.as<RankRec>();
-  XT_TRY(fill_u32(ctx, hist, 2 * kRankClasses, 0u, st));
+  hipLaunchKernelGGL(k_rank_clear, dim3((kNumCounters + 255) / 256), dim3(256), 0, st, counters, hist);
+  XT_HIP(ctx, hipGetLastError());
   hipLaunchKernelGGL(k_rank_prep, dim3(rank_grid(nv, 1024, 8192)), dim3(256), 0, st, nv, ne, off, S, crows, oc,
                      s.itcnt.as<uint32_t>(), hist, pvp, oc1);
   XT_HIP(ctx, hipGetLastError());

@@ -132,6 +132,7 @@ struct xt_ctx {
   std::recursive_mutex mu;
   xt::Scratch s;
   xt::DevBuf build;  // memory of graph builds (stream's work only)
+  uint64_t* h_counters = nullptr;  // pinned, kNumCounters: what a call reads back before it goes on or returns
   hipEvent_t ev[xt::kNumEv] = {};
   xt_timing timing = {};
   // Light edges: both out-lists at most this long; 0 picks kLightCut for one
