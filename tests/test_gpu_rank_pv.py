@@ -43,3 +43,25 @@ def test_credit_by_label(ctx, n, power, labels):
     a, b = g.count(per_vertex=True), _tiles(ctx, g, per_vertex=True)
     g.close()
     assert a[0] == b[0] and (a[1] == b[1]).all()
+
+
+@pytest.mark.parametrize("d", [63, 64, 65, 128, 255, 256, 257, 320, 512, 600])
+def test_rows_around_a_block_of_loads(ctx, d):
+    """Two rows of d smaller ranks (and one more) under d mutually joined hubs that a
+    fringe of pendant vertices lifts above them."""
+    rng = np.random.default_rng(d)
+    hubs = np.arange(d, dtype=np.int64)
+    a, b = np.triu_indices(d, 1)
+    u = [hubs[a], np.repeat([d, d + 1], d), np.array([d])]
+    v = [hubs[b], np.tile(hubs, 2), np.array([d + 1])]
+    n = d + 2 + 4 * d
+    u.append(np.repeat(hubs, 4))
+    v.append(np.arange(d + 2, n))
+    name = rng.permutation(n)
+    g = ctx.graph_from_edges(n, name[np.concatenate(u)], name[np.concatenate(v)])
+    _say("hubs", d)
+    total = d * (d - 1) * (d - 2) // 6 + 2 * (d * (d - 1) // 2) + d
+    assert g.count() == total
+    a, b = g.count(per_vertex=True), _tiles(ctx, g, per_vertex=True)
+    g.close()
+    assert a[0] == b[0] == total and (a[1] == b[1]).all()

@@ -1,4 +1,5 @@
-// rank.hip -- the count in rank space (gfx950): plain totals of one graph.
+// rank.hip -- the count of one graph in rank space (gfx950): totals, per-vertex
+// counts and owned ranges.
 //
 // Vertices are ranked by descending degree (rank 0 = the largest hub) and
 // every triangle w < v < u (ranks) is counted once, at its edge (u, v), as an
@@ -23,7 +24,8 @@
 // cache).  R-MAT s26: 353 ms with edge tiles, 186-189 here: k_rank_split 42,
 // k_rank_lists 11, k_rank_count 132-135.
 //
-// Five kernels, no scan over the vertices and no item list:
+// Six kernels, no scan over the vertices and no item list:
+//  k_rank_clear   counters and class histogram cleared
 //  k_rank_prep    degree classes counted, first and last row of every chunk
 //  k_rank_assign  ranks: counting sort of the vertices by degree class
 //  k_rank_split   per row, in place of the labels: ranks, smaller ones first
@@ -410,6 +412,26 @@ __global__ __launch_bounds__(kBlock) void k_rank_split(int64_t nv, int64_t ne, c
 }
 
 // ---------------------------------------------------------------------------
+// f(id) for the ids of a row, in order.  Beyond a wave's worth four loads are in
+// flight instead of one after another: a hub's 1,500 ids are read twice for its list
+// and by the wave of each of its chunks (R-MAT s22 6.35 -> 6.21 ms, per vertex with
+// the generator's labels 17.0 -> 16.3; rows of up to 64 ids as before).
+template <typename I, typename F>
+__device__ __forceinline__ void each_id(uint32_t n, I&& id, F&& f) {
+  if (n <= kWave) {
+    f(id(0u));
+    return;
+  }
+  for (uint32_t i = 0; i < n; i += 4 * kWave) {
+    uint32_t y[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++) y[k] = id(i + k * kWave);
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++)
+      if (i + k * kWave < n) f(y[k]);
+  }
+}
+
 // Lists and records, by independent waves.  A wave takes `rows` vertices at a
 // time, one per lane, few neighbouring ones from all over the graph (labels that
 // bring vertices of large degree together do not load one wave).  Their lists lie
@@ -645,13 +667,12 @@ __global__ __launch_bounds__(64) void k_rank_lists(int64_t nv, const int64_t* __
             place += (uint32_t)__builtin_amdgcn_readlane((int)w, __builtin_ctzll(m)) < w ? 1u : 0u;
         } else {
           uint32_t top = 0;  // groups in use
-          for (uint32_t i = 0; i < dd; i += kWave) {
-            const uint32_t w = id(i);
+          each_id(dd, id, [&](uint32_t w) {
             if (w < kHot) {
               atomicOr(&bits[w >> 6], 1ull << (w & 63));
               top = max(top, (w >> 13) + 1);
             }
-          }
+          });
           wave_lds_fence();
 #pragma unroll 1
           for (uint32_t k = 0; k < (uint32_t)kGroups; k++) {
@@ -669,8 +690,7 @@ __global__ __launch_bounds__(64) void k_rank_lists(int64_t nv, const int64_t* __
         uint16_t* hl = reinterpret_cast<uint16_t*>(lists + st + hot0);
         uint32_t* cl = reinterpret_cast<uint32_t*>(lists + st + cold0);
         uint32_t ncold = 0;
-        for (uint32_t i = 0; i < dd; i += kWave) {
-          const uint32_t w = id(i);
+        each_id(dd, id, [&](uint32_t w) {
           const bool cold = w >= kHot && w != kNoRank;
           const uint64_t cm = __builtin_amdgcn_ballot_w64(cold);
           if (w < kHot) {
@@ -688,13 +708,12 @@ __global__ __launch_bounds__(64) void k_rank_lists(int64_t nv, const int64_t* __
             if (r < 4 * ccc) cl[r] = w;
           }
           ncold += (uint32_t)__popcll(cm);
-        }
+        });
         wave_lds_fence();
-        if (dd > kWave)
-          for (uint32_t i = 0; i < dd; i += kWave) {
-            const uint32_t w = id(i);
-            if (w < kHot) bits[w >> 6] = 0ull;
-          }
+        if (dd > kWave) {  // uniform
+#pragma unroll
+          for (int k = 0; k < kGroups; k++) s_bits[k * kWave + lane] = make_ulonglong2(0, 0);
+        }
         if ((uint32_t)lane < 8 * hcc - min(hh, 8 * hcc)) hl[hh + lane] = 0xffff;
         if ((uint32_t)lane < 4 * ccc - min(ncold, 4 * ccc)) cl[ncold + lane] = kNoRank;
         mark0 += marks;
@@ -1108,10 +1127,9 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
       const uint32_t n_rest = RANGE && (v_own || (u0 & kOwnedBit && u0 != kNoRank)) ? prefix_rest(x) : 0;
       uint32_t at_v = 0;  // PV: hits credited to v
       if (ch > 0)
-        for (uint32_t i = 0; i < cd; i += kWave) {
-          const uint32_t y = id(i);
+        each_id(cd, id, [&](uint32_t y) {
           if (y < kHot) atomicOr(&s_bm[y >> 5], 1u << (y & 31));
-        }
+        });
       unsigned long long* s_map = reinterpret_cast<unsigned long long*>(s_mem);
       auto place = [&](uint32_t y) -> uint32_t {  // of hot id y of N(v)
         if constexpr (PV)
@@ -1137,13 +1155,12 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
             }
           }
           wave_lds_fence();
-          for (uint32_t i = 0; i < cd; i += kWave) {
-            const uint32_t y = id(i);
+          each_id(cd, id, [&](uint32_t y) {
             if (y < kHot) {
               const uint32_t p = place(y);
               if (p < kSlots) s_pv.label[p] = orig[y];
             }
-          }
+          });
           wave_lds_fence();
         }
       }
@@ -1268,11 +1285,8 @@ __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const
             if (t >> 16) atomicAdd(&pv[s_pv.label[2 * p + 1]], (unsigned long long)(t >> 16));
             if (t) s_pv.hits[p] = 0;
           }
-        if (cd <= 8 * kWave) {
-          for (uint32_t i = 0; i < cd; i += kWave) {
-            const uint32_t y = id(i);
-            if (y < kHot) s_bm[y >> 5] = 0;
-          }
+        if (cd <= kWave) {
+          if (w < kHot) s_bm[w >> 5] = 0;
         } else {
           clear_words(kWords / 4);
         }
