@@ -50,11 +50,11 @@ SPACE = {
     "tile_run": (4, 8, 16, 32, 64),
     "group_hash": (1, 2),
 }
-# The library's own choice (-1): a plain count in rank space, which takes none of
-# these knobs; any knob away from its default asks for the edge tiles.
+# The library's own choice (-1): a plain count in rank space, a batch of small graphs
+# in 16-bit lists, neither of which takes these knobs; any knob away from its
+# default asks for the edge tiles.
 DEFAULTS = {"light_cut": -1, "wave_owner": -1, "group_round": 2, "group_blocks": 4, "items_per_tile": 256,
             "tile_run": 16, "group_hash": 1}
-BATCH_DEFAULTS = dict(DEFAULTS, light_cut=8, wave_owner=64)
 
 
 def _time_graph(ctx, g, reps):
@@ -146,7 +146,7 @@ def tune(ctx, workload="rmat", scale=22, graphs=1024, reps=3, passes=2, cache=DE
             b.add_generated(2026, 0, graphs)
         runner = lambda: _time_batch(b, reps)  # noqa: E731
         key = "batch_%d" % graphs
-        start = BATCH_DEFAULTS
+        start = DEFAULTS
     else:
         raise ValueError(workload)
     t0 = time.perf_counter()
