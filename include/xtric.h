@@ -77,10 +77,12 @@ const char* xt_last_error(const xt_ctx* ctx);
 int xt_last_timing(const xt_ctx* ctx, xt_timing* out);
 /* Totals and owned ranges of one graph in degree orientation are counted in rank
  * space (vertices ranked by degree, lists of smaller ranks in 16 bits, bit maps in LDS), and so
- * are its per-vertex counts below 2^25 entries and, where the host passed in the
- * offsets and no row is longer than 256, counts in id orientation.  The knobs
+ * are its per-vertex counts below 2^27 entries and, where the host passed in the
+ * offsets and no row is longer than 256, counts in id orientation.  Batches whose
+ * graphs have at most 65535 vertices are counted over 16-bit lists.  The knobs
  * below belong to the edge tiles that all other counts use; a context on which
- * one of them is away from its default uses edge tiles for all of them.
+ * one of them is away from its default uses edge tiles for all of them.  A context
+ * keeps up to 512 MiB of device memory of its graph builds until it is destroyed.
  * Tuning knobs (set by xxtric_amd.autotune from measurements; 0 keeps the
  * current value): light_cut -- edges whose two out-lists are both at most this
  * long are intersected one per thread, the rest by the group kernel or wave

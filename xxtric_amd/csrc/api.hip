@@ -171,8 +171,8 @@ bool edge_tile_knobs(const xt_ctx* ctx) {
 // Per-vertex counts go to rank space below this many entries: above, hubs have
 // more hot neighbours than a wave has slots for, and their hits add to device
 // memory one by one (ms, rank space against edge tiles, the generator's labels in
-// brackets: R-MAT s14 0.11 and 0.43 (0.17 and 0.49), s18 0.80 and 1.09 (1.40 and
-// 1.78), s20 3.5 and 4.2 (4.4 and 4.9), s22 17.1 and 18.7 (17.0 and 21.1), s23
+// brackets: R-MAT s14 0.11 and 0.43 (0.17 and 0.49), s18 0.79 and 1.09 (1.33 and
+// 1.78), s20 3.4 and 4.2 (4.3 and 4.9), s22 16.7 and 18.7 (16.3 and 21.1), s23
 // 40.0 and 37.7 (43.3 and 41.4); G(n, p) of degree 64 on 200,000 0.83 and 2.5).
 constexpr int64_t kRankPvEntries = int64_t(1) << 27;
 // In id orientation out-lists are as long as rows; where rows are long, one

@@ -21,8 +21,8 @@
 //
 // Both passes that gather or stream are bound by the lines that miss L2 (about
 // 52-55 G lines of 128 bytes a second on this GPU, from HBM or from the 256 MB
-// cache).  R-MAT s26: 353 ms with edge tiles, 186-189 here: k_rank_split 42,
-// k_rank_lists 11, k_rank_count 132-135.
+// cache).  R-MAT s26: 353 ms with edge tiles, 182-188 here: k_rank_split 40-42,
+// k_rank_lists 10-11, k_rank_count 131-135 (949 GB: 7.1 TB/s).
 //
 // Six kernels, no scan over the vertices and no item list:
 //  k_rank_clear   counters and class histogram cleared
@@ -884,7 +884,7 @@ struct NoLds {};
 // kRange: a triangle with its labels above rlo counts as owned when one of its
 // vertices is owned, as local when two are.  Of u's list the owned ids are
 // streamed for every item, the others only where u or v is owned (rank 0 of 8
-// of R-MAT s23: 20.3 ms in edge tiles, 12.5 here, 6.1 of them in this kernel
+// of R-MAT s23: 20.3 ms in edge tiles, 12.3 here, 6.0 of them in this kernel
 // against 9.2 for the total).
 template <int MODE>
 __global__ __launch_bounds__(64) void k_rank_count(int64_t nv, int64_t ne, const int64_t* __restrict__ off,
