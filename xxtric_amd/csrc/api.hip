@@ -5,6 +5,7 @@
 #include <cstring>
 #include <vector>
 
+#include "xt_bounds.hpp"
 #include "xt_device.hpp"
 #include "xt_internal.hpp"
 
@@ -151,15 +152,7 @@ static int noalloc_init(xt_ctx* ctx, int device) {
 static int check_host_offsets(xt_ctx* ctx, int64_t nv, int64_t ne, const int64_t* off, int64_t* max_degree) {
   if (nv < 0 || ne < 0 || !off) return set_err(ctx, XT_ERR_ARG, "negative size or null offsets");
   if (nv >= (1LL << 31) - 1) return set_err(ctx, XT_ERR_ARG, "nv must be below 2^31-1 (int32 device ids)");
-  if (off[0] != 0 || off[nv] != ne) return set_err(ctx, XT_ERR_INPUT, "offsets must start at 0 and end at ne");
-  int64_t least = 0, most = 0;
-  for (int64_t i = 0; i < nv; i++) {
-    const int64_t d = off[i + 1] - off[i];
-    least = d < least ? d : least;
-    most = d > most ? d : most;
-  }
-  if (least < 0) return set_err(ctx, XT_ERR_INPUT, "offsets are not monotone");
-  if (max_degree) *max_degree = most;
+  if (const char* bad = check_offsets(nv, ne, off, max_degree)) return set_err(ctx, XT_ERR_INPUT, bad);
   return XT_OK;
 }
 
