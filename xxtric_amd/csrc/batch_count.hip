@@ -22,6 +22,7 @@
 // 8-byte record and write a 16-byte item per entry in about 20 launches.  Every row
 // a lane per item (up to 72 ids compared in registers): 2.46 ms; every row through
 // bit maps: 1.38 ms; tiny rows of up to 16 ids: 1.45 ms.
+#include "xt_bounds.hpp"
 #include "xt_device.hpp"
 #include "xt_internal.hpp"
 
@@ -515,7 +516,7 @@ static int64_t batch_chunk(const xt_ctx* ctx, int64_t ne) {
 }
 
 bool batch_small_fits(int64_t max_graph_vertices, int64_t ne) {
-  return max_graph_vertices <= 65535 && ne < (1ll << 32) - 64;
+  return max_graph_vertices <= 65535 && ne < kIndex32Entries;
 }
 
 int batch_small_reserve(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne) {

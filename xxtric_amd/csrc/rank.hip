@@ -33,9 +33,9 @@
 //                 16-bit, then cold 32-bit) and a 32-byte record
 //  k_rank_count   per chunk of entries, one wave: v's map, the lists of its
 //                 larger neighbours u streamed through it
-#include <cmath>
 #include <type_traits>
 
+#include "xt_bounds.hpp"
 #include "xt_device.hpp"
 #include "xt_hash.hpp"
 #include "xt_internal.hpp"
@@ -444,15 +444,6 @@ __device__ __forceinline__ void each_id(uint32_t n, I&& id, F&& f) {
 // are ranked by counting the smaller ones, more are sorted by a bit map of
 // their hot ids in LDS with running counts (an id's place is the count before
 // its word plus the bits below it).  Cold ids keep the row's order.
-constexpr int kListShards = 16;
-
-struct ListRoom {
-  uint64_t region, grant;  // lines of a shard's region; lines drawn at once
-  int rows;                // vertices of a wave: 16, 32 or 64
-  int together;            // log2 of the neighbouring vertices it takes at a time
-  int64_t nbatch;
-};
-
 template <int MODE>
 __global__ __launch_bounds__(64) void k_rank_lists(int64_t nv, const int64_t* __restrict__ off,
                                                    const uint64_t* __restrict__ oc, const uint64_t* __restrict__ oc1,
@@ -1393,47 +1384,8 @@ static unsigned rank_grid(int64_t n, int per, int64_t cap) {
   return (unsigned)g;
 }
 
-// Room for the lists of a simple graph, in 128-byte lines: |E+| = ne / 2 ids; a
-// list of d >= 2 ids is given at most min(d, d / 4 + 9.25) chunks (hot and cold
-// parts rounded up to chunks, then to list_room; two parts each: d / 4 + 11.5), a wave's lists at a time
-// rounded up to a line.  Grants but a wave's last are used to three quarters.
-// A region is left for the next when a request does not fit, so each may lose
-// one request: a grant, or 64 of the longest lists (at most 1.02 sqrt(ne) ids,
-// since out-neighbours have about the vertex's degree or more).
-static ListRoom rank_list_room(const xt_ctx* ctx, int64_t nv, int64_t ne, bool by_label, int parts, int64_t* lines) {
-  ListRoom r;
-  const int64_t waves = (int64_t)ctx->num_cus * 16;
-  r.rows = kWave;
-  while (r.rows > 16 && nv / r.rows < waves) r.rows >>= 1;
-  // Four neighbours read a quarter of a line of each vertex array: all right
-  // while these stay in the 256 MB cache (20 bytes a vertex).
-  r.together = nv <= (1ll << 22) ? 2 : 4;
-  r.nbatch = (nv + r.rows - 1) / r.rows;
-  const int64_t nlists = nv < ne / 4 ? nv : ne / 4;
-  const int64_t chunks = parts == 4 ? ne / 8 + 12 * nlists
-                         : ne / 8 + 10 * nlists < ne / 2 ? ne / 8 + 10 * nlists : ne / 2;
-  const int64_t need = chunks / 8 + r.nbatch + 1;
-  const int64_t grant = need / (waves * 32) < 8 ? 8 : need / (waves * 32);
-  const int64_t used = need + need / 3 + (r.nbatch < waves ? r.nbatch : waves) * grant;
-  const double longest = by_label ? (double)nv : 1.05 * std::sqrt((double)ne) + 64.0;
-  const int64_t most = grant + (int64_t)(64.0 * (longest / 4 + 12) / 8) + 1;
-  r.grant = (uint64_t)grant;
-  r.region = (uint64_t)(used / kListShards + most + 1);
-  *lines = (int64_t)r.region * kListShards;
-  return r;
-}
-
-// Ranked by label a list may hold every vertex: a record's 16 bits of cold
-// chunks hold the lists of this many vertices.
-constexpr int64_t kLabelRankMax = 4 * 65535;
-
-// Ranks, chunk starts of lists and entry indices fit their 32 bits.
 bool rank_fits(const xt_ctx* ctx, int64_t nv, int64_t ne, int mode) {
-  const bool by_label = mode == kOrientId;
-  if (nv >= (by_label ? kLabelRankMax : 1ll << 30) || ne >= (1ll << 32)) return false;
-  int64_t lines;
-  rank_list_room(ctx, nv, ne, by_label, 4, &lines);
-  return lines < (1ll << 29);
+  return rank_space_fits(ctx->num_cus, nv, ne, mode == kOrientId);
 }
 
 // Entries per wave of k_rank_count.
@@ -1454,7 +1406,7 @@ int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* o
   XT_TRY(ensure(ctx, s.itcnt, (size_t)nv * sizeof(uint32_t)));
   XT_TRY(ensure(ctx, s.rpart, (size_t)(ne + kWave) * sizeof(uint32_t)));  // a wave reads past a short row
   int64_t lines;
-  const ListRoom lr = rank_list_room(ctx, nv, ne, mode == kOrientId, range ? 4 : 2, &lines);
+  const ListRoom lr = rank_list_room(ctx->num_cus, nv, ne, mode == kOrientId, range ? 4 : 2, &lines);
   XT_TRY(ensure(ctx, s.rlists, (size_t)lines * 128));
   XT_TRY(ensure(ctx, s.rrec, (size_t)nv * sizeof(RankRec)));
   XT_TRY(ensure(ctx, s.rhist, (size_t)(2 * kRankClasses) * sizeof(uint32_t)));
