@@ -129,6 +129,10 @@ int xt_ctx_force_wide(xt_ctx* ctx, int on);
  * makes for its scratch (counts, batches, servers) fail with XT_ERR_NOMEM as
  * hipMalloc running out would.  0 turns it off. */
 int xt_ctx_fail_allocs(xt_ctx* ctx, int n);
+/* The same for the list memory of counts in rank space, which holds the lists of
+ * any simple graph: at most `lines` (0: no limit) of its 128-byte lines are used.
+ * A count that needs more is made with edge tiles.  Changes no result. */
+int xt_ctx_limit_lists(xt_ctx* ctx, int64_t lines);
 
 /* ---- device memory plumbing ------------------------------------------------
  * The CudaMalloc / CudaMemcpyHtoD / CudaMemcpyDtoH / CudaFree /

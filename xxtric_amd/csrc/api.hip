@@ -223,6 +223,9 @@ template int count_device_csr<int32_t>(xt_ctx*, Scratch&, int64_t, int64_t, cons
 template int count_device_csr<int64_t>(xt_ctx*, Scratch&, int64_t, int64_t, const int64_t*, const int64_t*,
                                        uint32_t, hipStream_t, bool, RankUse, const OwnedRange*);
 
+// The count lacks lists (kNoListRoom): what finish_count returns for the caller to count again.
+constexpr int kCountAgain = 2;
+
 // Reads the count, the input-error slots and the timing after a count; sums
 // (nullable, kNumCounters words) gets all counters.
 static int finish_count(xt_ctx* ctx, int64_t nv, uint32_t flags, hipStream_t st, bool timed,
@@ -234,6 +237,7 @@ static int finish_count(xt_ctx* ctx, int64_t nv, uint32_t flags, hipStream_t st,
                                hipMemcpyDeviceToHost, st));
   XT_HIP(ctx, hipStreamSynchronize(st));
   if (h[kBadIds]) return set_err(ctx, XT_ERR_INPUT, "neighbour id out of range [0, nv)");
+  if (h[kNoListRoom]) return kCountAgain;
   if (total) *total = sum_of(h, kSumTotal);
   if (sums) std::memcpy(sums, h, kNumCounters * sizeof(uint64_t));
   int64_t nep = 0, nheavy = 0, ntiles = 0, nwave = 0;
@@ -280,6 +284,21 @@ static int finish_count(xt_ctx* ctx, int64_t nv, uint32_t flags, hipStream_t st,
     }
   }
   return XT_OK;
+}
+
+// One timed count on the context's stream and its results.  The list memory of rank
+// space holds the lists of any simple graph; other input that runs out of it is
+// counted with edge tiles, which need none.
+static int count_and_finish(xt_ctx* ctx, int64_t nv, int64_t ne, const int64_t* off, const int32_t* tails,
+                            uint32_t flags, int64_t max_degree, const OwnedRange* range, uint64_t* total,
+                            uint64_t* per_vertex, uint64_t* sums = nullptr) {
+  int rc = kCountAgain;
+  for (int may_rank = 1; may_rank >= 0 && rc == kCountAgain; may_rank--) {
+    XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, nv, ne, off, tails, flags, ctx->stream, true,
+                                     RankUse{may_rank != 0, max_degree}, range));
+    rc = finish_count(ctx, nv, flags, ctx->stream, true, total, per_vertex, sums);
+  }
+  return rc;
 }
 
 // Host int64 ids -> int32 for the device layout.
@@ -455,6 +474,15 @@ int xt_ctx_force_wide(xt_ctx* ctx, int on) {
   });
 }
 
+int xt_ctx_limit_lists(xt_ctx* ctx, int64_t lines) {
+  return xt_guarded([&]() -> int {
+    if (!ctx || lines < 0) return XT_ERR_ARG;
+    std::lock_guard<std::recursive_mutex> lk(ctx->mu);
+    ctx->list_lines = lines;
+    return XT_OK;
+  });
+}
+
 int xt_dev_alloc(xt_ctx* ctx, size_t bytes, void** out) {
   return xt_guarded([&]() -> int {
     if (!ctx || !out) return XT_ERR_ARG;
@@ -576,8 +604,7 @@ int xt_count_csr(xt_ctx* ctx, int64_t nv, int64_t ne, const int64_t* offsets, co
     int32_t* d_tails = ctx->s.in_tails.as<int32_t>();
     XT_TRY(upload_csr(ctx, nv, ne, offsets, tails, 8, d_off, d_tails, st));
     if (flags & XT_VALIDATE) XT_TRY(validate<int32_t>(ctx, nv, ne, d_off, d_tails, (flags & XT_CHECK_SYMMETRY) != 0, st));
-    XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, nv, ne, d_off, d_tails, flags, st, true, RankUse{true, max_degree}));
-    return finish_count(ctx, nv, flags, st, true, total, per_vertex);
+    return count_and_finish(ctx, nv, ne, d_off, d_tails, flags, max_degree, nullptr, total, per_vertex);
   });
 }
 
@@ -600,14 +627,18 @@ int xt_single_gpu_count(xt_ctx* ctx, int64_t nv, const int64_t* d_indices, const
     // Offsets must be a valid index (and rows sorted) before the chunked
     // kernels search them; the reference launcher assumes the same.
     XT_TRY(validate<int64_t>(ctx, nv, ne, d_indices, d_edge_list, false, st));
-    XT_TRY(count_device_csr<int64_t>(ctx, ctx->s, nv, ne, d_indices, d_edge_list, XT_ORIENT_DEGREE, st, false, RankUse{true, -1}));
-    XT_TRY(launch_add_total(ctx, d_local_count, st));  // nothing if an id was out of range
-    XT_HIP(ctx, hipMemcpyAsync(ctx->h_counters, ctx->s.counters.as<uint64_t>() + kBadIds, sizeof(uint64_t),
-                               hipMemcpyDeviceToHost, st));
-    // The add reads the context's counters, which the next call on this
-    // context (on any stream) clears: it must be done before this returns.
-    XT_HIP(ctx, hipStreamSynchronize(st));
-    if (ctx->h_counters[0]) return set_err(ctx, XT_ERR_INPUT, "neighbour id out of range [0, nv)");
+    for (int may_rank = 1; may_rank >= 0; may_rank--) {  // again with edge tiles where the lists found no room
+      XT_TRY(count_device_csr<int64_t>(ctx, ctx->s, nv, ne, d_indices, d_edge_list, XT_ORIENT_DEGREE, st, false,
+                                       RankUse{may_rank != 0, -1}));
+      XT_TRY(launch_add_total(ctx, d_local_count, st));  // nothing then, or if an id was out of range
+      XT_HIP(ctx, hipMemcpyAsync(ctx->h_counters, ctx->s.counters.p, kNumSlots * sizeof(uint64_t),
+                                 hipMemcpyDeviceToHost, st));
+      // The add reads the context's counters, which the next call on this
+      // context (on any stream) clears: it must be done before this returns.
+      XT_HIP(ctx, hipStreamSynchronize(st));
+      if (ctx->h_counters[kBadIds]) return set_err(ctx, XT_ERR_INPUT, "neighbour id out of range [0, nv)");
+      if (!ctx->h_counters[kNoListRoom]) break;
+    }
     return XT_OK;
   });
 }
@@ -968,9 +999,7 @@ int xt_graph_count(xt_ctx* ctx, xt_graph* g, uint32_t flags, uint64_t* total, ui
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     XT_HIP(ctx, hipSetDevice(ctx->device));
     if (per_vertex && !(flags & XT_PER_VERTEX)) return set_err(ctx, XT_ERR_ARG, "per_vertex needs XT_PER_VERTEX");
-    hipStream_t st = ctx->stream;
-    XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, g->nv, g->ne, g->off, g->tails, flags, st, true, RankUse{true, g->max_degree}));
-    return finish_count(ctx, g->nv, flags, st, true, total, per_vertex);
+    return count_and_finish(ctx, g->nv, g->ne, g->off, g->tails, flags, g->max_degree, nullptr, total, per_vertex);
   });
 }
 
@@ -982,17 +1011,13 @@ int xt_graph_count_owned(xt_ctx* ctx, xt_graph* g, int64_t lo, int64_t hi, uint3
     XT_HIP(ctx, hipSetDevice(ctx->device));
     if (lo < 0 || hi < lo || hi > g->nv) return set_err(ctx, XT_ERR_ARG, "owned range must satisfy 0 <= lo <= hi <= nv");
     if (flags & XT_PER_VERTEX) return set_err(ctx, XT_ERR_ARG, "an owned-range count has no per-vertex output");
-    hipStream_t st = ctx->stream;
     // The owned-range count skips what cannot be owned, so the graph's total
     // takes a count of its own (run first: the timing kept is the owned count's).
-    if (total) {
-      XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, g->nv, g->ne, g->off, g->tails, flags, st, true, RankUse{true, g->max_degree}));
-      XT_TRY(finish_count(ctx, g->nv, flags, st, true, total, nullptr));
-    }
+    if (total)
+      XT_TRY(count_and_finish(ctx, g->nv, g->ne, g->off, g->tails, flags, g->max_degree, nullptr, total, nullptr));
     const OwnedRange range{lo, hi};
-    XT_TRY(count_device_csr<int32_t>(ctx, ctx->s, g->nv, g->ne, g->off, g->tails, flags, st, true, RankUse{true, g->max_degree}, &range));
     uint64_t h[kNumCounters];
-    XT_TRY(finish_count(ctx, g->nv, flags, st, true, nullptr, nullptr, h));
+    XT_TRY(count_and_finish(ctx, g->nv, g->ne, g->off, g->tails, flags, g->max_degree, &range, nullptr, nullptr, h));
     *owned = sum_of(h, kSumOwned);
     if (local) *local = sum_of(h, kSumLocal);
     return XT_OK;

@@ -1931,9 +1931,9 @@ __global__ __launch_bounds__(256) void k_inner(int64_t start, int64_t end, int64
 }
 
 // One wave: a shard of the sum per lane.
-// Adds the total, unless the count met ids out of range.
+// Adds the total, unless the count met ids out of range or lacks lists.
 __global__ void k_add_total(const uint64_t* __restrict__ counters, unsigned long long* __restrict__ out) {
-  if (counters[kBadIds]) return;
+  if (counters[kBadIds] || counters[kNoListRoom]) return;
   const uint64_t t = wave_sum_u64(counters[kNumSlots + (threadIdx.x & (kShards - 1)) * kNumSums + kSumTotal]);
   if (threadIdx.x == 0 && blockIdx.x == 0) atomicAdd(out, (unsigned long long)t);
 }

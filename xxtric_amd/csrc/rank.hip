@@ -482,7 +482,9 @@ __global__ __launch_bounds__(64) void k_rank_lists(int64_t nv, const int64_t* __
       }
       shard = (shard + 1) & (kListShards - 1);
     }
-    return kNoRank;  // only for input that is no simple graph
+    // Only for input that is no simple graph: the caller counts it with edge tiles.
+    atomicAdd((unsigned long long*)&counters[kNoListRoom], 1ull);
+    return kNoRank;
   };
   uint64_t edges = 0;
   for (int64_t batch = blockIdx.x; batch < lr.nbatch; batch += gridDim.x) {  // uniform
@@ -1406,7 +1408,8 @@ int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* o
   XT_TRY(ensure(ctx, s.itcnt, (size_t)nv * sizeof(uint32_t)));
   XT_TRY(ensure(ctx, s.rpart, (size_t)(ne + kWave) * sizeof(uint32_t)));  // a wave reads past a short row
   int64_t lines;
-  const ListRoom lr = rank_list_room(ctx->num_cus, nv, ne, mode == kOrientId, range ? 4 : 2, &lines);
+  ListRoom lr = rank_list_room(ctx->num_cus, nv, ne, mode == kOrientId, range ? 4 : 2, &lines);
+  if (ctx->list_lines > 0 && ctx->list_lines < lines) lr.region = (uint64_t)ctx->list_lines / kListShards;
   XT_TRY(ensure(ctx, s.rlists, (size_t)lines * 128));
   XT_TRY(ensure(ctx, s.rrec, (size_t)nv * sizeof(RankRec)));
   XT_TRY(ensure(ctx, s.rhist, (size_t)(2 * kRankClasses) * sizeof(uint32_t)));

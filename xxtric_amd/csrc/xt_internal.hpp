@@ -46,6 +46,7 @@ enum Slot : int {
   kTileQueue = 8,      // next tile of the persistent group kernel
   kStatMinHeavy = 9,   // same sum over heavy edges only
   kStatHeavyEdges = 10,// number of heavy edges
+  kNoListRoom = 11,    // waves that found no room for their lists (rank space)
   kWaveQueue = 14,     // next wave tile of k_count_waves, one queue per XCD (14..21)
   kNumSlots = 32
 };
@@ -149,6 +150,7 @@ struct xt_ctx {
   int64_t rank_chunks = 0;   // and its chunks of entries, a wave each
   bool force_wide = false;  // use the 64-bit offset layout of graphs with >= 2^32 entries everywhere
   int fail_allocs = 0;      // failure injection: scratch allocations left to fail
+  int64_t list_lines = 0;   // for tests: lines of list memory in rank space, 0 = as many as a simple graph needs
 };
 
 struct xt_graph {
@@ -240,7 +242,8 @@ struct RankUse {
 // The total, the per-vertex counts (pv != nullptr: pv[nv] is written) or an
 // owned range of one graph counted in rank space: adds to the sums kSumTotal
 // (an owned range: kSumOwned and kSumLocal) and kSumEdges.  split_done (nullable) is recorded once the lists stand.  Only
-// for sizes that rank_fits() accepts.
+// for sizes that rank_fits() accepts.  Where the slot kNoListRoom is set afterwards, the
+// sums lack the lists of some vertices: the graph is to be counted with edge tiles.
 bool rank_fits(const xt_ctx* ctx, int64_t nv, int64_t ne, int mode);
 template <typename T>
 int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* off, const T* tails, int mode,
