@@ -461,26 +461,28 @@ __global__ __launch_bounds__(kBlock) void k_validate(int64_t nv, int64_t ne,
   __shared__ int64_t s_off[kOffCap + 1];
   __shared__ int64_t s_lohi[2];
   if (counters[kBadOff]) return;  // whole grid: k_check_offsets found no index to walk
-  const int64_t eb = (int64_t)blockIdx.x * kChunk;
-  const int64_t ee = min(ne, eb + (int64_t)kChunk);
-  const ChunkRows r = chunk_rows(off, nv, eb, ee, s_off, s_lohi);
   uint32_t bad_id = 0, bad_row = 0, asym = 0;
-  for (int j = 0; j < kPerThread; j++) {
-    const int64_t e = eb + (int64_t)j * kBlock + threadIdx.x;
-    if (e >= ee) break;
-    const int64_t u = chunk_row_of(r, s_off, off, e);
-    const int64_t v = (int64_t)tails[e];
-    if (v < 0 || v >= nv) {
-      bad_id++;
-      continue;
+  for (int64_t eb = (int64_t)blockIdx.x * kChunk; eb < ne; eb += (int64_t)gridDim.x * kChunk) {  // uniform
+    const int64_t ee = min(ne, eb + (int64_t)kChunk);
+    const ChunkRows r = chunk_rows(off, nv, eb, ee, s_off, s_lohi);
+    for (int j = 0; j < kPerThread; j++) {
+      const int64_t e = eb + (int64_t)j * kBlock + threadIdx.x;
+      if (e >= ee) break;
+      const int64_t u = chunk_row_of(r, s_off, off, e);
+      const int64_t v = (int64_t)tails[e];
+      if (v < 0 || v >= nv) {
+        bad_id++;
+        continue;
+      }
+      const int64_t rend = chunk_off(r, s_off, off, u + 1);
+      if (e + 1 < rend && !((int64_t)tails[e + 1] > v)) bad_row++;
+      if (symmetry) {
+        const int64_t b0 = off[v], b1 = off[v + 1];
+        const int64_t p = lower_bound_dev<T>(tails, b0, b1, (T)u);
+        if (p >= b1 || (int64_t)tails[p] != u) asym++;
+      }
     }
-    const int64_t rend = chunk_off(r, s_off, off, u + 1);
-    if (e + 1 < rend && !((int64_t)tails[e + 1] > v)) bad_row++;
-    if (symmetry) {
-      const int64_t b0 = off[v], b1 = off[v + 1];
-      const int64_t p = lower_bound_dev<T>(tails, b0, b1, (T)u);
-      if (p >= b1 || (int64_t)tails[p] != u) asym++;
-    }
+    __syncthreads();  // the staged offsets are read
   }
   if (bad_id) atomicAdd((unsigned long long*)&counters[kBadIds], (unsigned long long)bad_id);
   if (bad_row) atomicAdd((unsigned long long*)&counters[kBadRows], (unsigned long long)bad_row);
@@ -488,7 +490,12 @@ __global__ __launch_bounds__(kBlock) void k_validate(int64_t nv, int64_t ne,
 }
 
 // Offsets check followed by the entry checks (which do nothing where it failed);
-// reads the verdict back (syncs).
+// reads the verdict back (syncs).  The entry checks are launched before it is known
+// that ne is the end of an index, and a device CSR's last offset may be anything: the
+// grid stops at kValidateBlocks (any graph below 2^31 entries has a workgroup per
+// chunk) and strides from there.
+constexpr int64_t kValidateBlocks = int64_t(1) << 20;
+
 template <typename T>
 int validate(xt_ctx* ctx, int64_t nv, int64_t ne, const int64_t* off, const T* tails,
              bool symmetry, hipStream_t st, uint64_t* counters) {
@@ -498,8 +505,9 @@ int validate(xt_ctx* ctx, int64_t nv, int64_t ne, const int64_t* off, const T* t
                      counters);
   XT_HIP(ctx, hipGetLastError());
   if (ne > 0) {
-    const int64_t nchunks = (ne + kChunk - 1) / kChunk;
-    hipLaunchKernelGGL((k_validate<T>), dim3((unsigned)nchunks), dim3(kBlock), 0, st, nv, ne, off,
+    const int64_t nchunks = ne / kChunk + (ne % kChunk != 0);
+    const int64_t grid = nchunks < kValidateBlocks ? nchunks : kValidateBlocks;
+    hipLaunchKernelGGL((k_validate<T>), dim3((unsigned)grid), dim3(kBlock), 0, st, nv, ne, off,
                        tails, symmetry ? 1 : 0, counters);
     XT_HIP(ctx, hipGetLastError());
   }
