@@ -61,14 +61,43 @@ static int index32() {
     bool ends = true;
     for (int64_t items = 1; items <= 300 && ends; items++) ends = walk((uint32_t)(ne - items), (uint32_t)ne) == items;
     for (bool by_label : {false, true}) {
-      const bool fits = xt::rank_space_fits(256, by_label ? 250000 : nv, ne, by_label);
+      const bool fits = xt::rank_space_fits(256, by_label ? 250000 : nv, ne, by_label ? 256 : -1);
       CHECK(!fits || ends);
       CHECK(by_label || fits == (ne < xt::kIndex32Entries));
     }
     CHECK(ends || ne >= xt::kIndex32Entries);
   }
   CHECK(walk((uint32_t)(top - 110), (uint32_t)(top - 10)) == -1);  // what the limit keeps out
-  CHECK(!xt::rank_space_fits(256, nv, top, false) && !xt::rank_space_fits(256, nv, top + 5, false));
+  CHECK(!xt::rank_space_fits(256, nv, top, -1) && !xt::rank_space_fits(256, nv, top + 5, -1));
+  return 0;
+}
+
+// Chunks a list of d ids is given, at most: eight hot ids or four cold ones to a
+// chunk, each part rounded up, then in full, half, quarter or eighth lines.  The
+// worst split has one id in every part but the last, cold one.
+static int64_t most_chunks(int64_t d, int parts) {
+  if (d < 2) return 0;  // no pair, no list
+  const int64_t others = parts - 1 < d - 1 ? parts - 1 : d - 1;
+  const int64_t t = others + (d - others + 3) / 4;
+  return t <= 2 ? t : t <= 4 ? 4 : (t + 7) / 8 * 8;
+}
+
+static int lists() {
+  for (int cus : {64, 256, 304})
+    for (int64_t nv : {64, 1000, 20001, 100000, 262139})
+      for (int64_t d : {1, 2, 31, 32, 33, 100, 255, 256}) {
+        if (d >= nv) continue;
+        const int64_t ne = nv * d;
+        for (int parts : {2, 4}) {
+          int64_t lines = 0;
+          const xt::ListRoom r = xt::rank_list_room(cus, nv, ne, d, parts, &lines);
+          // Room for every vertex's list of half its row and for a wave of whole rows in each region ...
+          CHECK(lines * 8 >= nv * most_chunks(d / 2, parts));
+          CHECK((int64_t)r.region * 8 >= r.rows * most_chunks(d, parts));
+          // ... but of that order: 6 bytes an entry, 500 a vertex and, for the waves' draws, 4 MB.
+          CHECK(lines * 128 <= 6 * ne + 500 * nv + (int64_t(4) << 20) * cus / 256 + (int64_t(1) << 20));
+        }
+      }
   return 0;
 }
 
@@ -76,7 +105,7 @@ int main(int argc, char** argv) {
   const struct {
     const char* name;
     int (*run)();
-  } groups[] = {{"offsets", offsets}, {"index32", index32}};
+  } groups[] = {{"offsets", offsets}, {"index32", index32}, {"lists", lists}};
   if (argc != 2) return 2;
   for (const auto& g : groups)
     if (std::strcmp(argv[1], g.name) == 0) {

@@ -23,7 +23,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("group", ["offsets", "index32"])
+@pytest.mark.parametrize("group", ["offsets", "index32", "lists"])
 def test_bounds(exe, group):
     r = subprocess.run([exe, group], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr

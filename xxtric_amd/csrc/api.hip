@@ -181,7 +181,7 @@ constexpr int64_t kRankIdDegree = 256;
 static bool ranks(const xt_ctx* ctx, int64_t nv, int64_t ne, int mode, bool per_vertex, int64_t max_degree) {
   if (mode == kOrientId && (max_degree < 0 || max_degree > kRankIdDegree)) return false;
   if (per_vertex && ne >= kRankPvEntries) return false;
-  return !edge_tile_knobs(ctx) && ne > 0 && rank_fits(ctx, nv, ne, mode);
+  return !edge_tile_knobs(ctx) && ne > 0 && rank_fits(ctx, nv, ne, mode, max_degree);
 }
 
 template <typename T>
@@ -198,7 +198,7 @@ int count_device_csr(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int6
   }
   if (rank.may && ranks(ctx, nv, ne, mode, pv != nullptr, rank.max_degree)) {
     if (timed) XT_HIP(ctx, hipEventRecord(ctx->ev[kEvStart], st));
-    XT_TRY(rank_count<T>(ctx, s, nv, ne, off, tails, mode, pv, range, st, timed ? ctx->ev[kEvOriented] : nullptr));
+    XT_TRY(rank_count<T>(ctx, s, nv, ne, off, tails, mode, rank.max_degree, pv, range, st, timed ? ctx->ev[kEvOriented] : nullptr));
     if (timed) XT_HIP(ctx, hipEventRecord(ctx->ev[kEvCounted], st));
     ctx->last_ranked = true;
     return XT_OK;

@@ -1386,8 +1386,8 @@ static unsigned rank_grid(int64_t n, int per, int64_t cap) {
   return (unsigned)g;
 }
 
-bool rank_fits(const xt_ctx* ctx, int64_t nv, int64_t ne, int mode) {
-  return rank_space_fits(ctx->num_cus, nv, ne, mode == kOrientId);
+bool rank_fits(const xt_ctx* ctx, int64_t nv, int64_t ne, int mode, int64_t max_degree) {
+  return rank_space_fits(ctx->num_cus, nv, ne, mode == kOrientId ? max_degree : -1);
 }
 
 // Entries per wave of k_rank_count.
@@ -1399,7 +1399,7 @@ static int64_t rank_chunk(const xt_ctx* ctx, int64_t ne) {
 
 template <typename T>
 int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* off, const T* tails, int mode,
-               uint64_t* pv, const OwnedRange* range, hipStream_t st, hipEvent_t split_done) {
+               int64_t max_degree, uint64_t* pv, const OwnedRange* range, hipStream_t st, hipEvent_t split_done) {
   const int64_t S = rank_chunk(ctx, ne);
   const int64_t nch = (ne + S - 1) / S, nchunks = (ne + kChunk - 1) / kChunk;
   XT_TRY(ensure(ctx, s.crows, (size_t)(2 * nch) * sizeof(int32_t)));
@@ -1408,7 +1408,7 @@ int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* o
   XT_TRY(ensure(ctx, s.itcnt, (size_t)nv * sizeof(uint32_t)));
   XT_TRY(ensure(ctx, s.rpart, (size_t)(ne + kWave) * sizeof(uint32_t)));  // a wave reads past a short row
   int64_t lines;
-  ListRoom lr = rank_list_room(ctx->num_cus, nv, ne, mode == kOrientId, range ? 4 : 2, &lines);
+  ListRoom lr = rank_list_room(ctx->num_cus, nv, ne, mode == kOrientId ? max_degree : -1, range ? 4 : 2, &lines);
   if (ctx->list_lines > 0 && ctx->list_lines < lines) lr.region = (uint64_t)ctx->list_lines / kListShards;
   XT_TRY(ensure(ctx, s.rlists, (size_t)lines * 128));
   XT_TRY(ensure(ctx, s.rrec, (size_t)nv * sizeof(RankRec)));
@@ -1477,9 +1477,9 @@ int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* o
   return XT_OK;
 }
 
-template int rank_count<int32_t>(xt_ctx*, Scratch&, int64_t, int64_t, const int64_t*, const int32_t*, int, uint64_t*,
+template int rank_count<int32_t>(xt_ctx*, Scratch&, int64_t, int64_t, const int64_t*, const int32_t*, int, int64_t, uint64_t*,
                                  const OwnedRange*, hipStream_t, hipEvent_t);
-template int rank_count<int64_t>(xt_ctx*, Scratch&, int64_t, int64_t, const int64_t*, const int64_t*, int, uint64_t*,
+template int rank_count<int64_t>(xt_ctx*, Scratch&, int64_t, int64_t, const int64_t*, const int64_t*, int, int64_t, uint64_t*,
                                  const OwnedRange*, hipStream_t, hipEvent_t);
 
 }  // namespace xt

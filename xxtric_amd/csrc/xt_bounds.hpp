@@ -44,9 +44,10 @@ struct ListRoom {
 // parts rounded up to chunks, then to list_room; two parts each: d / 4 + 11.5), a wave's lists at a time
 // rounded up to a line.  Grants but a wave's last are used to three quarters.
 // A region is left for the next when a request does not fit, so each may lose
-// one request: a grant, or 64 of the longest lists (at most 1.02 sqrt(ne) ids,
-// since out-neighbours have about the vertex's degree or more).
-inline ListRoom rank_list_room(int num_cus, int64_t nv, int64_t ne, bool by_label, int parts, int64_t* lines) {
+// one request: a grant, or 64 of the longest lists.  Ranked by degree these have at
+// most 1.02 sqrt(ne) ids, since out-neighbours have about the vertex's degree or
+// more; ranked by label (max_degree >= 0) a list is at most its row.
+inline ListRoom rank_list_room(int num_cus, int64_t nv, int64_t ne, int64_t max_degree, int parts, int64_t* lines) {
   ListRoom r;
   const int64_t waves = (int64_t)num_cus * 16;
   r.rows = 64;
@@ -61,7 +62,7 @@ inline ListRoom rank_list_room(int num_cus, int64_t nv, int64_t ne, bool by_labe
   const int64_t need = chunks / 8 + r.nbatch + 1;
   const int64_t grant = need / (waves * 32) < 8 ? 8 : need / (waves * 32);
   const int64_t used = need + need / 3 + (r.nbatch < waves ? r.nbatch : waves) * grant;
-  const double longest = by_label ? (double)nv : 1.05 * std::sqrt((double)ne) + 64.0;
+  const double longest = max_degree >= 0 ? (double)max_degree : 1.05 * std::sqrt((double)ne) + 64.0;
   const int64_t most = grant + (int64_t)(64.0 * (longest / 4 + 12) / 8) + 1;
   r.grant = (uint64_t)grant;
   r.region = (uint64_t)(used / kListShards + most + 1);
@@ -74,11 +75,12 @@ inline ListRoom rank_list_room(int num_cus, int64_t nv, int64_t ne, bool by_labe
 constexpr int64_t kLabelRankMax = 4 * 65535;
 
 // Ranks, chunk starts of lists and entry indices fit their 32 bits (entries also a
-// wave past the last).
-inline bool rank_space_fits(int num_cus, int64_t nv, int64_t ne, bool by_label) {
-  if (nv >= (by_label ? kLabelRankMax : 1ll << 30) || ne >= kIndex32Entries) return false;
+// wave past the last).  max_degree: the longest row where vertices are ranked by
+// label, -1 where by degree.
+inline bool rank_space_fits(int num_cus, int64_t nv, int64_t ne, int64_t max_degree) {
+  if (nv >= (max_degree >= 0 ? kLabelRankMax : 1ll << 30) || ne >= kIndex32Entries) return false;
   int64_t lines;
-  rank_list_room(num_cus, nv, ne, by_label, 4, &lines);
+  rank_list_room(num_cus, nv, ne, max_degree, 4, &lines);
   return lines < (1ll << 29);
 }
 

@@ -242,12 +242,12 @@ struct RankUse {
 // The total, the per-vertex counts (pv != nullptr: pv[nv] is written) or an
 // owned range of one graph counted in rank space: adds to the sums kSumTotal
 // (an owned range: kSumOwned and kSumLocal) and kSumEdges.  split_done (nullable) is recorded once the lists stand.  Only
-// for sizes that rank_fits() accepts.  Where the slot kNoListRoom is set afterwards, the
+// for sizes that rank_fits() accepts.  max_degree is read in id orientation alone.  Where the slot kNoListRoom is set afterwards, the
 // sums lack the lists of some vertices: the graph is to be counted with edge tiles.
-bool rank_fits(const xt_ctx* ctx, int64_t nv, int64_t ne, int mode);
+bool rank_fits(const xt_ctx* ctx, int64_t nv, int64_t ne, int mode, int64_t max_degree);
 template <typename T>
 int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* off, const T* tails, int mode,
-               uint64_t* pv, const OwnedRange* range, hipStream_t st, hipEvent_t split_done);
+               int64_t max_degree, uint64_t* pv, const OwnedRange* range, hipStream_t st, hipEvent_t split_done);
 
 // Whole single-graph count on the device (orientation + intersection).
 // rank: whether it may be counted in rank space, and the longest row (-1: unknown).
