@@ -197,6 +197,7 @@ int count_device_csr(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int6
     pv = s.pv.as<uint64_t>();
   }
   if (rank.may && ranks(ctx, nv, ne, mode, pv != nullptr, rank.max_degree)) {
+    XT_TRY(rank_reserve(ctx, s, nv, ne, mode, rank.max_degree, pv != nullptr, range != nullptr));
     if (timed) XT_HIP(ctx, hipEventRecord(ctx->ev[kEvStart], st));
     XT_TRY(rank_count<T>(ctx, s, nv, ne, off, tails, mode, rank.max_degree, pv, range, st, timed ? ctx->ev[kEvOriented] : nullptr));
     if (timed) XT_HIP(ctx, hipEventRecord(ctx->ev[kEvCounted], st));

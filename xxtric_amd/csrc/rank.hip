@@ -1397,26 +1397,41 @@ static int64_t rank_chunk(const xt_ctx* ctx, int64_t ne) {
   return S;
 }
 
-template <typename T>
-int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* off, const T* tails, int mode,
-               int64_t max_degree, uint64_t* pv, const OwnedRange* range, hipStream_t st, hipEvent_t split_done) {
+// The list memory of a count, cut short for tests.
+static ListRoom list_room(const xt_ctx* ctx, int64_t nv, int64_t ne, int mode, int64_t max_degree, bool range,
+                          int64_t* lines) {
+  ListRoom lr = rank_list_room(ctx->num_cus, nv, ne, mode == kOrientId ? max_degree : -1, range ? 4 : 2, lines);
+  if (ctx->list_lines > 0 && ctx->list_lines < *lines) lr.region = (uint64_t)ctx->list_lines / kListShards;
+  return lr;
+}
+
+int rank_reserve(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, int mode, int64_t max_degree, bool per_vertex,
+                 bool range) {
   const int64_t S = rank_chunk(ctx, ne);
-  const int64_t nch = (ne + S - 1) / S, nchunks = (ne + kChunk - 1) / kChunk;
-  XT_TRY(ensure(ctx, s.crows, (size_t)(2 * nch) * sizeof(int32_t)));
+  XT_TRY(ensure(ctx, s.crows, (size_t)(2 * ((ne + S - 1) / S)) * sizeof(int32_t)));
   XT_TRY(ensure(ctx, s.rank, (size_t)nv * sizeof(uint32_t)));
   XT_TRY(ensure(ctx, s.ocount, (size_t)nv * sizeof(uint64_t)));
   XT_TRY(ensure(ctx, s.itcnt, (size_t)nv * sizeof(uint32_t)));
   XT_TRY(ensure(ctx, s.rpart, (size_t)(ne + kWave) * sizeof(uint32_t)));  // a wave reads past a short row
   int64_t lines;
-  ListRoom lr = rank_list_room(ctx->num_cus, nv, ne, mode == kOrientId ? max_degree : -1, range ? 4 : 2, &lines);
-  if (ctx->list_lines > 0 && ctx->list_lines < lines) lr.region = (uint64_t)ctx->list_lines / kListShards;
+  list_room(ctx, nv, ne, mode, max_degree, range, &lines);
   XT_TRY(ensure(ctx, s.rlists, (size_t)lines * 128));
   XT_TRY(ensure(ctx, s.rrec, (size_t)nv * sizeof(RankRec)));
   XT_TRY(ensure(ctx, s.rhist, (size_t)(2 * kRankClasses) * sizeof(uint32_t)));
   if (range) XT_TRY(ensure(ctx, s.vrec, (size_t)nv * sizeof(uint64_t)));
+  if (per_vertex) XT_TRY(ensure(ctx, s.rorig, (size_t)nv * sizeof(uint32_t)));
+  return XT_OK;
+}
+
+template <typename T>
+int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* off, const T* tails, int mode,
+               int64_t max_degree, uint64_t* pv, const OwnedRange* range, hipStream_t st, hipEvent_t split_done) {
+  const int64_t S = rank_chunk(ctx, ne);
+  const int64_t nch = (ne + S - 1) / S, nchunks = (ne + kChunk - 1) / kChunk;
+  int64_t lines;
+  const ListRoom lr = list_room(ctx, nv, ne, mode, max_degree, range != nullptr, &lines);
   uint64_t* oc1 = range ? s.vrec.as<uint64_t>() : nullptr;
   const int64_t rlo = range ? range->lo : 0, rhi = range ? range->hi : 0;
-  if (pv) XT_TRY(ensure(ctx, s.rorig, (size_t)nv * sizeof(uint32_t)));
   uint32_t* orig = pv ? s.rorig.as<uint32_t>() : nullptr;
   unsigned long long* pvp = reinterpret_cast<unsigned long long*>(pv);
   uint64_t* counters = s.counters.as<uint64_t>();

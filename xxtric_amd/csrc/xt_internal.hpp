@@ -245,6 +245,9 @@ struct RankUse {
 // for sizes that rank_fits() accepts.  max_degree is read in id orientation alone.  Where the slot kNoListRoom is set afterwards, the
 // sums lack the lists of some vertices: the graph is to be counted with edge tiles.
 bool rank_fits(const xt_ctx* ctx, int64_t nv, int64_t ne, int mode, int64_t max_degree);
+// Grows the scratch that rank_count uses (which grows none itself).
+int rank_reserve(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, int mode, int64_t max_degree, bool per_vertex,
+                 bool range);
 template <typename T>
 int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* off, const T* tails, int mode,
                int64_t max_degree, uint64_t* pv, const OwnedRange* range, hipStream_t st, hipEvent_t split_done);
