@@ -82,7 +82,9 @@ int xt_last_timing(const xt_ctx* ctx, xt_timing* out);
  * graphs have at most 65535 vertices are counted over 16-bit lists.  The knobs
  * below belong to the edge tiles that all other counts use; a context on which
  * one of them is away from its default uses edge tiles for all of them.  A context
- * keeps up to 512 MiB of device memory of its graph builds until it is destroyed.
+ * keeps its counts' scratch and up to 512 MiB of device memory of its graph builds
+ * until it is destroyed, or until an allocation of its own fails and the running call
+ * does not use them.
  * Tuning knobs (set by xxtric_amd.autotune from measurements; 0 keeps the
  * current value): light_cut -- edges whose two out-lists are both at most this
  * long are intersected one per thread, the rest by the group kernel or wave
@@ -129,8 +131,12 @@ int xt_ctx_force_wide(xt_ctx* ctx, int on);
  * makes for its scratch (counts, batches, servers) fail with XT_ERR_NOMEM as
  * hipMalloc running out would.  0 turns it off. */
 int xt_ctx_fail_allocs(xt_ctx* ctx, int n);
-/* The same for the list memory of counts in rank space, which holds the lists of
- * any simple graph: at most `lines` (0: no limit) of its 128-byte lines are used.
+/* The next n device allocations of the context fail at their first try, as hipMalloc
+ * running out would; each is tried once more if the context could give back memory
+ * that it keeps from earlier calls and the running one does not use. */
+int xt_ctx_fail_tries(xt_ctx* ctx, int n);
+/* For tests: of the list memory of counts in rank space, which holds the lists of
+ * any simple graph, at most `lines` (0: no limit) 128-byte lines are used.
  * A count that needs more is made with edge tiles.  Changes no result. */
 int xt_ctx_limit_lists(xt_ctx* ctx, int64_t lines);
 

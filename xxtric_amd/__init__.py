@@ -105,6 +105,10 @@ class Context:
         """Failure injection: the next n scratch allocations fail with XT_ERR_NOMEM."""
         self._check(self._L.xt_ctx_fail_allocs(self.h, int(n)))
 
+    def fail_tries(self, n):
+        """Failure injection: the next n allocations fail once, before kept memory is given back."""
+        self._check(self._L.xt_ctx_fail_tries(self.h, int(n)))
+
     def limit_lists(self, lines):
         """For tests: use at most this many lines of list memory in rank space (0: no limit)."""
         self._check(self._L.xt_ctx_limit_lists(self.h, int(lines)))

@@ -95,6 +95,7 @@ _SIGS = {
     "xt_ctx_tune_hash": (_int, [_p, _int]),
     "xt_ctx_force_wide": (_int, [_p, _int]),
     "xt_ctx_fail_allocs": (_int, [_p, _int]),
+    "xt_ctx_fail_tries": (_int, [_p, _int]),
     "xt_ctx_limit_lists": (_int, [_p, _i64]),
     "xt_dev_alloc": (_int, [_p, ctypes.c_size_t, _pp]),
     "xt_dev_free": (_int, [_p, _p]),

@@ -87,6 +87,42 @@ int hip_err(xt_ctx* ctx, hipError_t e, const char* what) {
   return set_err(ctx, code, std::string(what) + ": " + hipGetErrorString(e));
 }
 
+// Frees kept memory that no running call uses: of graph builds, and the scratch of
+// the other way to count (edge tiles or rank space).  Returns whether there was any.
+static bool give_back(xt_ctx* ctx) {
+  std::lock_guard<std::recursive_mutex> lk(ctx->mu);
+  Scratch& s = ctx->s;
+  DevBuf* tiles[] = {&s.deg, &s.dplus, &s.tailcnt, &s.qscan, &s.ooff, &s.otails, &s.oflags, &s.items, &s.tileoff, &s.tiledesc};
+  DevBuf* ranks[] = {&s.rhist, &s.rank, &s.rorig, &s.ocount, &s.rpart, &s.rlists, &s.rrec};
+  bool any = false;
+  auto drop = [&](DevBuf& b) {
+    if (!b.p || b.fixed || (!any && hipDeviceSynchronize() != hipSuccess)) return;  // queued work may still use it
+    (void)hipFree(b.p);
+    b = DevBuf{};
+    any = true;
+  };
+  if (ctx->build_users == 0) drop(ctx->build);
+  if (ctx->ranking)
+    for (DevBuf* b : tiles) drop(*b);
+  else
+    for (DevBuf* b : ranks) drop(*b);
+  return any;
+}
+
+hipError_t dev_malloc(xt_ctx* ctx, void** p, size_t bytes) {
+  *p = nullptr;
+  hipError_t e = hipErrorOutOfMemory;
+  if (ctx->fail_tries > 0)
+    ctx->fail_tries--;
+  else
+    e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory) return e;
+  (void)hipGetLastError();  // not for the next launch to find
+  if (give_back(ctx)) e = hipMalloc(p, bytes);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
+}
+
 int ensure(xt_ctx* ctx, DevBuf& b, size_t bytes) {
   if (bytes == 0) bytes = 8;
   if (b.bytes >= bytes) return XT_OK;
@@ -101,12 +137,12 @@ int ensure(xt_ctx* ctx, DevBuf& b, size_t bytes) {
     b.bytes = 0;
   }
   const size_t want = (bytes + ((size_t)1 << 21) - 1) & ~(((size_t)1 << 21) - 1);
-  if (ctx && ctx->fail_allocs > 0) {
+  if (ctx->fail_allocs > 0) {
     ctx->fail_allocs--;
     return set_err(ctx, XT_ERR_NOMEM, std::string("device allocation of ") + std::to_string(want) +
                                           " bytes failed (injected)");
   }
-  hipError_t e = hipMalloc(&b.p, want);
+  hipError_t e = dev_malloc(ctx, &b.p, want);
   if (e != hipSuccess) {
     b.p = nullptr;
     return set_err(ctx, XT_ERR_NOMEM, std::string("device allocation of ") + std::to_string(want) +
@@ -475,6 +511,15 @@ int xt_ctx_force_wide(xt_ctx* ctx, int on) {
   });
 }
 
+int xt_ctx_fail_tries(xt_ctx* ctx, int n) {
+  return xt_guarded([&]() -> int {
+    if (!ctx || n < 0) return XT_ERR_ARG;
+    std::lock_guard<std::recursive_mutex> lk(ctx->mu);
+    ctx->fail_tries = n;
+    return XT_OK;
+  });
+}
+
 int xt_ctx_limit_lists(xt_ctx* ctx, int64_t lines) {
   return xt_guarded([&]() -> int {
     if (!ctx || lines < 0) return XT_ERR_ARG;
@@ -490,7 +535,7 @@ int xt_dev_alloc(xt_ctx* ctx, size_t bytes, void** out) {
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     XT_HIP(ctx, hipSetDevice(ctx->device));
     *out = nullptr;
-    XT_HIP(ctx, hipMalloc(out, bytes > 0 ? bytes : 1));
+    XT_HIP(ctx, dev_malloc(ctx, out, bytes > 0 ? bytes : 1));
     return XT_OK;
   });
 }
@@ -736,8 +781,8 @@ int xt_graph_from_csr(xt_ctx* ctx, int64_t nv, int64_t ne, const int64_t* offset
     g->max_degree = (flags & XT_CLEAN) ? -1 : max_degree;  // cleaning adds reverse entries
     g->nv = nv;
     g->ne = ne;
-    hipError_t e = hipMalloc(&g->off, (size_t)(nv + 1) * sizeof(int64_t));
-    if (e == hipSuccess) e = hipMalloc(&g->tails, (size_t)(ne > 0 ? ne : 1) * sizeof(int32_t));
+    hipError_t e = dev_malloc(ctx, &g->off, (size_t)(nv + 1) * sizeof(int64_t));
+    if (e == hipSuccess) e = dev_malloc(ctx, &g->tails, (size_t)(ne > 0 ? ne : 1) * sizeof(int32_t));
     if (e != hipSuccess) {
       if (g->off) (void)hipFree(g->off);
       delete g;
@@ -845,8 +890,8 @@ static int vite_to_device(xt_ctx* ctx, std::FILE* f, xt_graph* g) {
     return set_err(ctx, XT_ERR_INPUT, "vite: need 1 <= nv < 2^31-1 and ne >= 0");
   g->nv = nv;
   g->ne = ne;
-  XT_HIP(ctx, hipMalloc(&g->off, (size_t)(nv + 1) * sizeof(int64_t)));
-  XT_HIP(ctx, hipMalloc(&g->tails, (size_t)(ne > 0 ? ne : 1) * sizeof(int32_t)));
+  XT_HIP(ctx, dev_malloc(ctx, &g->off, (size_t)(nv + 1) * sizeof(int64_t)));
+  XT_HIP(ctx, dev_malloc(ctx, &g->tails, (size_t)(ne > 0 ? ne : 1) * sizeof(int32_t)));
   constexpr int64_t kBlock = 1 << 22;  // elements per pinned block
   struct Rec {
     E tail;
@@ -964,7 +1009,9 @@ int xt_count_edges(xt_ctx* ctx, int64_t nv, int64_t m, const int64_t* src, const
     xt_graph g;
     int rc = graph_from_edges(ctx, nv, m, src, dst, true, &g);
     if (rc == XT_OK) rc = xt_graph_count(ctx, &g, flags, total, per_vertex);
-    if (!g.lent) {
+    if (g.lent) {
+      ctx->build_users--;
+    } else {
       if (g.off) (void)hipFree(g.off);
       if (g.tails) (void)hipFree(g.tails);
     }

@@ -505,14 +505,14 @@ int xt_batch_create(xt_ctx* ctx, int64_t max_vertices, int64_t max_edges, int64_
     hipError_t e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreate(&b->ev0);
     if (e == hipSuccess) e = hipEventCreate(&b->ev1);
-    if (e == hipSuccess) e = hipMalloc(&b->goff, (size_t)(max_vertices + 1) * sizeof(int64_t));
-    if (e == hipSuccess) e = hipMalloc(&b->gtails, (size_t)max_edges * sizeof(int32_t));
-    if (e == hipSuccess) e = hipMalloc(&b->gid, (size_t)max_vertices * sizeof(int32_t));
-    if (e == hipSuccess) e = hipMalloc(&b->gbase, (size_t)max_graphs * sizeof(int32_t));
-    if (e == hipSuccess) e = hipMalloc(&b->loff, (size_t)(max_vertices + max_graphs) * sizeof(int64_t));
-    if (e == hipSuccess) e = hipMalloc(&b->ltails, (size_t)max_edges * sizeof(int32_t));
-    if (e == hipSuccess) e = hipMalloc(&b->gtotal, (size_t)max_graphs * sizeof(uint64_t));
-    if (e == hipSuccess) e = hipMalloc(&b->ptotal, (size_t)max_graphs * sizeof(uint64_t));
+    if (e == hipSuccess) e = dev_malloc(ctx, &b->goff, (size_t)(max_vertices + 1) * sizeof(int64_t));
+    if (e == hipSuccess) e = dev_malloc(ctx, &b->gtails, (size_t)max_edges * sizeof(int32_t));
+    if (e == hipSuccess) e = dev_malloc(ctx, &b->gid, (size_t)max_vertices * sizeof(int32_t));
+    if (e == hipSuccess) e = dev_malloc(ctx, &b->gbase, (size_t)max_graphs * sizeof(int32_t));
+    if (e == hipSuccess) e = dev_malloc(ctx, &b->loff, (size_t)(max_vertices + max_graphs) * sizeof(int64_t));
+    if (e == hipSuccess) e = dev_malloc(ctx, &b->ltails, (size_t)max_edges * sizeof(int32_t));
+    if (e == hipSuccess) e = dev_malloc(ctx, &b->gtotal, (size_t)max_graphs * sizeof(uint64_t));
+    if (e == hipSuccess) e = dev_malloc(ctx, &b->ptotal, (size_t)max_graphs * sizeof(uint64_t));
     if (e != hipSuccess) {
       int rc = hip_err(ctx, e, "xt_batch_create");
       batch_free(b);

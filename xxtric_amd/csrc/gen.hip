@@ -126,6 +126,7 @@ struct BuildMem {
   int64_t* off = nullptr;
   int32_t* tails = nullptr;
   void* own = nullptr;  // not kept
+  bool kept = false;    // in the context's memory, which counts its users
 };
 
 static int build_mem(xt_ctx* ctx, int64_t nk, int64_t nv, int key_bits, size_t input_bytes, bool with_csr, BuildMem* m) {
@@ -142,7 +143,7 @@ static int build_mem(xt_ctx* ctx, int64_t nk, int64_t nv, int key_bits, size_t i
   if (with_csr) total += offs + tails;
   char* p = nullptr;
   if (total > kBuildKeep) {
-    XT_HIP(ctx, hipMalloc(&m->own, total));
+    XT_HIP(ctx, dev_malloc(ctx, &m->own, total));
     p = static_cast<char*>(m->own);
   } else {
     DevBuf& b = ctx->build;
@@ -152,10 +153,12 @@ static int build_mem(xt_ctx* ctx, int64_t nk, int64_t nv, int key_bits, size_t i
         XT_HIP(ctx, hipFree(b.p));
         b = DevBuf{};
       }
-      XT_HIP(ctx, hipMalloc(&b.p, total));
+      XT_HIP(ctx, dev_malloc(ctx, &b.p, total));
       b.bytes = total;
     }
     p = b.as<char>();
+    m->kept = true;
+    ctx->build_users++;
   }
   m->ka = reinterpret_cast<uint64_t*>(p);
   m->kb = reinterpret_cast<uint64_t*>(p + keys);
@@ -167,9 +170,11 @@ static int build_mem(xt_ctx* ctx, int64_t nk, int64_t nv, int key_bits, size_t i
   return XT_OK;
 }
 
-static void build_mem_done(BuildMem& m) {
+static void build_mem_done(xt_ctx* ctx, BuildMem& m) {
   if (m.own) (void)hipFree(m.own);
+  if (m.kept) ctx->build_users--;
   m.own = nullptr;
+  m.kept = false;
 }
 
 // Sorted, merged (u << bits | v) keys (m.ka) -> CSR: radix sort over key_bits bits,
@@ -199,8 +204,8 @@ static int build_csr_from_keys(xt_ctx* ctx, const BuildMem& m, int64_t nk, int k
     g->off = m.off;
     g->tails = m.tails;
   } else {
-    XT_HIP(ctx, hipMalloc(&g->off, (size_t)(nv + 1) * sizeof(int64_t)));
-    XT_HIP(ctx, hipMalloc(&g->tails, (size_t)(ne > 0 ? ne : 1) * sizeof(int32_t)));
+    XT_HIP(ctx, dev_malloc(ctx, &g->off, (size_t)(nv + 1) * sizeof(int64_t)));
+    XT_HIP(ctx, dev_malloc(ctx, &g->tails, (size_t)(ne > 0 ? ne : 1) * sizeof(int32_t)));
   }
   if (nk > 0) {
     hipLaunchKernelGGL(k_scatter_unique, dim3(grid_of(nk)), dim3(256), 0, st, sorted, nk, (const uint32_t*)flags,
@@ -232,7 +237,7 @@ int gen_rmat(xt_ctx* ctx, int scale, int edgefactor, const uint32_t thr[3], uint
     rc = e == hipSuccess ? build_csr_from_keys(ctx, m, nk, 2 * scale, scale, nv, sentinel, g)
                          : hip_err(ctx, e, "R-MAT keys");
   }
-  build_mem_done(m);
+  build_mem_done(ctx, m);
   return rc;
 }
 
@@ -293,7 +298,8 @@ int graph_from_edges(xt_ctx* ctx, int64_t nv, int64_t m, const int64_t* src, con
     rc = set_err(ctx, XT_ERR_INPUT, "edge list id out of range [0, nv)");
   if (rc == XT_OK) rc = build_csr_from_keys(ctx, mem, nk, 2 * bits, bits, nv, sentinel, g);
   g->lent = mem.off != nullptr;
-  build_mem_done(mem);
+  if (g->lent) ctx->build_users++;  // the caller's, with the graph
+  build_mem_done(ctx, mem);
   return rc;
 }
 
@@ -342,7 +348,7 @@ int graph_clean(xt_ctx* ctx, xt_graph* g) {
     rc = e == hipSuccess ? build_csr_from_keys(ctx, m, nk, 2 * bits, bits, nv, sentinel, &out)
                          : hip_err(ctx, e, "graph clean keys");
   }
-  build_mem_done(m);
+  build_mem_done(ctx, m);
   if (rc != XT_OK) {
     if (out.off) (void)hipFree(out.off);
     if (out.tails) (void)hipFree(out.tails);
@@ -419,11 +425,11 @@ int gen_er(xt_ctx* ctx, int64_t n, uint64_t seed, uint64_t thr64, xt_graph* g) {
   if (n < 1 || n > (1LL << 31) - 1) return set_err(ctx, XT_ERR_ARG, "ER n out of range");
   hipStream_t st = ctx->stream;
   g->nv = n;
-  XT_HIP(ctx, hipMalloc(&g->off, (size_t)(n + 1) * sizeof(int64_t)));
+  XT_HIP(ctx, dev_malloc(ctx, &g->off, (size_t)(n + 1) * sizeof(int64_t)));
   int64_t ne = 0;
   XT_TRY(gen_er_rows(ctx, ctx->s, n, seed, thr64, g->off, nullptr, 0, &ne, st));
   g->ne = ne;
-  XT_HIP(ctx, hipMalloc(&g->tails, (size_t)(ne > 0 ? ne : 1) * sizeof(int32_t)));
+  XT_HIP(ctx, dev_malloc(ctx, &g->tails, (size_t)(ne > 0 ? ne : 1) * sizeof(int32_t)));
   XT_TRY(gen_er_rows(ctx, ctx->s, n, seed, thr64, g->off, g->tails, ne, &ne, st));
   XT_HIP(ctx, hipStreamSynchronize(st));
   return XT_OK;
@@ -482,10 +488,10 @@ int graph_slice(xt_ctx* ctx, const xt_graph* g, int64_t lo, int64_t hi, xt_graph
     rc = hip_err(ctx, e, what);
     return rc;
   };
-  hipError_t e = hipMalloc(&mark, (size_t)(nv > 0 ? nv : 1));
-  if (e == hipSuccess) e = hipMalloc(&deg, (size_t)(nv > 0 ? nv : 1) * sizeof(uint32_t));
-  if (e == hipSuccess) e = hipMalloc(&tmp, scan_tmp_bytes(nv > 0 ? nv : 1));
-  if (e == hipSuccess) e = hipMalloc(&out->off, (size_t)(nv + 1) * sizeof(int64_t));
+  hipError_t e = dev_malloc(ctx, &mark, (size_t)(nv > 0 ? nv : 1));
+  if (e == hipSuccess) e = dev_malloc(ctx, &deg, (size_t)(nv > 0 ? nv : 1) * sizeof(uint32_t));
+  if (e == hipSuccess) e = dev_malloc(ctx, &tmp, scan_tmp_bytes(nv > 0 ? nv : 1));
+  if (e == hipSuccess) e = dev_malloc(ctx, &out->off, (size_t)(nv + 1) * sizeof(int64_t));
   if (e != hipSuccess) fail(e, "hipMalloc(slice)");
   if (rc == XT_OK && nv > 0) {
     e = hipMemsetAsync(mark, 0, (size_t)nv, st);
@@ -507,7 +513,7 @@ int graph_slice(xt_ctx* ctx, const xt_graph* g, int64_t lo, int64_t hi, xt_graph
     if (e != hipSuccess) fail(e, "slice size");
   }
   if (rc == XT_OK) {
-    e = hipMalloc(&out->tails, (size_t)(ne > 0 ? ne : 1) * sizeof(int32_t));
+    e = dev_malloc(ctx, &out->tails, (size_t)(ne > 0 ? ne : 1) * sizeof(int32_t));
     if (e != hipSuccess) fail(e, "hipMalloc(slice tails)");
   }
   if (rc == XT_OK && nv > 0) {

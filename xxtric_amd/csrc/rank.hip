@@ -1407,6 +1407,11 @@ static ListRoom list_room(const xt_ctx* ctx, int64_t nv, int64_t ne, int mode, i
 
 int rank_reserve(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, int mode, int64_t max_degree, bool per_vertex,
                  bool range) {
+  struct Ranking {  // what an allocation that fails may free meanwhile
+    xt_ctx* ctx;
+    ~Ranking() { ctx->ranking = false; }
+  } ranking{ctx};
+  ctx->ranking = true;
   const int64_t S = rank_chunk(ctx, ne);
   XT_TRY(ensure(ctx, s.crows, (size_t)(2 * ((ne + S - 1) / S)) * sizeof(int32_t)));
   XT_TRY(ensure(ctx, s.rank, (size_t)nv * sizeof(uint32_t)));

@@ -133,6 +133,8 @@ struct xt_ctx {
   std::recursive_mutex mu;
   xt::Scratch s;
   xt::DevBuf build;  // memory of graph builds (stream's work only)
+  int build_users = 0;   // builds and lent graphs in it
+  bool ranking = false;  // scratch is being reserved for a count in rank space
   uint64_t* h_counters = nullptr;  // pinned, kNumCounters: what a call reads back before it goes on or returns
   hipEvent_t ev[xt::kNumEv] = {};
   xt_timing timing = {};
@@ -150,6 +152,7 @@ struct xt_ctx {
   int64_t rank_chunks = 0;   // and its chunks of entries, a wave each
   bool force_wide = false;  // use the 64-bit offset layout of graphs with >= 2^32 entries everywhere
   int fail_allocs = 0;      // failure injection: scratch allocations left to fail
+  int fail_tries = 0;       // ... and allocations left whose first try fails
   int64_t list_lines = 0;   // for tests: lines of list memory in rank space, 0 = as many as a simple graph needs
 };
 
@@ -168,6 +171,14 @@ int set_err(xt_ctx* ctx, int code, const std::string& msg);
 int hip_err(xt_ctx* ctx, hipError_t e, const char* what);
 // Ensure a scratch buffer holds at least `bytes`; contents are not preserved.
 int ensure(xt_ctx* ctx, DevBuf& b, size_t bytes);
+// hipMalloc for what the library keeps or hands out: where device memory runs out,
+// the memory that the context keeps from earlier calls and this one does not use is
+// freed, and the allocation tried once more.
+hipError_t dev_malloc(xt_ctx* ctx, void** p, size_t bytes);
+template <typename T>
+hipError_t dev_malloc(xt_ctx* ctx, T** p, size_t bytes) {
+  return dev_malloc(ctx, reinterpret_cast<void**>(p), bytes);
+}
 
 // ---- pipeline pieces (kernels live in the .hip files) ----
 // Exclusive scan of n uint32 -> int64 out[0..n] (out[n] = total).
