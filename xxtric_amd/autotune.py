@@ -28,7 +28,8 @@ is swept with the others held at the best setting so far, for at most
 with the library's HIP-event timers (median of `reps` runs) and its results
 are checked to be identical to the first setting's.  The trials and the
 choice are cached per workload in a JSON file, so later contexts apply the
-choice without measuring again.
+choice without measuring again, as long as the library's own choice, from which the
+search starts, is the same.
 
     python -m xxtric_amd.autotune --workload rmat --scale 26
     python -m xxtric_amd.autotune --workload batch --graphs 4096
@@ -152,7 +153,7 @@ def tune(ctx, workload="rmat", scale=22, graphs=1024, reps=3, passes=2, cache=DE
     t0 = time.perf_counter()
     best, trials = search(ctx, runner, start, passes=passes, log=log, label=key)
     default_ms = next(t["ms"] for t in trials if all(t[k] == start[k] for k in SPACE))
-    entry = {"best": best, "default_ms": default_ms, "trials": trials,
+    entry = {"best": best, "start": start, "default_ms": default_ms, "trials": trials,
              "search_s": round(time.perf_counter() - t0, 2), "time": time.strftime("%Y-%m-%d %H:%M:%S")}
     if cache:
         data = {}
@@ -166,13 +167,15 @@ def tune(ctx, workload="rmat", scale=22, graphs=1024, reps=3, passes=2, cache=DE
 
 
 def apply_cached(ctx, key, cache=DEFAULT_CACHE):
-    """Apply a cached choice; returns it, or None when the cache has no entry."""
+    """Apply a cached choice; returns it, or None when the cache has no entry, or one
+    whose search started from another default (a choice among edge tiles, made before
+    the library counted in rank space, would put the context back on them)."""
     if not os.path.exists(cache):
         return None
     with open(cache) as f:
         data = json.load(f)
     entry = data.get(key)
-    if not entry:
+    if not entry or entry.get("start") != DEFAULTS:
         return None
     b = dict(DEFAULTS, **{k: v for k, v in entry["best"].items() if k in SPACE})
     apply(ctx, b)
