@@ -110,28 +110,29 @@ static_assert(kNumCounters >= kRankClasses, "the grid covers both");
 
 // ---------------------------------------------------------------------------
 // Degree classes counted (one histogram per workgroup in LDS), per-row
-// counters cleared, and the first and last row of every S-entry chunk
+// counters cleared, and the first and last row of every chunk of 2^log2 entries
 // (crows[2c], crows[2c + 1]), each written by the row that holds the boundary.
-__global__ __launch_bounds__(256) void k_rank_prep(int64_t nv, int64_t ne, const int64_t* __restrict__ off, int64_t S,
+__global__ __launch_bounds__(256) void k_rank_prep(int64_t nv, int64_t ne, const int64_t* __restrict__ off, int log2,
                                                    int32_t* __restrict__ crows, uint64_t* __restrict__ oc,
                                                    uint32_t* __restrict__ ic, uint32_t* __restrict__ hist,
                                                    unsigned long long* __restrict__ pv, uint64_t* __restrict__ oc1) {
   __shared__ uint32_t s_h[kRankClasses];
   for (int k = threadIdx.x; k < kRankClasses; k += 256) s_h[k] = 0;
   __syncthreads();
-  const int64_t nchunks = (ne + S - 1) / S;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; u < nv; u += stride) {
-    const int64_t a = off[u], b = off[u + 1];
-    oc[u] = 0;
-    ic[u] = 0;
-    if (pv) pv[u] = 0;
-    if (oc1) oc1[u] = 0;
-    atomicAdd(&s_h[degree_class(b - a)], 1u);
-    if (a < 0 || b > ne || a >= b) continue;
-    for (int64_t c = (a + S - 1) / S; c * S < b; c++) crows[2 * c] = (int32_t)u;
-    for (int64_t c1 = a / S + 1; c1 * S <= b; c1++) crows[2 * c1 - 1] = (int32_t)u;
-    if (b == ne) crows[2 * nchunks - 1] = (int32_t)u;
+  for (int64_t u0 = (int64_t)blockIdx.x * blockDim.x; u0 < nv; u0 += stride) {  // uniform
+    const int64_t u = u0 + threadIdx.x;
+    int64_t a = 0, b = 0;
+    if (u < nv) {
+      a = off[u];
+      b = off[u + 1];
+      oc[u] = 0;
+      ic[u] = 0;
+      if (pv) pv[u] = 0;
+      if (oc1) oc1[u] = 0;
+      atomicAdd(&s_h[degree_class(b - a)], 1u);
+    }
+    mark_chunks(u, a, b, ne, log2, crows);
   }
   __syncthreads();
   for (int k = threadIdx.x; k < kRankClasses; k += 256)
@@ -1449,7 +1450,8 @@ int rank_count(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, const int64_t* o
   RankRec* rec = s.rrec.as<RankRec>();
   hipLaunchKernelGGL(k_rank_clear, dim3((kNumCounters + 255) / 256), dim3(256), 0, st, counters, hist);
   XT_HIP(ctx, hipGetLastError());
-  hipLaunchKernelGGL(k_rank_prep, dim3(rank_grid(nv, 1024, 8192)), dim3(256), 0, st, nv, ne, off, S, crows, oc,
+  hipLaunchKernelGGL(k_rank_prep, dim3(rank_grid(nv, 1024, 8192)), dim3(256), 0, st, nv, ne, off,
+                     __builtin_ctzll((uint64_t)S), crows, oc,
                      s.itcnt.as<uint32_t>(), hist, pvp, oc1);
   XT_HIP(ctx, hipGetLastError());
   if (mode == kOrientId)

@@ -151,6 +151,35 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
 }
 
+// The rows that hold the first and the last entry of every chunk of S = 2^log2
+// entries that row u = [a, b) of ne entries bounds: crows[2 c] and crows[2 c + 1].
+// Called by the whole wave, a row a lane (a >= b: none).  A row of many chunks is
+// marked by the wave together: one lane's marks go out one after another, 0.74 ms
+// for the 7,800 chunks of a star's hub (2,000,000 vertices; 0.02 together).
+__device__ __forceinline__ void mark_chunks(int64_t u, int64_t a, int64_t b, int64_t ne, int log2,
+                                            int32_t* __restrict__ crows) {
+  const int64_t m = (int64_t(1) << log2) - 1;
+  const bool row = a >= 0 && b <= ne && a < b;
+  const int64_t first = row ? (a + m) >> log2 : 0;  // chunks [first, starts) start in the row
+  const int64_t starts = row ? (b + m) >> log2 : 0;
+  const int64_t last = row ? a >> log2 : 0;         // chunks [last, ends) end in it
+  const int64_t ends = row ? b >> log2 : 0;
+  const bool many = starts - last > 8;
+  if (!many) {
+    for (int64_t c = first; c < starts; c++) crows[2 * c] = (int32_t)u;
+    for (int64_t c = last; c < ends; c++) crows[2 * c + 1] = (int32_t)u;
+  }
+  for (uint64_t left = __builtin_amdgcn_ballot_w64(many); left; left &= left - 1) {  // uniform
+    const int l = __builtin_ctzll(left);
+    const int64_t f = readlane64(first, l), s = readlane64(starts, l), e = readlane64(ends, l);
+    const int32_t row_u = __builtin_amdgcn_readlane((int)u, l);
+    const int lane = threadIdx.x & (kWave - 1);
+    for (int64_t c = f + lane; c < s; c += kWave) crows[2 * c] = row_u;
+    for (int64_t c = readlane64(last, l) + lane; c < e; c += kWave) crows[2 * c + 1] = row_u;
+  }
+  if (row && b == ne) crows[2 * ((ne + m) >> log2) - 1] = (int32_t)u;
+}
+
 // Exclusive block scan of one value per thread; *total receives the block sum.
 template <int kThreads>
 __device__ __forceinline__ int64_t block_excl_scan_i64(int64_t v, int64_t* s_tmp /* kThreads/64 */,
