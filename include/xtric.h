@@ -77,7 +77,8 @@ const char* xt_last_error(const xt_ctx* ctx);
 int xt_last_timing(const xt_ctx* ctx, xt_timing* out);
 /* Totals and owned ranges of one graph in degree orientation are counted in rank
  * space (vertices ranked by degree, lists of smaller ranks in 16 bits, bit maps in LDS), and so
- * are its per-vertex counts below 2^27 entries and, where the host passed in the
+ * are its per-vertex counts below 2^27 entries (unless it is dense: more than 64
+ * entries a vertex, and these times all entries at least 2^29) and, where the host passed in the
  * offsets and no row is longer than 256, counts in id orientation.  Batches whose
  * graphs have at most 65535 vertices are counted over 16-bit lists.  The knobs
  * below belong to the edge tiles that all other counts use; a context on which

@@ -44,3 +44,11 @@ def test_a_hub_of_thousands_of_chunks(own):
     u = np.concatenate([np.zeros(n - 1, np.int64), np.arange(1, n - 1)])
     v = np.concatenate([np.arange(1, n), np.arange(2, n)])
     _against_tiles(own, own.graph_from_edges(n, u, v))
+
+
+@pytest.mark.parametrize("clique,copies", [(1000, 1), (2000, 1), (200, 800), (1200, 12)])
+def test_per_vertex_counts_of_dense_graphs(own, clique, copies):
+    """Where nearly every id that is looked up is a hit, and out-lists are long."""
+    a, b = np.triu_indices(clique, 1)
+    base = (np.arange(copies) * clique)[:, None]
+    _against_tiles(own, own.graph_from_edges(clique * copies, (base + a).reshape(-1), (base + b).reshape(-1)), per_vertex=True)

@@ -204,6 +204,17 @@ bool edge_tile_knobs(const xt_ctx* ctx) {
 // 1.78), s20 3.4 and 4.2 (4.3 and 4.9), s22 16.7 and 18.7 (16.3 and 21.1), s23
 // 40.0 and 37.7 (43.3 and 41.4); G(n, p) of degree 64 on 200,000 0.83 and 2.5).
 constexpr int64_t kRankPvEntries = int64_t(1) << 27;
+// Nor do large dense graphs: every hit is credited on its own there (6 to 19 ps a
+// hit), where the group kernel counts the hits of long lists by masks (1 to 2 ps).
+// Dense: more than this many entries a vertex, and at least this many pairs of
+// entries of a row (ms, rank space against edge tiles: K_1000 1.08 and 0.82, K_2000
+// 16 and 1.9, K_4000 108 and 9.5; G(n, p) of degree 256 on 200,000 5.0 and 4.3, of
+// degree 3,600 on 12,000 114 and 36; R-MAT s18 of degree 104 5.5 and 4.7; below
+// the line K_300 0.17 and 0.50, G(n, p) of degree 500 on 1,000 0.29 and 0.44, R-MAT
+// s14 of degree 120 0.44 and 0.55).  A dense core among many sparse vertices is not
+// seen from these numbers.
+constexpr int64_t kRankPvDegree = 64;
+constexpr int64_t kRankPvPairs = int64_t(1) << 29;
 // In id orientation out-lists are as long as rows; where rows are long, one
 // wave's list or map waits for another (ms: RGG n = 200,000 0.18 and 0.31,
 // G(n, p) of degree 64 0.87 and 2.6, but R-MAT s14, rows to 3,700, 0.71 and 0.38).
@@ -216,7 +227,7 @@ constexpr int64_t kRankIdDegree = 256;
 // edge tiles, when set, ask for those.
 static bool ranks(const xt_ctx* ctx, int64_t nv, int64_t ne, int mode, bool per_vertex, int64_t max_degree) {
   if (mode == kOrientId && (max_degree < 0 || max_degree > kRankIdDegree)) return false;
-  if (per_vertex && ne >= kRankPvEntries) return false;
+  if (per_vertex && (ne >= kRankPvEntries || (ne / kRankPvDegree > nv && ne / nv * ne >= kRankPvPairs))) return false;
   return !edge_tile_knobs(ctx) && ne > 0 && rank_fits(ctx, nv, ne, mode, max_degree);
 }
 
