@@ -36,6 +36,7 @@ if int(os.environ.get("GPU_MAX_HW_QUEUES", "4") or "4") < 8:
 
 METRIC = "edges/s + %HBM roofline, R-MAT s26 (1 GPU); batched graphs/s, p99 latency"
 HBM_PEAK_GBS = 8000.0
+LINE_CEILING_G = 55.7  # random gathers of 4 bytes, profiles/memory_ceilings.md
 # rocprofv3 FETCH_SIZE / WRITE_SIZE summary of this workload; its lines
 # "traffic_bytes_per_launch: N" and "traffic_bytes_per_count: N" give the measured
 # HBM bytes of one launch of the intersection kernel and of all kernels of a count.
@@ -274,9 +275,12 @@ def measured_traffic(what):
 
 def roofline(r):
     """A count in rank space (the library's choice for this workload): the
-    intersection is k_rank_count, and its bytes and those of the whole count are
-    measured ones (the profile's, at the profile's scale), for what a count has to
-    read there has no formula in the statistics.
+    intersection is k_rank_count.  Its bytes and those of the whole count are the
+    lines that missed L2 in an earlier, profiled run of the same workload (at its
+    scale), for what a count has to read there has no formula in the statistics.
+    The 256 MB cache serves some of them, so the rates are upper bounds of what HBM
+    gave; what bounds the kernel is the rate of lines, beside the highest that
+    random gathers reach here.
 
     A count in edge tiles: the heavy-edge intersection, k_count_groups (owners with
     long out-lists) followed by k_count_waves (owners whose out-list fits a
@@ -303,6 +307,10 @@ def roofline(r):
            "kernel_ms": round(r["group_ms"], 3), "alg_bytes_per_launch": None if ranked else launch,
            "whole_count": whole}
     out.update(rate(launch, r["group_ms"]))
+    if ranked:
+        lines = launch / 128 / (r["group_ms"] * 1e-3) / 1e9 if launch else None
+        out.update({"bound": "lines that miss L2", "bytes_are": "FETCH_SIZE and WRITE_SIZE of a stored profile",
+                    "glines_per_s": lines and round(lines, 1), "gather_ceiling_glines_per_s": LINE_CEILING_G})
     return out
 
 

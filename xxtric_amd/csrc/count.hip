@@ -1852,12 +1852,12 @@ int reserve(xt_ctx* ctx, Scratch& s, int64_t nv, int64_t ne, bool per_vertex) {
 
 static size_t round256(size_t n) { return (n + 255) & ~(size_t)255; }
 
-// Of the counters only the slots' 192 bytes: the region holds the sums besides.
+// Of the counters only the slots: the region holds the sums besides.
 size_t carve_bytes(int64_t nv, int64_t ne) {
   Scratch tmp;
   size_t tot = 0;
   for_each_need(tmp, nv, ne, false, [&](DevBuf& b, size_t bytes) {
-    tot += round256(&b == &tmp.counters ? size_t{192} : bytes);
+    tot += round256(&b == &tmp.counters ? kNumSlots * sizeof(uint64_t) : bytes);
   });
   return tot;
 }

@@ -22,7 +22,7 @@
 // Both passes that gather or stream are bound by the lines that miss L2 (about
 // 52-55 G lines of 128 bytes a second on this GPU, from HBM or from the 256 MB
 // cache).  R-MAT s26: 353 ms with edge tiles, 182-188 here: k_rank_split 40-42,
-// k_rank_lists 10-11, k_rank_count 131-135 (949 GB: 7.1 TB/s).
+// k_rank_lists 10-11, k_rank_count 131-135 (949 GB of such lines, 55 G/s).
 //
 // Six kernels, no scan over the vertices and no item list:
 //  k_rank_clear   counters and class histogram cleared

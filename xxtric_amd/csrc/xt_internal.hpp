@@ -102,7 +102,7 @@ struct Scratch {
   DevBuf ooff;      // int64[nv+1]         oriented offsets
   DevBuf vrec;      // uint64[nv]          ooff[x] | d+(x) << 32 when |E+| < 2^32 (gathered per entry)
   DevBuf otails;    // int32[ne+4]         oriented out-lists, ascending ids (|E+| <= ne), padded
-  DevBuf counters;  // uint64[kNumCounters] slots (total, tile queue, input-error flags, statistics), then sharded sums
+  DevBuf counters;  // uint64[kNumCounters] slots (tile queue, input-error flags, statistics), then sharded sums
   DevBuf oflags;    // uint8[ne/8]         kept-entry mask per 8 CSR entries (orientation)
   DevBuf crows;     // int64[2*nchunks]    first and last row of each kChunk-entry input chunk
   DevBuf itcnt;     // uint32[nv]          heavy edges owned by each vertex
@@ -117,7 +117,7 @@ struct Scratch {
   DevBuf ocount;    // uint64[nv]          neighbours of smaller rank | those below 65535 << 32
   DevBuf rpart;     // uint32[ne]          rows as ranks, smaller ones first
   DevBuf rlists;    // 16 B chunks         lists of smaller ranks (hot 16-bit, cold 32-bit)
-  DevBuf rrec;      // 16 B[nv]            list record of every rank
+  DevBuf rrec;      // 32 B[nv]            list record of every rank
   DevBuf scan_tmp;  // int64[..]           block sums of the scans
   DevBuf in_off;    // int64[nv+1]         staged input offsets (xt_count_csr)
   DevBuf in_tails;  // int32[ne]           staged input ids (xt_count_csr)
